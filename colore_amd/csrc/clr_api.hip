@@ -204,6 +204,7 @@ int clr_upload_tables(clr_ctx *c, const clr_tables *t) {
   c->h_d1.assign(t->growth_d_arr, t->growth_d_arr + na);
   c->h_pd.assign(t->growth_pd_arr, t->growth_pd_arr + na);
   c->geo_nz = 0;   // shell geometry depends on the tables
+  c->shell_dr = 0;
   for (int i = 0; i < 6; i++) {
     c->h_bg_first[i] = src[i][0];
     c->h_bg_last[i] = src[i][na - 1];

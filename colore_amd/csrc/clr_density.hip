@@ -2,31 +2,31 @@
 // bias normalisation (density.c:1128-1393) on gfx950.
 //
 // k_transform : lognormalize / densclip in place.
-// k_shells    : one pass over the grid.  Each wavefront walks tiles of
-//               16 (x) x 16 (y) x 16 (z) cells, 64 rows of 16 x 4 cells (one
-//               cell per lane: a compact footprint keeps the table bins the
-//               lanes gather close together); per cell the
-//               radius, then from one packed FP32 table D(r), z(r) and every
-//               b_t(r); the shell index s = (int)(z*idz)+1 is taken from the
-//               FP32 z where that is more than 5e-4 of a shell away from a
-//               shell edge, otherwise from the reference's FP64 expressions
-//               (so the counts match bit for bit); then count, z and
-//               bias_model(delta, b_t(r)) for every tracer.  A lane's radius
-//               changes slowly along its 64 cells, so it adds into private
-//               FP64 accumulators of its current shell and logs finished
-//               shells (at most kSlots) in its own LDS slots; the lanes are
-//               combined once per tile with DPP wave sums, and lane 0 adds the
-//               result into the wavefront's own LDS accumulators.  Every
-//               addition happens in a fixed order: the sums are bitwise
-//               repeatable.  With `fused` the lognormal transform is applied
-//               in the same pass (one read and one write of the grid for both
-//               stages).
+// k_shells    : one pass over the grid.  Each wavefront walks tiles of 64-cell
+//               rows; per cell the radius, then from packed FP32 tables D(r),
+//               z(r) and every b_t(r); the shell index s = (int)(z*idz)+1 is
+//               taken from the FP32 z where that is more than 5e-4 of a shell
+//               away from a shell edge, otherwise from the reference's FP64
+//               expressions (so the counts match bit for bit); then count, z
+//               and bias_model(delta, b_t(r)) for every tracer, into FP64
+//               registers per shell of the tile, combined once per tile in a
+//               fixed order: the sums are bitwise repeatable.  With `fused`
+//               the lognormal transform is applied in the same pass (one read
+//               and one write of the grid for both stages).
+//               Bound by VALU issue: 76 instructions per row of 64 cells (155
+//               before) at 4 to 5 wavefronts per SIMD, 65 % of the issue
+//               slots.  At 1024^3, three tracers, fused: 3.53 ms (4.85 ms with one
+//               current-shell accumulator per lane, flushed by DPP sums at
+//               every second change of shell, which also took 0.52 ms at 64^3,
+//               now 13 us; 192^3 0.41 -> 0.078, 256^3 0.23 -> 0.078, 512^3
+//               0.64 -> 0.41 ms).
 // k_shell_final / k_norm_table : fixed-order reduction of the per-block
 //               partials, norm = count/sum, edge fill and linear
 //               interpolation in z onto the NA r-grid (density.c:1272-1355),
 //               all on the device.
 #include "clr_internal.h"
 #include <math.h>
+#include <algorithm>
 #include <vector>
 
 using namespace clr;
@@ -36,22 +36,8 @@ namespace {
 constexpr int kShellBlocks = 8192;
 constexpr int kShellThreads = 256;
 constexpr int kWaves = kShellThreads / 64;
-// A wavefront row is kTX consecutive x cells of kSub = 64/kTX adjacent y
-// rows (lane = x + kTX * sub-row): a short x extent keeps the radii, and so
-// the table bins the lanes gather, close together.  A tile is kTY x kTZ such
-// rows: kTX x (kTY kSub) x kTZ cells.
-#ifndef CLR_SHELL_TX
-#define CLR_SHELL_TX 16
-#endif
-constexpr int kTX = CLR_SHELL_TX, kSub = 64 / kTX;
-constexpr int kTY = 4, kTZ = 16;
-constexpr int kSlots = 1;
-#ifndef CLR_SHELL_PREFETCH
-#define CLR_SHELL_PREFETCH 2
-#endif
-constexpr int kPrefetch = CLR_SHELL_PREFETCH;   // rows of density in flight per wavefront
-static_assert((kTY * kTZ) % kPrefetch == 0, "prefetch distance must divide the tile rows");
 constexpr int kMaxTr = 8;
+constexpr int kRegWin = 4;   // shells of a tile's window (FP64 registers)
 
 struct ShellArgs {
   float *g;
@@ -59,60 +45,55 @@ struct ShellArgs {
   double dx, ox, oy, oz, idr, r_last, z_last, sigma2, idz;
   const double *r_arr, *zt;
   const double *sigma2_dev;   // when set, sigma^2 is read here instead of `sigma2`
-  const float4 *tab;   // per bin: (value, slope) of D, z, b_0 .. b_{NT-1} (k_pack_shell_table)
+  const float2 *tab;   // [2 + ntr][na]: (value, slope) per bin (k_pack_shell_table)
   float d1_last_f, z_last_f, idr_f, idz_f;
   float bz0[kMaxTr];
   int model[kMaxTr];
+  int nbin;              // shell_plan: staged table bins per tile
+  int mono;              // z(r) never decreases
 };
 
-// FP32 tables of one shell pass packed per bin i as (f_i, f_{i+1} - f_i) for
-// quantity 0 = D(r), 1 = z(r), 2 + t = b_t(r): one gather per cell, and
-// f_i + slope * t is the same FP32 value as f_i + (f_{i+1} - f_i) * t.
-// shell_tab_w(ntr) float4s per bin.
+// FP32 tables of one shell pass as (f_i, f_{i+1} - f_i) per bin i, one row of
+// na bins per quantity: 0 = D(r), 1 = z(r), 2 + t = b_t(r); f_i + slope * t is
+// the same FP32 value as f_i + (f_{i+1} - f_i) * t.
 struct ShellTabSrc {
   const float *d1f;
   const double *zt;
   const float *bzf[kMaxTr];
 };
-__host__ __device__ constexpr int shell_tab_w(int ntr) { return (2 * (2 + ntr) + 3) / 4; }
-__global__ void k_pack_shell_table(ShellTabSrc src, int ntr, int na, float4 *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_pack_shell_table(ShellTabSrc src, int na, float2 *__restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, q = blockIdx.y;
   if (i >= na) return;
-  const int w = shell_tab_w(ntr), j = i + 1 < na ? i + 1 : i;
-  float v[4 * shell_tab_w(kMaxTr)];
-  for (int k = 0; k < 4 * w; k++) v[k] = 0.f;
-  const float d0 = src.d1f[i], d1 = src.d1f[j], z0 = (float)src.zt[i], z1 = (float)src.zt[j];
-  v[0] = d0;
-  v[1] = d1 - d0;
-  v[2] = z0;
-  v[3] = z1 - z0;
-  for (int t = 0; t < ntr; t++) {
-    const float b0 = src.bzf[t][i], b1 = src.bzf[t][j];
-    v[4 + 2 * t] = b0;
-    v[5 + 2 * t] = b1 - b0;
+  const int j = i + 1 < na ? i + 1 : i;
+  float f0, f1;
+  if (q == 1) {
+    f0 = (float)src.zt[i];
+    f1 = (float)src.zt[j];
+  } else {
+    const float *f = q == 0 ? src.d1f : src.bzf[q - 2];
+    f0 = f[i];
+    f1 = f[j];
   }
-  for (int k = 0; k < w; k++) out[(size_t)i * w + k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+  out[(size_t)q * na + i] = make_float2(f0, f1 - f0);
 }
 
-template <int CTRL, int RM>
+template <int CTRL>
 __device__ inline double dpp_get(double v) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  const int l2 = __builtin_amdgcn_update_dpp(0, lo, CTRL, RM, 0xF, true);
-  const int h2 = __builtin_amdgcn_update_dpp(0, hi, CTRL, RM, 0xF, true);
+  const int l2 = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true);
+  const int h2 = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true);
   return __hiloint2double(h2, l2);
 }
 
-// Sum over the 64 lanes of a wavefront (all lanes active), broadcast.
-__device__ inline double wave_sum(double x) {
-  x += dpp_get<0xB1, 0xF>(x);    // quad_perm [1,0,3,2]
-  x += dpp_get<0x4E, 0xF>(x);    // quad_perm [2,3,0,1]
-  x += dpp_get<0x141, 0xF>(x);   // row_half_mirror
-  x += dpp_get<0x140, 0xF>(x);   // row_mirror
-  x += dpp_get<0x142, 0xA>(x);   // row_bcast:15 into rows 1,3
-  x += dpp_get<0x143, 0xC>(x);   // row_bcast:31 into rows 2,3
-  const int lo = __builtin_amdgcn_readlane(__double2loint(x), 63);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(x), 63);
-  return __hiloint2double(hi, lo);
+// Sum over each group of G consecutive lanes, in every lane of the group.
+template <int G>
+__device__ inline double lanes_sum(double x) {
+  if (G >= 2) x += dpp_get<0xB1>(x);     // quad_perm [1,0,3,2]
+  if (G >= 4) x += dpp_get<0x4E>(x);     // quad_perm [2,3,0,1]
+  if (G >= 8) x += dpp_get<0x141>(x);    // row_half_mirror
+  if (G >= 16) x += dpp_get<0x140>(x);   // row_mirror
+  if (G >= 32) x += __shfl_xor(x, 16);
+  if (G >= 64) x += __shfl_xor(x, 32);
+  return x;
 }
 
 __global__ __launch_bounds__(256) void k_transform(float *__restrict__ g, int N, int ngx, double dx,
@@ -140,46 +121,26 @@ __global__ __launch_bounds__(256) void k_transform(float *__restrict__ g, int N,
   }
 }
 
-// Combine the slot-k accumulators of all lanes (slot values in LDS,
-// vals[q * 64 + lane]): lanes are grouped by shell id (in order of the lowest
-// lane) and each group is summed with DPP.
-template <int NQ>
-__device__ inline void flush_slot(unsigned long long mask, int key, const double *vals, double *myacc,
-                                  int lane) {
-  while (mask) {
-    const int leader = __ffsll((long long)mask) - 1;
-    const int sl = __builtin_amdgcn_readlane(key, leader);
-    const bool mine = ((mask >> lane) & 1ull) && key == sl;
-    const unsigned long long mm = __ballot(mine);
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-      const double v = wave_sum(mine ? vals[q * 64 + lane] : 0.0);
-      if (lane == 0) myacc[sl * NQ + q] += v;
-    }
-    mask &= ~mm;
-  }
-}
-
 // bias_model (common.h:414-431) for the shell sums, on the raw hardware
-// exp2/log2 and a fast reciprocal (a few ulp: the sums are of FP32 terms),
-// without branches (the model is uniform, the sign of d is not):
+// exp2/log2 and a fast reciprocal (a few ulp: the sums are of FP32 terms):
 //   0: (1+d)^b = exp2(b l2),            l2 = log2(1+d)
 //   1: d < 0: exp(b d/(1+d)) = exp2(b q), q = log2(e) d/(1+d); else 1 + b d
 //   2: max(1 + b d, 0)
-// l2 and q are shared by the tracers; d <= -1 (or NaN) gives 0.
-__device__ inline float bias_sum_term(float d, float l2, float q, float b, int model) {
-  const float e = __builtin_amdgcn_exp2f(b * (model == 0 ? l2 : q));
-  const float lin = fmaxf(__builtin_fmaf(b, d, 1.f), 0.f);
-  const bool use_exp = model == 0 || (model == 1 && d < 0.f);
-  return d > -1.f ? (use_exp ? e : lin) : 0.f;
-}
-
-// LDS per block: kWaves x nz x NQ accumulators, then per wavefront kSlots x
-// NQ x 64 logged shell sums and kSlots x 64 shell ids.
-template <int NT>
-constexpr size_t shell_lds_bytes(int nz) {
-  return (size_t)kWaves * nz * (2 + NT) * sizeof(double) +
-         (size_t)kWaves * kSlots * 64 * ((2 + NT) * sizeof(double) + sizeof(int));
+// d <= -1 (or NaN) gives 0.
+template <int MODEL>
+__device__ inline float bias_sum_term(float d, float l2, float b) {
+  float v;
+  if (MODEL == 0) {
+    v = __builtin_amdgcn_exp2f(b * l2);
+  } else {
+    v = fmaxf(__builtin_fmaf(b, d, 1.f), 0.f);
+    if (MODEL == 1) {
+      const float q = 1.44269504f * d * __builtin_amdgcn_rcpf(1.f + d);
+      const float e = __builtin_amdgcn_exp2f(b * q);
+      v = d < 0.f ? e : v;
+    }
+  }
+  return d > -1.f ? v : 0.f;
 }
 
 // z(r) of cell (ix,iy,iz) by the reference's FP64 expressions (density.c:
@@ -193,174 +154,281 @@ __device__ inline double cell_z_f64(const ShellArgs &a, int ix, int iy, int iz) 
 }
 
 // M0: every tracer uses bias model 0 (no other model's code in the loop).
-template <int NT, bool M0>
-__global__ __launch_bounds__(kShellThreads) __attribute__((amdgpu_waves_per_eu(6))) void k_shells(ShellArgs a,
-                                                                                      double *__restrict__ partial) {
-  constexpr int NQ = 2 + NT;
-  constexpr int W = shell_tab_w(NT);
+// A tile is ROWS rows along y of TX x TZ (x, z) cells, TX TZ = 64 (TX = 4:
+// one row of 4 x 4 x 4 cells); STAGE: its part of the r-tables is staged in
+// LDS (see shell_plan).
+//
+// A lane adds its cells, in the program's order, to FP64 registers, one set
+// per shell of the tile's window (kRegWin shells), and at the end of a tile
+// the 64 lanes of a (shell, quantity) are added up through LDS in a fixed
+// order: the sums repeat bit for bit, and the loop has no test for a change of
+// shell.  A tile that spans more shells takes further passes; one outside the
+// last shell (48 % of a box) only gets its lognormal transform.
+template <int NT, bool M0, int TX, int ROWS, bool STAGE>
+__global__ __launch_bounds__(kShellThreads) __attribute__((amdgpu_waves_per_eu(NT <= 2 ? 5 : (NT <= 4 ? 4 : 2)))) void
+k_shells(ShellArgs a, double *__restrict__ partial) {
+  constexpr int NQ = 2 + NT, NF = 1 + NT;
+  constexpr bool CUBE = TX == 4;
+  constexpr int TY = CUBE ? 4 : 1, TZ = 64 / (TX * TY);
+  constexpr int U = ROWS > 1 ? 2 : 1;   // rows worked together
   extern __shared__ double acc[];
-  const int nz = a.nz, N = a.N;
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int nz = a.nz, N = a.N, nbin = a.nbin;
+  const int nwaves = blockDim.x / 64, lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   double *myacc = acc + (size_t)wave * nz * NQ;
-  double *logv = acc + (size_t)kWaves * nz * NQ + (size_t)wave * kSlots * NQ * 64;   // [slot][q][lane]
-  int *logid = (int *)(acc + (size_t)kWaves * nz * NQ + (size_t)kWaves * kSlots * NQ * 64) + wave * kSlots * 64;
-  for (int i = threadIdx.x; i < kWaves * nz * NQ; i += blockDim.x) acc[i] = 0;
+  // the wavefront's LDS: one shell's [NF][64] sums and the tile's part of the
+  // tables, [NQ][nbin] (value, slope)
+  double *wsum = acc + (size_t)nwaves * nz * NQ + (size_t)wave * (NF * 64 + nbin * NQ);
+  float2 *seg = (float2 *)(wsum + NF * 64);
+  for (int i = threadIdx.x; i < nwaves * nz * NQ; i += blockDim.x) acc[i] = 0;
   __syncthreads();
   const float ox = (float)a.ox, oy = (float)a.oy, oz = (float)a.oz, dxf = (float)a.dx;
   const float s2f = (float)(a.sigma2_dev ? *a.sigma2_dev : a.sigma2);
-  const int ntx = (N + kTX - 1) / kTX, nty = N / (kTY * kSub), ntz = N / kTZ;
-  const long ntiles = (long)ntx * nty * ntz;
-  const long nw = (long)gridDim.x * kWaves;
-  // all lanes' logged shells into the wavefront's accumulators
-  auto flush_all = [&](int nslot) {
+  const int ntx = N / TX, nty = N / (TY * ROWS), ntz = N / TZ;
+  const int ntiles = ntx * nty * ntz;
+  const int nw = (int)gridDim.x * nwaves;
+  for (int tile = (int)blockIdx.x * nwaves + wave; tile < ntiles; tile += nw) {
+    const int tx = tile % ntx, rest = tile / ntx;
+    const int ty = rest % nty, tz = rest / nty;
+    const int ix = tx * TX + lane % TX, iy0 = ty * TY * ROWS + (lane / TX) % TY, iz = tz * TZ + lane / (TX * TY);
+    float *const tb = a.g + ((size_t)iz * N + iy0) * a.ngx + ix;
+    const int ystep = TY * a.ngx;
+    // densities of U rows, and of the U after them (two groups ahead in the
+    // loops below)
+    float d[U], dn[U];
+    auto load = [&](int r, float *v) {
 #pragma unroll
-    for (int k = 0; k < kSlots; k++)
-      flush_slot<NQ>(__ballot(k < nslot), logid[k * 64 + lane], logv + (size_t)k * NQ * 64, myacc, lane);
-  };
-  for (long tile = (long)blockIdx.x * kWaves + wave; tile < ntiles; tile += nw) {
-    const int tx = (int)(tile % ntx);
-    const long rest = tile / ntx;
-    const int ty = (int)(rest % nty), tz = (int)(rest / nty);
-    const int ix = tx * kTX + lane % kTX, ly = lane / kTX;
-    const int iy0 = ty * kTY * kSub + ly;   // the lane's y in the tile's first row
-    const bool valid = ix < N;
-    int nslot = 0, cur = -1;
-    double cacc[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) cacc[q] = 0;
-    const float x32 = coord_f32(ix, dxf, ox);
-    // The next row's density and table bins are loaded while the current row
-    // is processed.  Bin lookup: FP32 radius (absolute error ~1e-3 cell), one
-    // index for D, z and every b_t (f_of_r32 semantics).
-    struct Bin {
-      float4 C[W];
-      float tq;
-      bool e0, e1;
+      for (int u = 0; u < U; u++) v[u] = tb[(r + u) * ystep];
     };
-    auto fetch = [&](int rr2, Bin &bn) {
-      const int iy2 = iy0 + (rr2 % kTY) * kSub, iz2 = tz * kTZ + (rr2 / kTY);
-      const float y32 = coord_f32(iy2, dxf, oy), z32 = coord_f32(iz2, dxf, oz);
-      const TabPos tp = tab_pos_f32(radius_f32(x32, y32, z32), a.idr_f, a.na);
-      bn.e0 = tp.e0;
-      bn.e1 = tp.e1;
-      bn.tq = tp.tq;
+    load(0, d);
+    if (ROWS > U) load(U, dn);
+    auto next = [&](int r) {   // after the rows r .. r+U-1
 #pragma unroll
-      for (int k = 0; k < W; k++) bn.C[k] = a.tab[(size_t)tp.i0 * W + k];
+      for (int u = 0; u < U; u++) d[u] = dn[u];
+      if (r + 2 * U < ROWS) load(r + 2 * U, dn);
     };
-    // the lane's cell in the tile's first row; rows at uniform offsets from it
-    float *const tb = a.g + ((size_t)(tz * kTZ) * N + iy0) * a.ngx + (valid ? ix : 0);
-    const auto roff = [&](int r) { return ((size_t)(r / kTY) * N + (r % kTY) * kSub) * a.ngx; };
-    // densities kPrefetch rows ahead (the loads that wait on HBM), table bins
-    // one row ahead (cache hits), issued bins first so that waiting for them
-    // never waits for a later density
-    float dq[kPrefetch];
+    // table bins and shells that the tile's radii can fall in: its nearest
+    // and farthest point, 1e-5 of the radius and 0.01 shell further out
+    int s_lo, s_hi, b_lo, nb;
+    bool edge;
+    {
+      const float xa = coord_f32(tx * TX, dxf, ox), xb = coord_f32(tx * TX + TX - 1, dxf, ox);
+      const float ya = coord_f32(ty * TY * ROWS, dxf, oy), yb = coord_f32((ty + 1) * TY * ROWS - 1, dxf, oy);
+      const float za = coord_f32(tz * TZ, dxf, oz), zb = coord_f32(tz * TZ + TZ - 1, dxf, oz);
+      const float xn = fmaxf(fmaxf(xa, -xb), 0.f), yn = fmaxf(fmaxf(ya, -yb), 0.f), zn = fmaxf(fmaxf(za, -zb), 0.f);
+      const float xf = fmaxf(-xa, xb), yf = fmaxf(-ya, yb), zf = fmaxf(-za, zb);
+      const float rlo = radius_f32(xn, yn, zn) * (1.f - 1e-5f), rhi = radius_f32(xf, yf, zf) * (1.f + 1e-5f);
+      const TabPos plo = tab_pos_f32(rlo, a.idr_f, a.na), phi = tab_pos_f32(rhi, a.idr_f, a.na);
+      edge = plo.e0 || phi.e1;
+      const int i_lo = plo.e1 ? a.na - 1 : plo.i0, i_hi = phi.e1 ? a.na - 1 : phi.i0;
+      if (a.mono) {
+        const float2 tl = a.tab[a.na + plo.i0], th = a.tab[a.na + phi.i0];
+        const float zl = plo.e0 ? 0.f : (plo.e1 ? a.z_last_f : tl.x + tl.y * plo.tq);
+        const float zh = phi.e0 ? 0.f : (phi.e1 ? a.z_last_f : th.x + th.y * phi.tq);
+        s_lo = (int)(zl * a.idz_f - 0.01f) + 1;
+        s_hi = (int)(zh * a.idz_f + 0.01f) + 1;
+      } else {
+        s_lo = 0;
+        s_hi = nz - 1;
+      }
+      s_lo = __builtin_amdgcn_readfirstlane(max(s_lo, 0));
+      s_hi = __builtin_amdgcn_readfirstlane(min(s_hi, nz - 1));
+      b_lo = __builtin_amdgcn_readfirstlane(i_lo);
+      nb = __builtin_amdgcn_readfirstlane(i_hi - i_lo + 1);
+      edge = __builtin_amdgcn_readfirstlane((int)edge) != 0;
+    }
+    const bool inside = s_lo < nz;
+    if (!inside && !a.fused) continue;
+    if (STAGE) {
+      nb = min(nb, nbin);
+      for (int q = 0; q < (inside ? NQ : 1); q++)
+        for (int i = lane; i < nb; i += 64) seg[q * nbin + i] = a.tab[q * a.na + b_lo + i];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+    // (value, slope) of quantity q at a cell's bin; an entry past the tile's
+    // bins is only looked up for cells at the table's ends, which take the
+    // edge values
+    auto entry = [&](const TabPos &p, int q) {
+      if (!STAGE) return a.tab[q * a.na + p.i0];
+      return seg[q * nbin + (int)min((unsigned)(p.i0 - b_lo), (unsigned)(nb - 1))];
+    };
+    const float x32 = coord_f32(ix, dxf, ox), z32 = coord_f32(iz, dxf, oz), z2 = z32 * z32;
+    // the lane's cell in row r: x, z fixed, y = iy0 + TY r.  With TY = 1 the
+    // row's y is the wavefront's: lane r holds row r's y
+    const float yl = CUBE ? 0.f : coord_f32(iy0 + lane, dxf, oy);
+    auto radius_at = [&](int r) {
+      const float y32 = CUBE ? coord_f32(iy0 + TY * r, dxf, oy)
+                             : __int_as_float(__builtin_amdgcn_readlane(__float_as_int(yl), r));
+      return __builtin_amdgcn_sqrtf(__builtin_fmaf(x32, x32, __builtin_fmaf(y32, y32, z2)));
+    };
+    // Table position in row r.  The fraction of a bin is r idr - i0 rounded
+    // once (fma), in every second group of four y rows from the rounded
+    // product: sums of FP32 terms shift by a few 1e-9 with the choice, and
+    // this one keeps them equal to those of earlier builds.
+    auto pos_at = [&](int r) {
+      const float rf = radius_at(r);
+      TabPos p = tab_pos_f32(rf, a.idr_f, a.na);
+      const bool odd = (((ty * TY * ROWS + r) >> 2) & 1) != 0;
+      p.tq = __builtin_fmaf(odd ? rf * a.idr_f : rf, odd ? 1.f : a.idr_f, -(float)p.i0);
+      return p;
+    };
+    if (!inside) {
+      // no shell in reach: the transform alone
+#pragma unroll 1
+      for (int r = 0; r < ROWS; r += U) {
+        float o[U];
 #pragma unroll
-    for (int j = 0; j < kPrefetch; j++) dq[j] = valid ? tb[roff(j)] : 0.f;
-    Bin bnext;
-    fetch(0, bnext);
-    for (int r0 = 0; r0 < kTY * kTZ; r0 += kPrefetch)
+        for (int u = 0; u < U; u++) o[u] = d[u];
+        next(r);
 #pragma unroll
-    for (int j = 0; j < kPrefetch; j++) {
-      const int rr = r0 + j;
-      const int iy = iy0 + (rr % kTY) * kSub, iz = tz * kTZ + (rr / kTY);
-      int s = -1;
-      double v[NQ];
-      float dl = dq[j];
-      const Bin bn = bnext;
-      if (rr + 1 < kTY * kTZ) fetch(rr + 1, bnext);
-      if (rr + kPrefetch < kTY * kTZ && valid) dq[j] = tb[roff(rr + kPrefetch)];
-      if (valid) {
-        float comp[NQ];
-        const bool e0 = bn.e0, e1 = bn.e1;
-        {
-          const float tq = bn.tq;
-          float f[4 * W];
+        for (int u = 0; u < U; u++) {
+          const TabPos p = pos_at(r + u);
+          const float2 e = entry(p, 0);
+          o[u] = lognormal_f32(o[u], growth_at(p, e.x, e.y, a.d1_last_f), s2f);
+        }
 #pragma unroll
-          for (int k = 0; k < W; k++) {
-            f[4 * k + 0] = bn.C[k].x;
-            f[4 * k + 1] = bn.C[k].y;
-            f[4 * k + 2] = bn.C[k].z;
-            f[4 * k + 3] = bn.C[k].w;
+        for (int u = 0; u < U; u++) tb[(r + u) * ystep] = o[u];
+      }
+      continue;
+    }
+    // the tile's shells, kRegWin at a time (later passes use the transformed
+    // cells)
+    for (int wb = s_lo; wb <= s_hi; wb += kRegWin) {
+      const int wn = min(kRegWin, nz - wb);
+      const bool fuse = a.fused && wb == s_lo;
+      double ra[kRegWin][NF];
+      uint32_t rc[kRegWin];
+#pragma unroll
+      for (int k = 0; k < kRegWin; k++) {
+        rc[k] = 0u;
+#pragma unroll
+        for (int q = 0; q < NF; q++) ra[k][q] = 0;
+      }
+      if (wb != s_lo) {   // a later pass: the rows once more
+        load(0, d);
+        if (ROWS > U) load(U, dn);
+      }
+      {
+#pragma unroll 1
+        for (int g = 0; g < ROWS; g += U) {
+          TabPos tp[U];
+          float2 C[U][NQ];
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            tp[u] = pos_at(g + u);
+#pragma unroll
+            for (int q = 0; q < NQ; q++) C[u][q] = entry(tp[u], q);
+          }
+          // the U rows step by step, so that their dependent chains interleave
+          float comp[U][NQ], dl[U];
+          bool ends[U];   // at the table's ends: the reference's edge values
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int q = 0; q < NQ; q++) comp[u][q] = __builtin_fmaf(C[u][q].y, tp[u].tq, C[u][q].x);
+            dl[u] = d[u];
+            ends[u] = false;
+          }
+          next(g);
+          if (edge) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+              ends[u] = tp[u].e0 || tp[u].e1;
+              comp[u][0] = tp[u].e0 ? 1.f : (tp[u].e1 ? a.d1_last_f : comp[u][0]);
+              comp[u][1] = tp[u].e0 ? 0.f : (tp[u].e1 ? a.z_last_f : comp[u][1]);
+#pragma unroll
+              for (int t = 0; t < NT; t++) comp[u][2 + t] = tp[u].e0 ? a.bz0[t] : (tp[u].e1 ? 1.f : comp[u][2 + t]);
+            }
+          }
+          if (fuse) {
+            // the same float as lognormal_f32 of the fused count pass
+#pragma unroll
+            for (int u = 0; u < U; u++) dl[u] = lognormal_f32(dl[u], comp[u][0], s2f);
+#pragma unroll
+            for (int u = 0; u < U; u++) tb[(g + u) * ystep] = dl[u];
+          }
+          // shell index: FP32 z (error < 5e-5 shell) unless within 5e-4
+          // shell of an edge (or at the table ends), where the reference's
+          // FP64 radius and z decide
+          double zz[U];
+          int ind[U];
+          bool near[U], any = false;
+#pragma unroll
+          for (int u = 0; u < U; u++) {
+            zz[u] = (double)comp[u][1];
+            const float sf = comp[u][1] * a.idz_f;
+            ind[u] = (int)sf + 1;
+            near[u] = ends[u] || !(fabsf(__builtin_amdgcn_fractf(sf) - 0.5f) < 0.5f - 5e-4f);
+            any = any || near[u];
+          }
+          if (any) {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+              if (near[u]) {
+                zz[u] = cell_z_f64(a, ix, iy0 + TY * (g + u), iz);
+                ind[u] = (int)(zz[u] * a.idz) + 1;
+              }
+          }
+          float term[U][NT > 0 ? NT : 1], l2[U];
+#pragma unroll
+          for (int u = 0; u < U; u++) l2[u] = __builtin_amdgcn_logf(1.f + dl[u]);
+#pragma unroll
+          for (int t = 0; t < NT; t++) {
+            if (M0 || a.model[t] == 0) {
+#pragma unroll
+              for (int u = 0; u < U; u++) term[u][t] = bias_sum_term<0>(dl[u], l2[u], comp[u][2 + t]);
+            } else if (a.model[t] == 1) {
+#pragma unroll
+              for (int u = 0; u < U; u++) term[u][t] = bias_sum_term<1>(dl[u], l2[u], comp[u][2 + t]);
+            } else {
+#pragma unroll
+              for (int u = 0; u < U; u++) term[u][t] = bias_sum_term<2>(dl[u], l2[u], comp[u][2 + t]);
+            }
           }
 #pragma unroll
-          for (int q = 0; q < NQ; q++) comp[q] = f[2 * q] + f[2 * q + 1] * tq;
-          if (e0 || e1) {
-            comp[0] = e0 ? 1.f : a.d1_last_f;
-            comp[1] = e0 ? 0.f : a.z_last_f;
+          for (int u = 0; u < U; u++) {
+            const unsigned slot = (unsigned)(ind[u] - wb);
 #pragma unroll
-            for (int t = 0; t < NT; t++) comp[2 + t] = e0 ? a.bz0[t] : 1.f;
+            for (int k = 0; k < kRegWin; k++)
+              if (slot == (unsigned)k) {
+                rc[k]++;
+                ra[k][0] += zz[u];
+#pragma unroll
+                for (int t = 0; t < NT; t++) ra[k][1 + t] += (double)term[u][t];
+              }
           }
         }
-        if (a.fused) {
-          // the same float as lognormal_f32 of the fused count pass
-          const TabPos tp{0, bn.tq, e0, e1};
-          const float D = growth_at(tp, bn.C[0].x, bn.C[0].y, a.d1_last_f);
-          dl = lognormal_f32(dl, D, s2f);
-          tb[roff(rr)] = dl;
-        }
-        // shell index: FP32 z (error < 5e-5 shell) unless within 5e-4 shell of
-        // an edge (or at the table ends), where the reference's FP64 radius
-        // and z decide
-        double zz = (double)comp[1];
-        const float sf = comp[1] * a.idz_f;
-        int ind = (int)sf + 1;
-        const float fr = sf - floorf(sf);
-        if (e0 || e1 || !(fr > 5e-4f && fr < 1.f - 5e-4f)) {
-          zz = cell_z_f64(a, ix, iy, iz);
-          ind = (int)(zz * a.idz) + 1;
-        }
-        if (ind >= 0 && ind < nz) {
-          s = ind;
-          v[0] = 1.0;
-          v[1] = zz;
-          const float l2 = __builtin_amdgcn_logf(1.f + dl);
-          const float q = M0 ? 0.f : 1.44269504f * dl * __builtin_amdgcn_rcpf(1.f + dl);
-#pragma unroll
-          for (int t = 0; t < NT; t++)
-            v[2 + t] = (double)(M0 ? (dl > -1.f ? __builtin_amdgcn_exp2f(comp[2 + t] * l2) : 0.f)
-                                   : bias_sum_term(dl, l2, q, comp[2 + t], a.model[t]));
-        }
       }
-      const bool change = s >= 0 && s != cur;
-      // a lane whose slots are full flushes them first (wave-collective, rare)
-      if (__ballot(change && cur >= 0 && nslot == kSlots)) {
-        flush_all(nslot);
-        nslot = 0;
-      }
-      if (change) {
-        if (cur >= 0) {
+      // the window's rows into the wavefront's accumulators
+      constexpr int P = NF > 8 ? 16 : (NF > 4 ? 8 : (NF > 2 ? 4 : NF)), G = 64 / P;   // G lanes per quantity
+      const int q = lane / G, part = lane % G;
 #pragma unroll
-          for (int q = 0; q < NQ; q++) logv[((size_t)nslot * NQ + q) * 64 + lane] = cacc[q];
-          logid[nslot * 64 + lane] = cur;
-          nslot++;
-        }
-        cur = s;
+      for (int k = 0; k < kRegWin; k++) {
+        if (k >= wn || __ballot(rc[k] != 0u) == 0ull) continue;
 #pragma unroll
-        for (int q = 0; q < NQ; q++) cacc[q] = 0;
-      }
-      if (s >= 0) {
+        for (int f = 0; f < NF; f++) wsum[f * 64 + lane] = ra[k][f];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        double v = 0;
+        if (q < NF)
 #pragma unroll
-        for (int q = 0; q < NQ; q++) cacc[q] += v[q];
+          for (int j = 0; j < P; j++) v += wsum[q * 64 + G * j + part];
+        v = lanes_sum<G>(v);
+        int n = (int)rc[k];
+        for (int o = 1; o < 64; o <<= 1) n += __shfl_xor(n, o);
+        if (part == 0 && q < NF) myacc[(wb + k) * NQ + 1 + q] += v;
+        if (lane == 0) myacc[(wb + k) * NQ] += (double)n;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
       }
     }
-    // end of tile: the current shell goes into a slot (flushing first if full)
-    if (__ballot(cur >= 0 && nslot == kSlots)) {
-      flush_all(nslot);
-      nslot = 0;
-    }
-    if (cur >= 0) {
-#pragma unroll
-      for (int q = 0; q < NQ; q++) logv[((size_t)nslot * NQ + q) * 64 + lane] = cacc[q];
-      logid[nslot * 64 + lane] = cur;
-      nslot++;
-    }
-    flush_all(nslot);
   }
   __syncthreads();
   double *out = partial + (size_t)blockIdx.x * nz * NQ;
   for (int i = threadIdx.x; i < nz * NQ; i += blockDim.x) {
     double v = 0;
-    for (int w = 0; w < kWaves; w++) v += acc[(size_t)w * nz * NQ + i];
+    for (int w = 0; w < nwaves; w++) v += acc[(size_t)w * nz * NQ + i];
     out[i] = v;
   }
 }
@@ -620,18 +688,89 @@ __global__ __launch_bounds__(256) void k_norm_table(const double *__restrict__ s
   }
 }
 
-template <int NT, bool M0>
-void launch_shells(dim3 g, dim3 b, size_t lds, hipStream_t s, const ShellArgs &a, double *partial) {
-  if (lds > 64 * 1024)
-    (void)hipFuncSetAttribute((const void *)k_shells<NT, M0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL((k_shells<NT, M0>), g, b, lds, s, a, partial);
+// The tiling of a shell pass: the largest tile that spans at most kRegWin
+// shells (from its diagonal and the narrowest shell), since a tile's fixed
+// costs -- its bounds, the staging, the sums at its end -- are of the order of
+// two rows' work.  16 x 16 x 4 and 16 x 8 x 4 cells with their table bins in
+// LDS while a wavefront's LDS stays within 10 KB (16 wavefronts per CU); then
+// 8 x 4 x 8 cells, too few for the staging to pay; then 4 x 4 x 4, which span
+// the fewest shells (64^3 .. 192^3 of a deep box, where further passes may be
+// needed all the same).
+struct ShellPlan {
+  int kind, nbin, waves, blocks;
+  size_t lds;
+};
+constexpr int kShellTile[4][4] = {{4, 4, 4, 0}, {8, 4, 8, 0}, {16, 8, 4, 1}, {16, 16, 4, 1}};   // cells in x, y, z; staged
+int shell_plan(clr_ctx *c, int nz, int NT, ShellPlan &p) {
+  if (c->shell_dr <= 0) {
+    // narrowest shell below r(L/2), and whether z(r) never decreases
+    const std::vector<double> &zz = c->h_z, &rr = c->h_r;
+    const double dz = c->zmax_half_box / (nz - 2);
+    double last = 0, narrow = 1e300;
+    int k = 1;
+    c->shell_mono = 1;
+    for (int i = 1; i < c->na; i++) {
+      if (!(zz[i] >= zz[i - 1])) c->shell_mono = 0;
+      while (k < nz - 1 && zz[i] >= k * dz) {
+        narrow = std::min(narrow, rr[i] - last);
+        last = rr[i];
+        k++;
+      }
+    }
+    c->shell_dr = std::max(std::min(narrow, c->L), 1e-3 * c->dx);
+  }
+  size_t winb = 0;
+  int cells = 64;
+  for (p.kind = 3; p.kind >= 0; p.kind--) {
+    const int *t = kShellTile[p.kind];
+    const double d = c->dx * sqrt((t[0] - 1.) * (t[0] - 1.) + (t[1] - 1.) * (t[1] - 1.) + (t[2] - 1.) * (t[2] - 1.));
+    p.nbin = t[3] ? (int)std::min((double)c->na, ceil((d + 4e-5 * c->L) * c->glob_idr) + 3) : 0;
+    winb = (size_t)(1 + NT) * 64 * sizeof(double) + (size_t)p.nbin * (2 + NT) * sizeof(float2);
+    cells = t[0] * t[1] * t[2];
+    if (p.kind == 0 || (ceil(d / c->shell_dr) + 1 <= kRegWin && winb <= 10 * 1024)) break;
+  }
+  const size_t accb = (size_t)nz * (2 + NT) * sizeof(double);
+  for (p.waves = kWaves; p.waves > 1 && p.waves * (accb + winb) > 160 * 1024;) p.waves /= 2;
+  p.lds = p.waves * (accb + winb);
+  const long tiles = (long)c->N * c->N * c->N / cells;
+  p.blocks = (int)std::min<long>(kShellBlocks, (tiles + p.waves - 1) / p.waves);
+  return p.lds <= 160 * 1024 ? CLR_OK : CLR_ERR_ARG;
 }
-using ShellFn = void (*)(dim3, dim3, size_t, hipStream_t, const ShellArgs &, double *);
-#define CLR_SHELL_FNS(M0)                                                                                  \
-  {launch_shells<0, M0>, launch_shells<1, M0>, launch_shells<2, M0>, launch_shells<3, M0>, launch_shells<4, M0>, \
-   launch_shells<5, M0>, launch_shells<6, M0>, launch_shells<7, M0>, launch_shells<8, M0>}
-const ShellFn kShellFns[2][kMaxTr + 1] = {CLR_SHELL_FNS(false), CLR_SHELL_FNS(true)};
+
+template <int NT, bool M0, int TX, int ROWS, bool STAGE>
+void launch_shells(const ShellPlan &p, hipStream_t s, const ShellArgs &a, double *partial) {
+  if (p.lds > 64 * 1024)
+    (void)hipFuncSetAttribute((const void *)k_shells<NT, M0, TX, ROWS, STAGE>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds);
+  hipLaunchKernelGGL((k_shells<NT, M0, TX, ROWS, STAGE>), dim3(p.blocks), dim3(64 * p.waves), p.lds, s, a, partial);
+}
+using ShellFn = void (*)(const ShellPlan &, hipStream_t, const ShellArgs &, double *);
+#define CLR_SHELL_FNS(...)                                                                                  \
+  {launch_shells<0, __VA_ARGS__>, launch_shells<1, __VA_ARGS__>, launch_shells<2, __VA_ARGS__>,             \
+   launch_shells<3, __VA_ARGS__>, launch_shells<4, __VA_ARGS__>, launch_shells<5, __VA_ARGS__>,             \
+   launch_shells<6, __VA_ARGS__>, launch_shells<7, __VA_ARGS__>, launch_shells<8, __VA_ARGS__>}
+const ShellFn kShellFns[2][4][kMaxTr + 1] = {
+    {CLR_SHELL_FNS(false, 4, 1, false), CLR_SHELL_FNS(false, 8, 4, false), CLR_SHELL_FNS(false, 16, 8, true),
+     CLR_SHELL_FNS(false, 16, 16, true)},
+    {CLR_SHELL_FNS(true, 4, 1, false), CLR_SHELL_FNS(true, 8, 4, false), CLR_SHELL_FNS(true, 16, 8, true),
+     CLR_SHELL_FNS(true, 16, 16, true)}};
 #undef CLR_SHELL_FNS
+
+// Runs the shell pass and its fixed-order reduction (fin[nz][2 + ntr]).
+int run_shells(clr_ctx *c, hipStream_t s, ShellArgs &a, bool all0, double *partial, double *fin, hipEvent_t after) {
+  ShellPlan p;
+  const int rc = shell_plan(c, a.nz, a.ntr, p);
+  if (rc) return clr_fail(c, rc, "too many shells x tracers (%d x %d)", a.nz, a.ntr);
+  a.nbin = p.nbin;
+  a.mono = c->shell_mono;
+  kShellFns[all0 ? 1 : 0][p.kind][a.ntr](p, s, a, partial);
+  CLR_HIP(c, hipGetLastError());
+  if (after) CLR_HIP(c, hipEventRecord(after, s));
+  const int nvals = a.nz * (2 + a.ntr);
+  hipLaunchKernelGGL(k_shell_final, dim3((unsigned)nvals), dim3(256), 0, s, partial, p.blocks, nvals, fin);
+  CLR_HIP(c, hipGetLastError());
+  return CLR_OK;
+}
 
 }  // namespace
 
@@ -664,7 +803,7 @@ int clr_launch_density(clr_ctx *c, int dens_type, double sigma2) {
 // through the address hipGetSymbolAddress returns on that device.
 // ---------------------------------------------------------------------------
 constexpr size_t kNoAllocVals = 320;
-constexpr size_t kNoAllocTabFloat4 = (size_t)CLR_NA * shell_tab_w(kMaxTr);
+constexpr size_t kNoAllocTabFloat4 = (size_t)CLR_NA * (2 + kMaxTr) / 2;
 constexpr size_t kNoAllocDoubles = (size_t)kShellBlocks * kNoAllocVals + kNoAllocVals + 2 * (size_t)kNormMaxShells +
                                    2 * (size_t)kMaxTr;
 constexpr size_t kNoAllocBytes = (kNoAllocDoubles * sizeof(double) + 255) / 256 * 256 + kNoAllocTabFloat4 * 16;
@@ -736,28 +875,26 @@ int clr_launch_norms(clr_ctx *c, int lognormal_fused, double sigma2, int cap, in
   a.d1_last_f = (float)c->h_bg_last[2];
   a.idr_f = (float)c->glob_idr;
   const int nq = 2 + ntr;
-  static size_t (*const kLds[kMaxTr + 1])(int) = {shell_lds_bytes<0>, shell_lds_bytes<1>, shell_lds_bytes<2>,
-                                                   shell_lds_bytes<3>, shell_lds_bytes<4>, shell_lds_bytes<5>,
-                                                   shell_lds_bytes<6>, shell_lds_bytes<7>, shell_lds_bytes<8>};
-  const size_t lds = kLds[ntr](nz);
-  if (lds > 160 * 1024) return clr_fail(c, CLR_ERR_ARG, "too many shells x tracers (%d x %d)", nz, ntr);
+  {
+    ShellPlan plan;
+    if (shell_plan(c, nz, ntr, plan)) return clr_fail(c, CLR_ERR_ARG, "too many shells x tracers (%d x %d)", nz, ntr);
+  }
   bool all0 = true;
   for (int t = 0; t < ntr; t++) all0 = all0 && a.model[t] == CLR_BIAS_EXPONENTIAL;
   const size_t nvals = (size_t)nz * nq;
-  const int w = shell_tab_w(ntr);
   double *partial, *fin, *work;
-  float4 *tab;
+  float2 *tab;
   if (scratch_base) {
     // no allocation: everything in the device's static scratch
     if (nvals > kNoAllocVals)
       return clr_fail(c, CLR_ERR_ARG, "%d shells x (2 + %d tracers) = %zu values exceed the %zu of the static scratch",
                       nz, ntr, nvals, kNoAllocVals);
-    if ((size_t)na * w > kNoAllocTabFloat4)
+    if ((size_t)na * nq > 2 * kNoAllocTabFloat4)
       return clr_fail(c, CLR_ERR_ARG, "r-tables of %d entries exceed the static scratch", na);
     partial = (double *)scratch_base;
     fin = partial + (size_t)kShellBlocks * nvals;
     work = fin + nvals;
-    tab = (float4 *)((char *)scratch_base + (kNoAllocDoubles * sizeof(double) + 255) / 256 * 256);
+    tab = (float2 *)((char *)scratch_base + (kNoAllocDoubles * sizeof(double) + 255) / 256 * 256);
   } else {
     const size_t need = (size_t)kShellBlocks * nvals + nvals + 2 * nz + 2 * ntr;
     int rc = clr_ensure(c, (void **)&c->red, &c->red_n, need * sizeof(double));
@@ -765,22 +902,20 @@ int clr_launch_norms(clr_ctx *c, int lognormal_fused, double sigma2, int cap, in
     partial = c->red;
     fin = c->red + (size_t)kShellBlocks * nvals;
     work = fin + nvals;
-    rc = clr_ensure(c, &c->misc, &c->misc_n, (size_t)na * w * sizeof(float4));
+    rc = clr_ensure(c, &c->misc, &c->misc_n, (size_t)na * nq * sizeof(float2));
     if (rc) return rc;
-    tab = (float4 *)c->misc;
+    tab = (float2 *)c->misc;
   }
   a.tab = tab;
 
   CLR_HIP(c, hipEventRecord(c->ev0, c->stream));
-  hipLaunchKernelGGL(k_pack_shell_table, dim3((na + 255) / 256), dim3(256), 0, c->stream, tsrc, ntr, na, tab);
+  hipLaunchKernelGGL(k_pack_shell_table, dim3((na + 255) / 256, nq), dim3(256), 0, c->stream, tsrc, na, tab);
   CLR_HIP(c, hipGetLastError());
   CLR_HIP(c, hipEventRecord(c->ev2, c->stream));
-  kShellFns[all0 ? 1 : 0][ntr](dim3(kShellBlocks), dim3(kShellThreads), lds, c->stream, a, partial);
-  CLR_HIP(c, hipGetLastError());
-  CLR_HIP(c, hipEventRecord(c->ev3, c->stream));
-  hipLaunchKernelGGL(k_shell_final, dim3((unsigned)nvals), dim3(256), 0, c->stream, partial, kShellBlocks,
-                     (int)nvals, fin);
-  CLR_HIP(c, hipGetLastError());
+  {
+    const int rc = run_shells(c, c->stream, a, all0, partial, fin, c->ev3);
+    if (rc) return rc;
+  }
   if (ntr > 0) {
     NormOuts outs{};
     for (int t = 0; t < ntr; t++) {
@@ -874,19 +1009,16 @@ template <int NT>
 int shell_pass_to_host(clr_ctx *c, ShellArgs &a, const ShellTabSrc &tsrc, int nz, std::vector<double> &h) {
   const int na = c->na, nq = 2 + NT;
   const size_t nvals = (size_t)nz * nq;
-  const int w = shell_tab_w(NT);
   int rc = clr_ensure(c, (void **)&c->red, &c->red_n, ((size_t)kShellBlocks * nvals + nvals) * sizeof(double));
   if (rc) return rc;
   double *partial = c->red, *fin = c->red + (size_t)kShellBlocks * nvals;
-  rc = clr_ensure(c, &c->misc, &c->misc_n, (size_t)na * w * sizeof(float4));
+  rc = clr_ensure(c, &c->misc, &c->misc_n, (size_t)na * nq * sizeof(float2));
   if (rc) return rc;
-  a.tab = (const float4 *)c->misc;
-  hipLaunchKernelGGL(k_pack_shell_table, dim3((na + 255) / 256), dim3(256), 0, c->stream, tsrc, NT, na,
-                     (float4 *)c->misc);
-  launch_shells<NT, true>(dim3(kShellBlocks), dim3(kShellThreads), shell_lds_bytes<NT>(nz), c->stream, a, partial);
-  hipLaunchKernelGGL(k_shell_final, dim3((unsigned)nvals), dim3(256), 0, c->stream, partial, kShellBlocks,
-                     (int)nvals, fin);
-  CLR_HIP(c, hipGetLastError());
+  a.tab = (const float2 *)c->misc;
+  hipLaunchKernelGGL(k_pack_shell_table, dim3((na + 255) / 256, nq), dim3(256), 0, c->stream, tsrc, na,
+                     (float2 *)c->misc);
+  rc = run_shells(c, c->stream, a, true, partial, fin, nullptr);
+  if (rc) return rc;
   h.resize(nvals);
   CLR_HIP(c, hipMemcpyAsync(h.data(), fin, nvals * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   CLR_HIP(c, hipStreamSynchronize(c->stream));
@@ -1066,7 +1198,7 @@ int clr_prepare_norms(clr_ctx *c) {
   int rc = clr_ensure(c, (void **)&c->red, &c->red_n,
                       ((size_t)kShellBlocks * nvals + nvals + 2 * nz + 2 * ntr) * sizeof(double));
   if (rc) return rc;
-  rc = clr_ensure(c, &c->misc, &c->misc_n, (size_t)c->na * shell_tab_w(ntr) * sizeof(float4));
+  rc = clr_ensure(c, &c->misc, &c->misc_n, (size_t)c->na * (2 + ntr) * sizeof(float2));
   if (rc) return rc;
   for (int t = 0; t < ntr; t++) {
     TracerDev &T = c->tr[tk[t]][tp[t]];
@@ -1124,14 +1256,13 @@ int clr_enqueue_norms(clr_ctx *c, hipStream_t st, const double *sigma2_dev) {
   a.idz_f = (float)a.idz;
   a.d1_last_f = (float)c->h_bg_last[2];
   a.idr_f = (float)c->glob_idr;
-  a.tab = (const float4 *)c->misc;
-  static size_t (*const kLds[kMaxTr + 1])(int) = {shell_lds_bytes<0>, shell_lds_bytes<1>, shell_lds_bytes<2>,
-                                                   shell_lds_bytes<3>, shell_lds_bytes<4>, shell_lds_bytes<5>,
-                                                   shell_lds_bytes<6>, shell_lds_bytes<7>, shell_lds_bytes<8>};
+  a.tab = (const float2 *)c->misc;
   double *partial = c->red, *fin = c->red + (size_t)kShellBlocks * nvals, *work = fin + nvals;
-  hipLaunchKernelGGL(k_pack_shell_table, dim3((na + 255) / 256), dim3(256), 0, st, tsrc, ntr, na, (float4 *)c->misc);
-  kShellFns[all0 ? 1 : 0][ntr](dim3(kShellBlocks), dim3(kShellThreads), kLds[ntr](nz), st, a, partial);
-  hipLaunchKernelGGL(k_shell_final, dim3((unsigned)nvals), dim3(256), 0, st, partial, kShellBlocks, (int)nvals, fin);
+  hipLaunchKernelGGL(k_pack_shell_table, dim3((na + 255) / 256, nq), dim3(256), 0, st, tsrc, na, (float2 *)c->misc);
+  {
+    const int rc = run_shells(c, st, a, all0, partial, fin, nullptr);
+    if (rc) return rc;
+  }
   hipLaunchKernelGGL(k_norm_table, dim3((unsigned)((na + 255) / 256), (unsigned)ntr), dim3(256), 0, st, fin, nz, nq,
                      zmax, c->bg, c->bg + na, c->glob_idr, c->r_last, c->h_bg_last[1], na, outs, work + 2 * nz);
   CLR_HIP(c, hipGetLastError());

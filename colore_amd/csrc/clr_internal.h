@@ -72,6 +72,8 @@ struct clr_ctx {
   double r_last = 0;
   double h_bg_first[6] = {0}, h_bg_last[6] = {0};   // first/last entries of each bg table
   double zmax_half_box = 0;                           // z(L/2), get_bg(L/2, BG_Z)
+  double shell_dr = 0;      // narrowest normalisation shell below r(L/2) (0: not computed yet)
+  int shell_mono = 0;       // z(r) never decreases
   int32_t *r2n = nullptr;   // RING -> NEST table at r2n_nside
   int r2n_nside = 0;
   double *pk = nullptr;     // logkarr[numk], pkarr[numk]
