@@ -129,6 +129,8 @@ struct clr_ctx {
   size_t tidal_n = 0;
   void *velrec = nullptr;    // velocity-difference + density records, 4 floats per cell (clr_los.hip)
   size_t velrec_n = 0;
+  void *lpt_ws = nullptr;    // clr_lpt_density's grids (clr_lpt.hip)
+  size_t lpt_ws_n = 0;
   std::string los_plan;
   void *los_buf = nullptr;
   size_t los_buf_n = 0;

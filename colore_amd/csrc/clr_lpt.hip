@@ -8,11 +8,11 @@
 // place); 2LPT adds the six digradients, the second-order source and its
 // displacement.  The transforms are the project's own (clr_fft3d: the
 // Stockham engine of the field stage, run forward as the conjugate of the
-// inverse transform of the conjugate).  One thread per grid cell then
-// computes the cell's particle position (FP32 as the reference stores it,
-// wrapped into the box), one thread per particle adds its NGP, CIC or TSC
-// weights to the zeroed density grid with FP32 atomics, and a last pass
-// subtracts 1.
+// inverse transform of the conjugate).  The particles' positions (one per
+// cell, FP32 as the reference stores it, wrapped into the box) then put their
+// CIC or TSC weights into their tile's region in LDS, and a last pass adds the
+// regions and subtracts 1; NGP and grids below 64^3 add to the zeroed density
+// grid with FP32 atomics.
 #include "clr_internal.h"
 #include <math.h>
 #include <vector>
@@ -144,17 +144,10 @@ __device__ inline int wrapn(int v, int N) {
   return v;
 }
 
-// one thread per cell: the particle's position x + D1 psi1 (+ D2 psi2) +
-// x_obs, FP32, wrapped into [0, L) (density.c:481-505, 852-875)
-__global__ __launch_bounds__(256) void k_lpt_pos(PosArgs a) {
+// The position of cell (ix,iy,iz)'s particle: x + D1 psi1 (+ D2 psi2) + x_obs,
+// FP32, wrapped into [0, L) (density.c:481-505, 852-875).
+__device__ inline void lpt_position(const PosArgs &a, int ix, int iy, int iz, size_t idx, float p[3]) {
 #pragma clang fp contract(off)
-  const int N = a.N;
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)N * N * N) return;
-  const int ix = (int)(t % N);
-  const long long rw = t / N;
-  const int iy = (int)(rw % N), iz = (int)(rw / N);
-  const size_t idx = (size_t)ix + (size_t)a.ngx * (size_t)rw;
   float xv[3];
   xv[0] = (float)((ix + 0.0) * (double)a.dxf - a.ox);
   xv[1] = (float)((iy + 0.0) * (double)a.dxf - a.oy);
@@ -164,7 +157,6 @@ __global__ __launch_bounds__(256) void k_lpt_pos(PosArgs a) {
   const double dg = f_of_r(a.r_arr, a.dd1, a.idr, a.r_last, r, 1.0, a.d1_last);
   const double obs[3] = {a.ox, a.oy, a.oz};
   const float d[3] = {a.d0[idx], a.d1[idx], a.d2[idx]};
-  float p[3];
   if (a.s0) {
     const double d2g = f_of_r(a.r_arr, a.dd2, a.idr, a.r_last, r, a.d2_first, a.d2_last);
     const float s[3] = {a.s0[idx], a.s1[idx], a.s2[idx]};
@@ -179,6 +171,20 @@ __global__ __launch_bounds__(256) void k_lpt_pos(PosArgs a) {
     if (p[ax] < 0) p[ax] = (float)(p[ax] + a.L);
     if (p[ax] >= a.L) p[ax] = (float)(p[ax] - a.L);
   }
+}
+
+// one thread per cell: the particle's position, stored (the positions of
+// clr_lpt_density's pos_out and of the untiled deposits)
+__global__ __launch_bounds__(256) void k_lpt_pos(PosArgs a) {
+  const int N = a.N;
+  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= (long long)N * N * N) return;
+  const int ix = (int)(t % N);
+  const long long rw = t / N;
+  const int iy = (int)(rw % N), iz = (int)(rw / N);
+  const size_t idx = (size_t)ix + (size_t)a.ngx * (size_t)rw;
+  float p[3];
+  lpt_position(a, ix, iy, iz, idx, p);
   a.p0[idx] = p[0];
   a.p1[idx] = p[1];
   a.p2[idx] = p[2];
@@ -242,31 +248,42 @@ __global__ __launch_bounds__(256) void k_lpt_deposit(const float *__restrict__ p
   }
 }
 
-// The same CIC / TSC assignment with the weights first summed in LDS: a
-// block takes a 16^3 tile of particles (16 per thread) and holds the grid
-// region of the tile grown by 2 cells on every side (20^3 floats, 32 KB, so
-// that several blocks share a CU); weights landing in the region go to LDS,
-// the ones further out straight to the grid, and the region is then added to
-// the grid once (about 2 global atomics per particle instead of 8 for CIC, 27
-// for TSC).  Tiles of 32 x 16 x 16 with 4-cell margins (90 KB, two blocks
-// per CU) took 8 ms more for a 1024^3 CIC deposit; tiles from 8^3 to
-// 32 x 8 x 8 with 1- to 3-cell margins came within 1 ms of this one.  Needs N >= 64 and
-// N a multiple of 16, so that the region never wraps onto itself.
-constexpr int kDTX = 16, kDTY = 16, kDTZ = 16, kDHalo = 2;
-constexpr int kDRX = kDTX + 2 * kDHalo, kDRY = kDTY + 2 * kDHalo, kDRZ = kDTZ + 2 * kDHalo;
-constexpr size_t kDepositLds = (size_t)kDRX * kDRY * kDRZ * sizeof(float);
+// The same CIC / TSC assignment with the weights summed in LDS: a block takes a
+// 16^3 tile of particles and holds the grid region of the tile grown by 2
+// cells on every side (20^3); weights landing in the region go to LDS, the few
+// further out straight to the zeroed grid.  The region is then stored as FP32,
+// in whole lines, to the block's own part of `regs`, and k_lpt_gather adds the
+// up to eight regions that cover a cell.  The positions are computed here
+// (STORED: read, where the caller wanted them stored), which saves their
+// 3 x 4 bytes per particle written and read again (1.0 ms at 512^3).
+// R is the region's type.  double (64 KB, two blocks of 512 threads per CU):
+// a wavefront's ds_add_f64 takes 9 clocks of the CU's LDS, its ds_add_f32 194,
+// conflict-free or not -- with float the LDS adds alone took 4.5 of the
+// deposit's 5.6 ms at 512^3 (CIC; 17 ms for TSC).  The whole 1LPT density at
+// 512^3 took 10.55 ms (TSC 23.4) and takes 5.67 (6.39); this kernel is now
+// bound by the positions' FP64 chain and their loads.  Below 256^3 the region
+// stays float (256 threads): norms of shells of a few hundred cells keep the
+// rounding of FP32 sums in this order to 1e-9, and FP64 sums (more exact, 0.28
+// -> 0.02 ms at 128^3, TSC) move them by 2e-9.
+// Needs N >= 64 and N a multiple of 16, so that a region never wraps onto
+// itself.
+constexpr int kDT = 16, kDHalo = 2, kDR = kDT + 2 * kDHalo;
+constexpr int kDRegion = kDR * kDR * kDR;
+constexpr int kDWideN = 256;   // FP64 regions from this grid size on
 
-__global__ __launch_bounds__(256) void k_lpt_deposit_tiled(const float *__restrict__ px, const float *__restrict__ py,
-                                                           const float *__restrict__ pz, float *__restrict__ g,
-                                                           int N, int ngxi, float iag, int interp) {
+template <class R, bool CIC, bool STORED>
+__global__ __launch_bounds__(64 * sizeof(R)) void k_lpt_deposit_tiled(PosArgs a, float *__restrict__ g, float *__restrict__ regs,
+                                                           float iag) {
 #pragma clang fp contract(off)
-  extern __shared__ float reg[];
-  const size_t ngx = (size_t)ngxi, pl = (size_t)N * ngx;
-  const int ntx = N / kDTX, nty = N / kDTY;
+  constexpr int kDThreads = 64 * sizeof(R);
+  __shared__ R reg[kDRegion];
+  const int N = a.N;
+  const size_t ngx = (size_t)a.ngx, pl = (size_t)N * ngx;
+  const int nt = N / kDT;
   const int b = blockIdx.x;
-  const int tx = b % ntx, ty = (b / ntx) % nty, tz = b / (ntx * nty);
-  const int ox = tx * kDTX - kDHalo, oy = ty * kDTY - kDHalo, oz = tz * kDTZ - kDHalo;
-  for (int i = threadIdx.x; i < kDRX * kDRY * kDRZ; i += blockDim.x) reg[i] = 0.f;
+  const int tx = b % nt, ty = (b / nt) % nt, tz = b / (nt * nt);
+  const int ox = tx * kDT - kDHalo, oy = ty * kDT - kDHalo, oz = tz * kDT - kDHalo;
+  for (int i = threadIdx.x; i < kDRegion; i += kDThreads) reg[i] = 0;
   __syncthreads();
   // relative coordinate of cell c in the region along one axis (c in [0, N))
   auto rel = [N](int c, int o) {
@@ -275,62 +292,130 @@ __global__ __launch_bounds__(256) void k_lpt_deposit_tiled(const float *__restri
     if (d >= N) d -= N;
     return d;
   };
-  auto add = [&](int cx, int cy, int cz, float w) {
-    const int rx = rel(cx, ox), ry = rel(cy, oy), rz = rel(cz, oz);
-    if (rx < kDRX && ry < kDRY && rz < kDRZ) atomicAdd(&reg[rx + kDRX * (ry + kDRY * rz)], w);
-    else atomicAdd(g + cx + ngx * cy + pl * cz, w);
-  };
-  for (int q = threadIdx.x; q < kDTX * kDTY * kDTZ; q += blockDim.x) {
-    const int lx = q % kDTX, ly = (q / kDTX) % kDTY, lz = q / (kDTX * kDTY);
-    const size_t idx = (size_t)(tx * kDTX + lx) + ngx * ((size_t)(ty * kDTY + ly) + (size_t)N * (tz * kDTZ + lz));
-    const float p[3] = {px[idx], py[idx], pz[idx]};
-    if (interp == 1) {
-      int i0[3], i1[3];
-      float a0[3], a1[3];
-#pragma unroll
-      for (int ax = 0; ax < 3; ax++) {
-        const float xs = p[ax] * iag;
-        const int c = (int)xs;
-        a1[ax] = xs - c;
-        a0[ax] = 1 - a1[ax];
-        i0[ax] = wrapn(c, N);
-        i1[ax] = wrapn(c + 1, N);
-      }
-#pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const int bx = c & 1, by = (c >> 1) & 1, bz = c >> 2;
-        add(bx ? i1[0] : i0[0], by ? i1[1] : i0[1], bz ? i1[2] : i0[2],
-            (bx ? a1[0] : a0[0]) * (by ? a1[1] : a0[1]) * (bz ? a1[2] : a0[2]));
-      }
+  const int lx = threadIdx.x % kDT, ly = threadIdx.x / kDT % kDT;
+  const int ix = tx * kDT + lx, iy = ty * kDT + ly;
+  for (int lz = threadIdx.x / (kDT * kDT); lz < kDT; lz += kDThreads / (kDT * kDT)) {
+    const int iz = tz * kDT + lz;
+    const size_t idx = (size_t)ix + ngx * ((size_t)iy + (size_t)N * iz);
+    float p[3];
+    if (STORED) {
+      p[0] = a.p0[idx];
+      p[1] = a.p1[idx];
+      p[2] = a.p2[idx];
     } else {
-      int ic[3][3];
-      float wt[3][3];
+      lpt_position(a, ix, iy, iz, idx, p);
+    }
+    constexpr int S = CIC ? 2 : 3;
+    int c0[3], cell[3][S];
+    float wt[3][S];
+    const int o[3] = {ox, oy, oz};
+    bool in = true;   // every weight of the particle falls in the region
+    int r0[3];
 #pragma unroll
-      for (int ax = 0; ax < 3; ax++) {
-        const float xs = p[ax] * iag;
+    for (int ax = 0; ax < 3; ax++) {
+      const float xs = p[ax] * iag;
+      if (CIC) {
+        const int c = (int)xs;
+        wt[ax][1] = xs - c;
+        wt[ax][0] = 1 - wt[ax][1];
+        c0[ax] = c;
+      } else {
         const int i0 = (int)floorf((float)((double)xs + 0.5));
         const float d = xs - i0;
         wt[ax][0] = (float)(0.5 * (0.5 - d) * (0.5 - d));
-        wt[ax][2] = (float)(0.5 * (0.5 + d) * (0.5 + d));
+        wt[ax][S - 1] = (float)(0.5 * (0.5 + d) * (0.5 + d));
         wt[ax][1] = (float)(0.75 - d * d);
-        ic[ax][0] = wrapn(i0 - 1, N);
-        ic[ax][1] = wrapn(i0, N);
-        ic[ax][2] = wrapn(i0 + 1, N);
+        c0[ax] = i0 - 1;
       }
-      for (int sz = 0; sz < 3; sz++)
-        for (int sy = 0; sy < 3; sy++)
+      r0[ax] = rel(wrapn(c0[ax], N), o[ax]);
+      in = in && r0[ax] <= kDR - S;
+    }
+    if (in) {
+      R *const q = reg + r0[0] + kDR * (r0[1] + kDR * r0[2]);
 #pragma unroll
-          for (int sx = 0; sx < 3; sx++)
-            add(ic[0][sx], ic[1][sy], ic[2][sz], wt[0][sx] * wt[1][sy] * wt[2][sz]);
+      for (int sz = 0; sz < S; sz++)
+#pragma unroll
+        for (int sy = 0; sy < S; sy++)
+#pragma unroll
+          for (int sx = 0; sx < S; sx++)
+            atomicAdd(q + sx + kDR * (sy + kDR * sz), (R)(wt[0][sx] * wt[1][sy] * wt[2][sz]));
+    } else {
+#pragma unroll
+      for (int ax = 0; ax < 3; ax++)
+#pragma unroll
+        for (int k = 0; k < S; k++) cell[ax][k] = wrapn(c0[ax] + k, N);
+      for (int sz = 0; sz < S; sz++)
+        for (int sy = 0; sy < S; sy++)
+#pragma unroll
+          for (int sx = 0; sx < S; sx++) {
+            const float w = wt[0][sx] * wt[1][sy] * wt[2][sz];
+            const int rx = rel(cell[0][sx], ox), ry = rel(cell[1][sy], oy), rz = rel(cell[2][sz], oz);
+            if (rx < kDR && ry < kDR && rz < kDR) atomicAdd(&reg[rx + kDR * (ry + kDR * rz)], (R)w);
+            else atomicAdd(g + cell[0][sx] + ngx * cell[1][sy] + pl * cell[2][sz], w);
+          }
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < kDRX * kDRY * kDRZ; i += blockDim.x) {
-    const float v = reg[i];
-    if (v == 0.f) continue;
-    const int rx = i % kDRX, ry = (i / kDRX) % kDRY, rz = i / (kDRX * kDRY);
-    const int cx = wrapn(ox + rx, N), cy = wrapn(oy + ry, N), cz = wrapn(oz + rz, N);
-    atomicAdd(g + cx + ngx * cy + pl * cz, v);
+  float4 *const out = (float4 *)(regs + (size_t)b * kDRegion);
+  for (int i = threadIdx.x; i < kDRegion / 4; i += kDThreads) {
+    const R *r = reg + 4 * i;
+    out[i] = make_float4((float)r[0], (float)r[1], (float)r[2], (float)r[3]);
+  }
+}
+
+// delta = rho - 1 (density.c:609-622): per cell what went straight to the
+// grid plus the regions that cover it (its own tile's and, within 2 cells of a
+// face, the neighbours'), in a fixed order.
+__global__ __launch_bounds__(256) void k_lpt_gather(const float *__restrict__ regs, float *__restrict__ g, int N,
+                                                    int ngx) {
+  const int nt = N / kDT;
+  const int b = blockIdx.x;
+  const int tx = b % nt, ty = (b / nt) % nt, tz = b / (nt * nt);
+  const int lx = threadIdx.x % kDT, ly = threadIdx.x / kDT;
+  // along one axis: a cell's places (tile, index) in its own and a neighbour's region
+  auto other = [nt](int t, int l, int &t2, int &r2) {
+    if (l < kDHalo) {
+      t2 = t == 0 ? nt - 1 : t - 1;
+      r2 = l + kDT + kDHalo;
+      return true;
+    }
+    t2 = t == nt - 1 ? 0 : t + 1;
+    r2 = l - kDT + kDHalo;
+    return l >= kDT - kDHalo;
+  };
+  int txn, rxn, tyn, ryn;
+  const bool bx = other(tx, lx, txn, rxn), by = other(ty, ly, tyn, ryn);
+  float *const col = g + (size_t)(tx * kDT + lx) + (size_t)ngx * ((size_t)(ty * kDT + ly) + (size_t)N * (tz * kDT));
+  const size_t pl = (size_t)N * ngx;
+  // the four (x, y) places, the cell's own first; 16 cells along z from each
+  const float *src[4];
+  bool on[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const bool kx = k & 1, ky = k >> 1;
+    on[k] = (!kx || bx) && (!ky || by);
+    src[k] = regs + (size_t)((kx ? txn : tx) + nt * (ky ? tyn : ty)) * kDRegion + (kx ? rxn : lx + kDHalo) +
+             kDR * (ky ? ryn : ly + kDHalo);
+  }
+  const size_t tstep = (size_t)nt * nt * kDRegion;
+#pragma unroll
+  for (int z0 = 0; z0 < kDT; z0 += 8) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = col[(size_t)(z0 + j) * pl];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (!on[k]) continue;
+#pragma unroll
+      for (int j = 0; j < 8; j++) v[j] += src[k][tstep * tz + (size_t)kDR * kDR * (z0 + j + kDHalo)];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {   // z0 + j is known: planes 0, 1, 14, 15 of the tile
+        int tzn, rzn;
+        if (other(tz, z0 + j, tzn, rzn)) v[j] += src[k][tstep * tzn + (size_t)kDR * kDR * rzn];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++) col[(size_t)(z0 + j) * pl] = v[j] - 1.f;
   }
 }
 
@@ -344,8 +429,28 @@ __global__ __launch_bounds__(256) void k_lpt_norm(float *__restrict__ g, int N, 
   g[idx] = (float)(g[idx] * 1.0f - 1.);
 }
 
+template <class R>
+void launch_deposit(dim3 g, hipStream_t s, const PosArgs &a, float *dens, float *regs, float iag, bool cic, bool stored) {
+  const dim3 b(64 * sizeof(R));
+  if (cic && stored) hipLaunchKernelGGL((k_lpt_deposit_tiled<R, true, true>), g, b, 0, s, a, dens, regs, iag);
+  else if (cic) hipLaunchKernelGGL((k_lpt_deposit_tiled<R, true, false>), g, b, 0, s, a, dens, regs, iag);
+  else if (stored) hipLaunchKernelGGL((k_lpt_deposit_tiled<R, false, true>), g, b, 0, s, a, dens, regs, iag);
+  else hipLaunchKernelGGL((k_lpt_deposit_tiled<R, false, false>), g, b, 0, s, a, dens, regs, iag);
+}
 
 }  // namespace
+
+// Gives the LPT workspace back: always, or when it is more than a quarter of
+// what would then be free (allocating it anew for each call took 2 ms at
+// 128^3 and up to 35 ms at 512^3).
+static void lpt_release(clr_ctx *c, bool always) {
+  size_t fr = 0, tot = 0;
+  if (!c->lpt_ws) return;
+  if (!always && hipMemGetInfo(&fr, &tot) == hipSuccess && c->lpt_ws_n <= (fr + c->lpt_ws_n) / 4) return;
+  (void)hipFree(c->lpt_ws);
+  c->lpt_ws = nullptr;
+  c->lpt_ws_n = 0;
+}
 
 int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
   if (!c->have_fields) return clr_fail(c, CLR_ERR_STATE, "clr_gaussian_fields must run first");
@@ -359,13 +464,32 @@ int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
   // the six digradients, whose first three become psi2 and last three hold
   // the positions
   const int nbuf = order == 1 ? 3 : 8;
-  float *ps[8] = {nullptr};
-  for (int i = 0; i < nbuf; i++) {
-    if (hipMalloc((void **)&ps[i], gbytes) != hipSuccess) {
-      for (int j = 0; j < i; j++) (void)hipFree(ps[j]);
-      return clr_fail(c, CLR_ERR_HIP, "out of device memory for the LPT grids");
+  const bool tiled = interp != 0 && N >= 64 && N % kDT == 0;
+  const size_t reg_bytes = (size_t)(N / kDT) * (N / kDT) * (N / kDT) * kDRegion * sizeof(float);
+  // one workspace for the grids and the tiles' regions, kept for the next call
+  // (lpt_release).  The regions need 1.95 grids: 2LPT has them free by then,
+  // 1LPT asks for two more grids and without them stores the positions and
+  // deposits with atomics.
+  const size_t need = gbytes * nbuf + (tiled && order == 1 ? reg_bytes : 0);
+  bool own_regs = tiled;
+  if (c->lpt_ws_n < need) {
+    lpt_release(c, true);
+    if (hipMalloc(&c->lpt_ws, need) == hipSuccess) {
+      c->lpt_ws_n = need;
+    } else {
+      (void)hipGetLastError();
+      own_regs = tiled && order == 2;
+      if (hipMalloc(&c->lpt_ws, gbytes * nbuf) != hipSuccess) {
+        (void)hipGetLastError();
+        c->lpt_ws = nullptr;
+        return clr_fail(c, CLR_ERR_HIP, "out of device memory for the LPT grids");
+      }
+      c->lpt_ws_n = gbytes * nbuf;
     }
   }
+  float *ps[8] = {nullptr};
+  for (int i = 0; i < nbuf; i++) ps[i] = (float *)((char *)c->lpt_ws + gbytes * i);
+  float *regs = nullptr;
   int rc = CLR_OK, fr = CLR_OK;   // fr: the first transform error
   hipError_t e = hipSuccess;
   const long long modes = (long long)N * N * NH, cells = (long long)N * N * N;
@@ -419,8 +543,8 @@ int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
       pos[i] = g[3 + i];
     }
   }
-  if (ok()) {
-    PosArgs a{};
+  PosArgs a{};
+  {
     a.d0 = dsp[0];
     a.d1 = dsp[1];
     a.d2 = dsp[2];
@@ -445,6 +569,10 @@ int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
     a.dxf = (float)(c->L / N);
     a.N = N;
     a.ngx = ngx;
+  }
+  // positions stored only where they are asked for or the deposit reads them
+  const bool stored = pos_out || !own_regs || order == 2;
+  if (ok() && stored) {
     hipLaunchKernelGGL(k_lpt_pos, gc, blk, 0, c->stream, a);
     e = hipGetLastError();
   }
@@ -459,30 +587,29 @@ int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
         for (size_t i = 0; i < plane.size(); i++) pos_out[3 * i + ax] = plane[i];
     }
   }
+  // 1LPT: the regions follow the three grids.  2LPT: the positions are stored
+  // (in the last digradients) and the regions take the first-order grids; the
+  // density grid held psi_z until then
   if (ok()) e = hipMemsetAsync(c->dens, 0, gbytes, c->stream);
   if (ok()) {
-    if (interp != 0 && N >= 64 && N % kDTX == 0) {
-      e = hipFuncSetAttribute((const void *)k_lpt_deposit_tiled, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kDepositLds);
-      const unsigned tiles = (unsigned)((N / kDTX) * (N / kDTY) * (N / kDTZ));
-      if (e == hipSuccess)
-        hipLaunchKernelGGL(k_lpt_deposit_tiled, dim3(tiles), blk, kDepositLds, c->stream, pos[0], pos[1], pos[2],
-                           c->dens, N, ngx, (float)(N / c->L), interp);
+    const float iag = (float)(N / c->L);
+    if (own_regs) {
+      regs = order == 1 ? ps[0] + 3 * (gbytes / sizeof(float)) : ps[0];
+      const dim3 gt((unsigned)((N / kDT) * (N / kDT) * (N / kDT)));
+      if (N >= kDWideN) launch_deposit<double>(gt, c->stream, a, c->dens, regs, iag, interp == 1, stored);
+      else launch_deposit<float>(gt, c->stream, a, c->dens, regs, iag, interp == 1, stored);
+      hipLaunchKernelGGL(k_lpt_gather, gt, blk, 0, c->stream, regs, c->dens, N, ngx);
     } else {
-      hipLaunchKernelGGL(k_lpt_deposit, gc, blk, 0, c->stream, pos[0], pos[1], pos[2], c->dens, N, ngx,
-                         (float)(N / c->L), interp);
+      hipLaunchKernelGGL(k_lpt_deposit, gc, blk, 0, c->stream, pos[0], pos[1], pos[2], c->dens, N, ngx, iag, interp);
+      hipLaunchKernelGGL(k_lpt_norm, gc, blk, 0, c->stream, c->dens, N, ngx);
     }
-    if (e == hipSuccess) e = hipGetLastError();
-  }
-  if (ok()) {
-    hipLaunchKernelGGL(k_lpt_norm, gc, blk, 0, c->stream, c->dens, N, ngx);
     e = hipGetLastError();
   }
   if (ok()) e = hipEventRecord(c->ev1, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (fr != CLR_OK) rc = fr;   // clr_fft3d has set the message
   else if (e != hipSuccess) rc = clr_fail(c, CLR_ERR_HIP, "LPT: %s", hipGetErrorString(e));
-  for (int i = 0; i < nbuf; i++) (void)hipFree(ps[i]);
+  lpt_release(c, false);
   if (rc) return rc;
   float ms = 0;
   hipEventElapsedTime(&ms, c->ev0, c->ev1);
