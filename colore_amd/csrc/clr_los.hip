@@ -2,14 +2,18 @@
 // isw_get_beam_properties (isw.c:78-147) on gfx950.
 //
 // One thread per HEALPix pixel (NEST order, so neighbouring lanes march
-// neighbouring rays and their stencil reads share cache lines).  The march
-// uses nr = N/2 radial steps of dr = r_max/nr (get_radial_params,
-// common.c:333-337); at each step the NGP cell of (rm u + x_obs)/dx is read
-// (interpolate_from_grid, beaming.c:120-268, periodic in x, y and z on one
-// GPU).  kappa: transverse trace of the 19-point tidal tensor of phi
-// (get_element, beaming.c:31-117) weighted by rm D (1+z) dr and rm^2 D (1+z)
-// dr, cumulative over the source planes sorted by distance; ISW: phi weighted
-// by 2 PD(rm) dr.  Accumulation in FP64.
+// neighbouring rays and their reads share cache lines), or several for small
+// maps.  The march uses nr = N/2 radial steps of dr = r_max/nr
+// (get_radial_params, common.c:333-337); at each step the NGP cell of
+// (rm u + x_obs)/dx is read (interpolate_from_grid, beaming.c:120-268,
+// periodic in x, y and z on one GPU).  kappa: transverse trace of the 19-point
+// tidal tensor of phi (get_element, beaming.c:31-117) weighted by rm D (1+z)
+// dr and rm^2 D (1+z) dr, cumulative over the source planes sorted by
+// distance; ISW: phi weighted by 2 PD(rm) dr.  Accumulation in FP64.
+// 1024^3, nside 512, three planes: kappa 8.87 ms (11.15 with FP64 cell
+// indices, three loads per record and a block per row for the records), of
+// which the records 4.4 (13.3 GB written) and the march 4.5 (bound by the
+// records' fetch); ISW 2.11 ms (3.51), bound by its vector instructions.
 #include "clr_internal.h"
 #include <algorithm>
 #include <math.h>
@@ -23,10 +27,11 @@ constexpr int kMaxPlanes = 100;   // NPLANES_MAX, common.h:133
 
 struct LosArgs {
   const float *phi;
+  const float2 *t6;       // k_records' tidal records, or null
   int N, ngx;
   double idx, dr, ox, oy, oz;
-  int nr, nplanes, which;
-  int irmin[kMaxPlanes], irmax[kMaxPlanes];
+  int nr, nplanes, lg;    // 2^lg lanes per pixel
+  int irmax[kMaxPlanes];
   double inv_rmax[kMaxPlanes];
 };
 
@@ -36,25 +41,94 @@ __device__ inline int wrapi(long v, int N) {
   return (int)v;
 }
 
+// The NGP cells of a march: step i reads cell (long)((rm u + x_obs) idx + 1/2)
+// per axis, rm = (i + 1/2) dr, wrapped once.  The position is kept in 32.32
+// fixed point, base + i step, whose integer half is the cell; it is off by at
+// most (i + 1) 2^-33 + 2^-40 of a cell, so where the fraction comes within
+// 2^-20 of a cell edge (or the position is negative, where the reference
+// truncates towards zero) the FP64 expression decides: the same cells as it,
+// for 2 + 2 integer operations per axis instead of 5 FP64 ones and 4 to wrap.
+// Needs |x| < 2^30 cells and at most 2^12 steps.
+struct Ray {
+  double u[3];
+  int64_t base[3], step[3];
+};
+__device__ inline void ray_setup(Ray &r, double dr, double idx, double ox, double oy, double oz) {
+  const double o[3] = {ox, oy, oz};
+#pragma unroll
+  for (int ax = 0; ax < 3; ax++) {
+    const double st = r.u[ax] * dr * idx;
+    r.step[ax] = llrint(st * 4294967296.0);
+    r.base[ax] = llrint((0.5 * st + o[ax] * idx + 0.5) * 4294967296.0);
+  }
+}
+// The cell of step i, x = base + i step.
+__device__ inline void ray_cell(const Ray &r, const int64_t x[3], int i, int N, double dr, double idx, double ox,
+                                double oy, double oz, int c[3]) {
+#pragma clang fp contract(off)
+  constexpr uint32_t G = 1u << 12;   // 2^-20
+  bool close = false;
+#pragma unroll
+  for (int ax = 0; ax < 3; ax++) {
+    c[ax] = (int)(x[ax] >> 32);
+    close = close || (uint32_t)x[ax] + G < 2 * G || c[ax] < 0;
+    c[ax] = c[ax] >= N ? c[ax] - N : c[ax];
+  }
+  if (close) {
+    const double rm = (i + 0.5) * dr;
+    c[0] = wrapi((long)((rm * r.u[0] + ox) * idx + 0.5), N);
+    c[1] = wrapi((long)((rm * r.u[1] + oy) * idx + 0.5), N);
+    c[2] = wrapi((long)((rm * r.u[2] + oz) * idx + 0.5), N);
+  }
+}
+
+// Second differences of phi at a cell (get_element, beaming.c:79-116), in FP32
+// as the reference evaluates them on flouble values: xx, xy, xz, yy, yz, zz.
+__device__ inline void tidal_at(const float *__restrict__ phi, int N, size_t ngx, size_t plane, const int c[3],
+                                float t[6]) {
+#pragma clang fp contract(off)
+  const int xh = c[0] == N - 1 ? 0 : c[0] + 1, xl = c[0] == 0 ? N - 1 : c[0] - 1;
+  const int yh = c[1] == N - 1 ? 0 : c[1] + 1, yl = c[1] == 0 ? N - 1 : c[1] - 1;
+  const int zh = c[2] == N - 1 ? 0 : c[2] + 1, zl = c[2] == 0 ? N - 1 : c[2] - 1;
+  const size_t Z0 = (size_t)c[2] * plane, ZH = (size_t)zh * plane, ZL = (size_t)zl * plane;
+  const size_t Y0 = (size_t)c[1] * ngx, YH = (size_t)yh * ngx, YL = (size_t)yl * ngx;
+  const int X0 = c[0];
+  const float c0 = phi[X0 + Y0 + Z0];
+  t[0] = phi[xh + Y0 + Z0] + phi[xl + Y0 + Z0] - 2 * c0;
+  t[3] = phi[X0 + YH + Z0] + phi[X0 + YL + Z0] - 2 * c0;
+  t[1] = 0.25f * (phi[xh + YH + Z0] + phi[xl + YL + Z0] - phi[xh + YL + Z0] - phi[xl + YH + Z0]);
+  t[5] = phi[X0 + Y0 + ZH] + phi[X0 + Y0 + ZL] - 2 * c0;
+  t[2] = 0.25f * (phi[xh + Y0 + ZH] + phi[xl + Y0 + ZL] - phi[xh + Y0 + ZL] - phi[xl + Y0 + ZH]);
+  t[4] = 0.25f * (phi[X0 + YH + ZH] + phi[X0 + YL + ZL] - phi[X0 + YH + ZL] - phi[X0 + YL + ZH]);
+}
+
+// kappa (KAPPA) or ISW march: 2^lg consecutive lanes per pixel, each taking
+// every 2^lg-th step (ONE: a lane per pixel, so that the step and its weights
+// are the wavefront's), summed per source plane.  REC: the tidal records of
+// k_records, one 24-byte read per step, instead of 19 stencil reads.
+template <bool KAPPA, bool REC, bool ONE>
 __global__ __launch_bounds__(256) void k_los(LosArgs a, const double *__restrict__ fac1,
                                              const double *__restrict__ fac2, int64_t nside, int64_t npix,
                                              float *__restrict__ out) {
-#pragma clang fp contract(off)
-  const int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lg = ONE ? 0 : a.lg, sub = ONE ? 0 : (int)(t & ((1 << lg) - 1)), K = 1 << lg;
+  const int64_t ip = t >> lg;
   if (ip >= npix) return;
-  double u[3];
-  pix2vec_nest(nside, ip, u);
+  Ray ray;
+  pix2vec_nest(nside, ip, ray.u);
+  ray_setup(ray, a.dr, a.idx, a.ox, a.oy, a.oz);
   const int N = a.N;
   const size_t ngx = (size_t)a.ngx, plane = (size_t)N * ngx;
   const float *__restrict__ phi = a.phi;
   double rot[6];
-  if (a.which == 0) {
-    double cth = u[2];
+  if (KAPPA) {
+#pragma clang fp contract(off)
+    double cth = ray.u[2];
     if (cth >= 1) cth = 1;
     if (cth <= -1) cth = -1;
     const double sth = sqrt((1 - cth) * (1 + cth));
     double cph = 1, sph = 0;
-    if (sth != 0) { cph = u[0] / sth; sph = u[1] / sth; }
+    if (sth != 0) { cph = ray.u[0] / sth; sph = ray.u[1] / sth; }
     const double pre = a.idx * a.idx;
     rot[0] = (cth * cth * cph * cph + sph * sph) * pre;
     rot[1] = (2 * cph * sph * (cth * cth - 1)) * pre;
@@ -64,141 +138,201 @@ __global__ __launch_bounds__(256) void k_los(LosArgs a, const double *__restrict
     rot[5] = (sth * sth) * pre;
   }
   double k1 = 0, k2 = 0;
-  const double obs[3] = {a.ox, a.oy, a.oz};
+  constexpr int U = KAPPA && !REC ? 1 : 4;   // steps in flight
+  int i = sub;
   for (int pl = 0; pl < a.nplanes; pl++) {
-    for (int irr = a.irmin[pl]; irr <= a.irmax[pl]; irr++) {
-      const double rm = (irr + 0.5) * a.dr;
-      int ix[3];
-      for (int ax = 0; ax < 3; ax++) {
-        const double xn = (rm * u[ax] + obs[ax]) * a.idx;
-        ix[ax] = wrapi((long)(xn + 0.5), N);
-      }
-      const size_t o = (size_t)ix[2] * plane + (size_t)ix[1] * ngx + ix[0];
-      if (a.which == 1) {
-        k1 += (double)phi[o] * fac1[irr];
-        continue;
-      }
-      const int xh = ix[0] == N - 1 ? 0 : ix[0] + 1, xl = ix[0] == 0 ? N - 1 : ix[0] - 1;
-      const int yh = ix[1] == N - 1 ? 0 : ix[1] + 1, yl = ix[1] == 0 ? N - 1 : ix[1] - 1;
-      const int zh = ix[2] == N - 1 ? 0 : ix[2] + 1, zl = ix[2] == 0 ? N - 1 : ix[2] - 1;
-      const size_t Z0 = (size_t)ix[2] * plane, ZH = (size_t)zh * plane, ZL = (size_t)zl * plane;
-      const size_t Y0 = (size_t)ix[1] * ngx, YH = (size_t)yh * ngx, YL = (size_t)yl * ngx;
-      // the second differences in FP32, as get_element evaluates them on
-      // flouble values (beaming.c:79-116)
-      const float c0 = phi[ix[0] + Y0 + Z0];
-      float t[6];
-      t[0] = phi[xh + Y0 + Z0] + phi[xl + Y0 + Z0] - 2 * c0;
-      t[3] = phi[ix[0] + YH + Z0] + phi[ix[0] + YL + Z0] - 2 * c0;
-      t[1] = 0.25f * (phi[xh + YH + Z0] + phi[xl + YL + Z0] - phi[xh + YL + Z0] - phi[xl + YH + Z0]);
-      t[5] = phi[ix[0] + Y0 + ZH] + phi[ix[0] + Y0 + ZL] - 2 * c0;
-      t[2] = 0.25f * (phi[xh + Y0 + ZH] + phi[xl + Y0 + ZL] - phi[xh + Y0 + ZL] - phi[xl + Y0 + ZH]);
-      t[4] = 0.25f * (phi[ix[0] + YH + ZH] + phi[ix[0] + YL + ZL] - phi[ix[0] + YH + ZL] - phi[ix[0] + YL + ZH]);
-      double dotp = 0;
-      for (int q = 0; q < 6; q++) dotp += rot[q] * (double)t[q];
-      k1 += dotp * fac1[irr];
-      k2 += dotp * fac2[irr];
+    const int last = a.irmax[pl];
+    int64_t x[3], kstep[3];
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) {
+      x[ax] = ray.base[ax] + (int64_t)i * ray.step[ax];
+      kstep[ax] = ray.step[ax] << lg;
     }
-    const double v = a.which == 0 ? (k1 - a.inv_rmax[pl] * k2) : k1;
-    out[(size_t)pl * npix + ip] = (float)v;
+    for (; i <= last; i += U * K) {
+      float tt[U][6];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        // (steps past the plane's last are read, not added)
+        int c[3];
+        ray_cell(ray, x, i + u * K, N, a.dr, a.idx, a.ox, a.oy, a.oz, c);
+#pragma unroll
+        for (int ax = 0; ax < 3; ax++) x[ax] += kstep[ax];
+        if (!KAPPA) {
+          tt[u][0] = phi[(size_t)c[2] * plane + (size_t)c[1] * ngx + c[0]];
+        } else if (REC) {
+          const float *r = (const float *)(a.t6 + (((size_t)c[2] * N + c[1]) * N + c[0]) * 3);
+          __builtin_memcpy(tt[u], r, 16);
+          __builtin_memcpy(tt[u] + 4, r + 4, 8);
+        } else {
+          tidal_at(phi, N, ngx, plane, c, tt[u]);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int j = i + u * K;
+        if (j > last) break;
+        if (!KAPPA) {
+          k1 = fma((double)tt[u][0], fac1[j], k1);
+        } else {
+          double dot = rot[0] * (double)tt[u][0];
+#pragma unroll
+          for (int q = 1; q < 6; q++) dot = fma(rot[q], (double)tt[u][q], dot);
+          k1 = fma(dot, fac1[j], k1);
+          k2 = fma(dot, fac2[j], k2);
+        }
+      }
+    }
+    // the next plane's first step of this lane
+    if (i > last) i -= (i - last - 1) / K * K;
+    double v = KAPPA ? k1 - a.inv_rmax[pl] * k2 : k1;
+    for (int o = 1; o < K; o <<= 1) v += __shfl_xor(v, o);
+    if (sub == 0) out[(size_t)pl * npix + ip] = (float)v;
   }
 }
 
-// The transverse-Hessian inputs of get_element (beaming.c:79-116) for every
-// cell a march can reach (centre within sqrt(r2lim) of the observer) once:
-// t6[cell][6] = (xx, xy, xz, yy, yz, zz) second differences of phi in FP32,
-// the same expressions k_los evaluates per sample, so a march over t6 reads
-// one 24-byte record per step instead of 19 stencil values.
-__global__ __launch_bounds__(256) void k_tidal(const float *__restrict__ phi, int N, int ngx, float dxf, float ox,
-                                               float oy, float oz, float r2lim, float2 *__restrict__ t6) {
+// Per-cell records for the marches, for the cells within sqrt(r2lim) of the
+// observer (no march reaches the others: the box corners are 42 % of the
+// cube).  TID: the tidal records t6[cell][6], tidal_at's second differences;
+// VEL: vrec[cell] = phi's unscaled central differences in FP32 (get_element,
+// RETURN_VEL) and the density.  A block takes 64 x 4 cells and walks nzb
+// planes of z: three planes of phi with their halo in LDS (the next one's
+// loads in flight), so phi is read once (1.5 times with the halos; a block per
+// row read it 7 times from L2), and the 24-byte records go through LDS so that
+// consecutive lanes store consecutive float2.  Bound by the records' writes.
+constexpr int kRecX = 64, kRecY = 4;
+template <bool TID, bool VEL>
+__global__ __launch_bounds__(256) void k_records(const float *__restrict__ phi, const float *__restrict__ dens, int N,
+                                                 int ngx, int nzb, float dxf, float ox, float oy, float oz, float r2lim,
+                                                 float2 *__restrict__ t6, float4 *__restrict__ vrec) {
 #pragma clang fp contract(off)
-  const size_t row = blockIdx.x;
-  const int iz = (int)(row / N), iy = (int)(row % N);
-  const float yc = iy * dxf - oy, zc = iz * dxf - oz;
-  const float rho2 = yc * yc + zc * zc;
-  if (rho2 > r2lim) return;   // no march reaches this row
+  constexpr int LX = kRecX + 2, LY = kRecY + 2, LP = LX * LY;
+  __shared__ float pl[3][LP];
+  __shared__ float2 st[TID ? 256 * 3 : 1];
+  __shared__ unsigned char ok[TID ? 256 : 1];
+  const int x0 = blockIdx.x * kRecX, y0 = blockIdx.y * kRecY, zb = blockIdx.z * nzb;
+  const int ze = min(zb + nzb, N);
+  // the block's planes: those whose nearest cell is in reach (an interval)
+  const float xa = x0 * dxf - ox, xb = (min(x0 + kRecX, N) - 1) * dxf - ox;
+  const float ya = y0 * dxf - oy, yb = (y0 + kRecY - 1) * dxf - oy;
+  // distances along an axis are periodic: a march or a CIC corner may wrap
+  const float box = N * dxf;
+  auto dist = [box](float x) { const float d = fabsf(x); return fminf(d, box - d); };
+  auto nearest = [box](float lo, float hi) {
+    return fmaxf(fminf(fmaxf(lo, -hi), box - fmaxf(-lo, hi)), 0.f);
+  };
+  const float xn = nearest(xa, xb), yn = nearest(ya, yb), rn = xn * xn + yn * yn;
+  int z0 = zb, z1 = ze;
+  auto far = [&](int z) { const float zc = dist(z * dxf - oz); return zc * zc + rn > r2lim; };
+  while (z0 < z1 && far(z0)) z0++;
+  while (z1 > z0 && far(z1 - 1)) z1--;
+  if (z0 >= z1) return;
   const size_t plane = (size_t)N * ngx;
-  const int yh = iy == N - 1 ? 0 : iy + 1, yl = iy == 0 ? N - 1 : iy - 1;
-  const int zh = iz == N - 1 ? 0 : iz + 1, zl = iz == 0 ? N - 1 : iz - 1;
-  const size_t Z0 = (size_t)iz * plane, ZH = (size_t)zh * plane, ZL = (size_t)zl * plane;
-  const size_t Y0 = (size_t)iy * ngx, YH = (size_t)yh * ngx, YL = (size_t)yl * ngx;
-  // 256 cells at a time: the records go through LDS so that consecutive
-  // lanes store consecutive float2 of the row (a lane's own 24-byte record
-  // would spread each store over 1.5 KB)
-  __shared__ float2 st[256 * 3];
-  __shared__ unsigned char ok[256];
-  for (int x0 = 0; x0 < N; x0 += 256) {
-    const int ix = x0 + threadIdx.x;
-    const float xc = ix * dxf - ox;
-    const bool in = ix < N && !(xc * xc + rho2 > r2lim);
-    ok[threadIdx.x] = in;
+  // the thread's (up to two) places of a plane's LDS image and their rows
+  size_t src[2];
+  int dst[2];
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const int e = (int)threadIdx.x + 256 * k, cx = e % LX, cy = e / LX;
+    int gx = x0 - 1 + cx, gy = y0 - 1 + cy;
+    gx = gx < 0 ? gx + N : (gx >= N ? gx - N : gx);
+    if (gx >= N) gx = 0;   // columns past a grid narrower than the tile: not used
+    gy = gy < 0 ? gy + N : (gy >= N ? gy - N : gy);
+    dst[k] = e < LP ? e : -1;
+    src[k] = e < LP ? (size_t)gy * ngx + gx : 0;
+  }
+  auto fetch = [&](int z, float v[2]) {
+    const int zw = z < 0 ? z + N : (z >= N ? z - N : z);
+#pragma unroll
+    for (int k = 0; k < 2; k++) v[k] = dst[k] >= 0 ? phi[(size_t)zw * plane + src[k]] : 0.f;
+  };
+  auto put = [&](int s, const float v[2]) {
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+      if (dst[k] >= 0) pl[s][dst[k]] = v[k];
+  };
+  float v[2];
+  fetch(z0 - 1, v);
+  put(0, v);
+  fetch(z0, v);
+  put(1, v);
+  fetch(z0 + 1, v);
+  const int lx = threadIdx.x % kRecX, ly = threadIdx.x / kRecX;
+  const int ix = x0 + lx, iy = y0 + ly, o = (ly + 1) * LX + lx + 1;
+  const float xc = dist(ix * dxf - ox), yc = dist(iy * dxf - oy), rho2 = xc * xc + yc * yc;
+  for (int z = z0, s = 0; z < z1; z++, s = s == 2 ? 0 : s + 1) {
+    // slots s, s+1, s+2 (mod 3) hold planes z-1, z, z+1
+    const int s1 = s == 2 ? 0 : s + 1, s2 = s1 == 2 ? 0 : s1 + 1;
+    put(s2, v);
+    if (z + 1 < z1) fetch(z + 2, v);
+    __syncthreads();
+    const float zc = dist(z * dxf - oz);
+    const bool in = ix < N && !(zc * zc + rho2 > r2lim);
+    const size_t cell = ((size_t)z * N + iy) * N + ix;
+    const float *L = pl[s] + o, *M = pl[s1] + o, *H = pl[s2] + o;
     if (in) {
-      const int xh = ix == N - 1 ? 0 : ix + 1, xl = ix == 0 ? N - 1 : ix - 1;
-      const float c0 = phi[ix + Y0 + Z0];
-      float t[6];
-      t[0] = phi[xh + Y0 + Z0] + phi[xl + Y0 + Z0] - 2 * c0;
-      t[3] = phi[ix + YH + Z0] + phi[ix + YL + Z0] - 2 * c0;
-      t[1] = 0.25f * (phi[xh + YH + Z0] + phi[xl + YL + Z0] - phi[xh + YL + Z0] - phi[xl + YH + Z0]);
-      t[5] = phi[ix + Y0 + ZH] + phi[ix + Y0 + ZL] - 2 * c0;
-      t[2] = 0.25f * (phi[xh + Y0 + ZH] + phi[xl + Y0 + ZL] - phi[xh + Y0 + ZL] - phi[xl + Y0 + ZH]);
-      t[4] = 0.25f * (phi[ix + YH + ZH] + phi[ix + YL + ZL] - phi[ix + YH + ZL] - phi[ix + YL + ZH]);
-      st[3 * threadIdx.x] = make_float2(t[0], t[1]);
-      st[3 * threadIdx.x + 1] = make_float2(t[2], t[3]);
-      st[3 * threadIdx.x + 2] = make_float2(t[4], t[5]);
+      const float c0 = M[0], xl = M[-1], xh = M[1], yl = M[-LX], yh = M[LX], zl = L[0], zh = H[0];
+      if (VEL) vrec[cell] = make_float4(xh - xl, yh - yl, zh - zl, dens[((size_t)z * N + iy) * ngx + ix]);
+      if (TID) {
+        const float txx = xh + xl - 2 * c0, tyy = yh + yl - 2 * c0, tzz = zh + zl - 2 * c0;
+        const float txy = 0.25f * (M[1 + LX] + M[-1 - LX] - M[1 - LX] - M[-1 + LX]);
+        const float txz = 0.25f * (H[1] + L[-1] - L[1] - H[-1]);
+        const float tyz = 0.25f * (H[LX] + L[-LX] - L[LX] - H[-LX]);
+        st[3 * threadIdx.x] = make_float2(txx, txy);
+        st[3 * threadIdx.x + 1] = make_float2(txz, tyy);
+        st[3 * threadIdx.x + 2] = make_float2(tyz, tzz);
+      }
     }
+    if (TID) ok[threadIdx.x] = in;
     __syncthreads();
-    float2 *o = t6 + (row * N + x0) * 3;
-    const int nk = 3 * min(256, N - x0);
-    for (int k = threadIdx.x; k < nk; k += 256)
-      if (ok[k / 3]) o[k] = st[k];
-    __syncthreads();
+    if (TID) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const int e = (int)threadIdx.x + 256 * k, row = e / (3 * kRecX), w = e % (3 * kRecX);
+        if (ok[row * kRecX + w / 3])   // (streamed past the L2: 9.31 -> 8.87 ms for kappa at 1024^3)
+          __builtin_nontemporal_store(*(const double *)&st[e],
+                                      (double *)&t6[(((size_t)z * N + y0 + row) * N + x0) * 3 + w]);
+      }
+    }
   }
 }
 
-// The kappa march of k_los over the precomputed t6 records.
-__global__ __launch_bounds__(256) void k_los_t6(LosArgs a, const float2 *__restrict__ t6,
-                                                const double *__restrict__ fac1, const double *__restrict__ fac2,
-                                                int64_t nside, int64_t npix, float *__restrict__ out) {
-#pragma clang fp contract(off)
-  const int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (ip >= npix) return;
-  double u[3];
-  pix2vec_nest(nside, ip, u);
-  const int N = a.N;
-  double rot[6];
-  {
-    double cth = u[2];
-    if (cth >= 1) cth = 1;
-    if (cth <= -1) cth = -1;
-    const double sth = sqrt((1 - cth) * (1 + cth));
-    double cph = 1, sph = 0;
-    if (sth != 0) { cph = u[0] / sth; sph = u[1] / sth; }
-    const double pre = a.idx * a.idx;
-    rot[0] = (cth * cth * cph * cph + sph * sph) * pre;
-    rot[1] = (2 * cph * sph * (cth * cth - 1)) * pre;
-    rot[2] = (-2 * cth * sth * cph) * pre;
-    rot[3] = (cth * cth * sph * sph + cph * cph) * pre;
-    rot[4] = (-2 * cth * sth * sph) * pre;
-    rot[5] = (sth * sth) * pre;
-  }
-  double k1 = 0, k2 = 0;
-  const double obs[3] = {a.ox, a.oy, a.oz};
-  for (int pl = 0; pl < a.nplanes; pl++) {
-    for (int irr = a.irmin[pl]; irr <= a.irmax[pl]; irr++) {
-      const double rm = (irr + 0.5) * a.dr;
-      int ix[3];
-      for (int ax = 0; ax < 3; ax++) {
-        const double xn = (rm * u[ax] + obs[ax]) * a.idx;
-        ix[ax] = wrapi((long)(xn + 0.5), N);
-      }
-      const float2 *r = t6 + (((size_t)ix[2] * N + ix[1]) * N + ix[0]) * 3;
-      const float2 p0 = r[0], p1 = r[1], p2 = r[2];
-      const float t[6] = {p0.x, p0.y, p1.x, p1.y, p2.x, p2.y};
-      double dotp = 0;
-      for (int q = 0; q < 6; q++) dotp += rot[q] * (double)t[q];
-      k1 += dotp * fac1[irr];
-      k2 += dotp * fac2[irr];
-    }
-    out[(size_t)pl * npix + ip] = (float)(k1 - a.inv_rmax[pl] * k2);
+void launch_records(clr_ctx *c, bool tidal, bool vel, float rlim) {
+  const int N = c->N;
+  // 32 planes per block, fewer while that leaves less than 8 blocks per CU
+  const int cols = (N + kRecX - 1) / kRecX * (N / kRecY);
+  int nzb = 32;
+  while (nzb > 4 && cols * ((N + nzb - 1) / nzb) < 2048) nzb /= 2;
+  const dim3 g((N + kRecX - 1) / kRecX, N / kRecY, (N + nzb - 1) / nzb);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, g, dim3(256), 0, c->stream, c->npot, c->dens, N, c->ngx, nzb, (float)c->dx, (float)c->obs[0],
+                       (float)c->obs[1], (float)c->obs[2], rlim * rlim, (float2 *)c->tidal, (float4 *)c->velrec);
+  };
+  if (tidal && vel) go(k_records<true, true>);
+  else if (tidal) go(k_records<true, false>);
+  else go(k_records<false, true>);
+}
+
+// Lanes per pixel of a march over nstep steps: as many as bring npix pixels to
+// a quarter of a million threads (4 wavefronts on every SIMD), with 8 steps or
+// more each, at most 16.  nside 32 on 512^3: ISW 194 -> 46 us, a custom map 287 -> 49; nside
+// 64 on 192^3: ISW 57 -> 24, custom map 85 -> 42.
+int lanes_lg(int64_t npix, int nstep) {
+  int lg = 0;
+  while (lg < 4 && (npix << lg) < (1 << 18) && (nstep >> lg) >= 16) lg++;
+  return lg;
+}
+
+template <bool KAPPA>
+void launch_los(const LosArgs &a, const double *df, int nside, float *dout, hipStream_t s) {
+  const int64_t npix = 12LL * nside * nside;
+  const dim3 g((unsigned)(((npix << a.lg) + 255) / 256)), b(256);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, b, 0, s, a, df, df + a.nr, (int64_t)nside, npix, dout); };
+  if (KAPPA && a.t6) {
+    if (a.lg == 0) go(k_los<KAPPA, true, true>);
+    else go(k_los<KAPPA, true, false>);
+  } else {
+    if (a.lg == 0) go(k_los<KAPPA, false, true>);
+    else go(k_los<KAPPA, false, false>);
   }
 }
 
@@ -235,14 +369,13 @@ static int los_setup(clr_ctx *c, int which, int nside, int nplanes, const double
   a.oz = c->obs[2];
   a.nr = nr;
   a.nplanes = nplanes;
-  a.which = which;
   for (int i = 0; i < nplanes; i++) {
     const int ih = (int)(rs[order[i]] * idr + 0.5);
     a.inv_rmax[i] = 1. / (ih * dr);
     a.irmax[i] = std::min(ih, nr - 1);
   }
-  a.irmin[0] = 0;
-  for (int i = 1; i < nplanes; i++) a.irmin[i] = a.irmax[i - 1] + 1;
+  // (plane i adds the steps after plane i-1's last)
+  a.lg = lanes_lg(12LL * nside * nside, a.irmax[nplanes - 1] + 1);
   const double *rr = c->h_r.data(), *zz = c->h_z.data(), *dd = c->h_d1.data(), *pd = c->h_pd.data();
   f12.assign(2 * (size_t)nr, 0.0);
   for (int i = 0; i < nr; i++) {
@@ -280,11 +413,16 @@ int clr_launch_los(clr_ctx *c, int which, int nside, int nplanes, const double *
   double *df = (double *)c->misc;
   float *dout = (float *)(df + 2 * nr);
   CLR_HIP(c, hipMemcpyAsync(df, f12.data(), 2 * nr * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  // kappa over a precomputed tidal grid (24 bytes per cell) when it fits in
-  // a quarter of the free device memory; the direct 19-point march otherwise
+  // kappa over precomputed tidal records (24 bytes per cell) when they fit in
+  // a quarter of the free device memory and the march reads enough of them: a
+  // record costs 8 ps per cell in reach, a step 3 ps with and 18 ps without them
+  // (1024^3, nside 512), so the direct march is the faster one below about 0.4
+  // steps per cell (0.96 -> 0.14 ms at 512^3, nside 32)
+  const double steps = (double)npix * (a.irmax[nplanes - 1] + 1);
+  const double reach = std::min(1.0, 4.18879 * pow(c->r_max / c->L, 3)) * pow((double)c->N, 3);
   const size_t t6_bytes = (size_t)c->N * c->N * c->N * 6 * sizeof(float);
   bool use_t6 = false;
-  if (which == 0) {
+  if (which == 0 && steps >= 0.4 * reach) {
     size_t fr = 0, tot = 0;
     if (c->tidal_n >= t6_bytes) use_t6 = true;
     else if (hipMemGetInfo(&fr, &tot) == hipSuccess && t6_bytes <= fr / 4) use_t6 = true;
@@ -296,15 +434,11 @@ int clr_launch_los(clr_ctx *c, int which, int nside, int nplanes, const double *
   }
   CLR_HIP(c, hipEventRecord(c->ev0, c->stream));
   if (use_t6) {
-    hipLaunchKernelGGL(k_tidal, dim3((unsigned)((size_t)c->N * c->N)), dim3(256), 0, c->stream, c->npot, c->N,
-                       c->ngx, (float)c->dx, (float)c->obs[0], (float)c->obs[1], (float)c->obs[2],
-                       (float)((c->r_max + 2 * c->dx) * (c->r_max + 2 * c->dx)), (float2 *)c->tidal);
-    hipLaunchKernelGGL(k_los_t6, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, c->stream, a,
-                       (const float2 *)c->tidal, df, df + nr, (int64_t)nside, npix, dout);
-  } else {
-    hipLaunchKernelGGL(k_los, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, c->stream, a, df, df + nr,
-                       (int64_t)nside, npix, dout);
+    launch_records(c, true, false, (float)(c->r_max + 2 * c->dx));
+    a.t6 = (const float2 *)c->tidal;
   }
+  if (which == 0) launch_los<true>(a, df, nside, dout, c->stream);
+  else launch_los<false>(a, df, nside, dout, c->stream);
   CLR_HIP(c, hipGetLastError());
   CLR_HIP(c, hipEventRecord(c->ev1, c->stream));
   CLR_HIP(c, hipMemcpyAsync(out, dout, (size_t)npix * nplanes * sizeof(float), hipMemcpyDeviceToHost, c->stream));
@@ -343,10 +477,9 @@ int clr_enqueue_kappa(clr_ctx *c, hipStream_t s) {
   LosArgs a;
   memcpy(&a, c->los_plan.data(), sizeof(LosArgs));
   a.phi = c->npot;
-  const int64_t npix = 12LL * c->los_nside * c->los_nside;
+  a.t6 = nullptr;
   double *df = (double *)c->los_buf;
-  hipLaunchKernelGGL(k_los, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, s, a, df, df + a.nr,
-                     (int64_t)c->los_nside, npix, (float *)(df + 2 * a.nr));
+  launch_los<true>(a, df, c->los_nside, (float *)(df + 2 * a.nr), s);
   CLR_HIP(c, hipGetLastError());
   return CLR_OK;
 }
@@ -380,8 +513,8 @@ struct BeamArgs {
   const double *r_arr, *z_arr, *v1_arr;   // background r-tables
   const double *a2r;                      // r(a) at a = i/(na-1) (r_of_z, cosmo.c:101-112)
   const double *fac;                      // fac_r_0, fac_r_1, fac_r_2 (nr each)
-  const float4 *vrec;                     // per cell (k_cell_records): phi's central differences, delta
-  const float2 *t6;                       // per cell (k_tidal): the tidal tensor's second differences
+  const float4 *vrec;                     // per cell (k_records): phi's central differences, delta
+  const float2 *t6;                       // per cell (k_records): the tidal tensor's second differences
 };
 
 // The reference wraps once (beaming.c:129-133), which covers every cell the
@@ -432,22 +565,6 @@ __device__ inline void vel_tid_at(const float *__restrict__ phi, int N, size_t n
   t[1] = 0.25f * (phi[xh + YH + Z0] + phi[xl + YL + Z0] - phi[xh + YL + Z0] - phi[xl + YH + Z0]);
   t[2] = 0.25f * (phi[xh + Y0 + ZH] + phi[xl + Y0 + ZL] - phi[xh + Y0 + ZL] - phi[xl + Y0 + ZH]);
   t[4] = 0.25f * (phi[ix + YH + ZH] + phi[ix + YL + ZL] - phi[ix + YH + ZL] - phi[ix + YL + ZH]);
-}
-
-// Per cell: phi's unscaled central differences in FP32 (as vel_at takes
-// them) and the density, one 16-byte record, so that the CIC and NGP reads
-// of the source passes take one load per cell instead of six (plus one).
-__global__ __launch_bounds__(256) void k_cell_records(const float *__restrict__ phi, const float *__restrict__ dens,
-                                                      int N, int ngx, float4 *__restrict__ out) {
-#pragma clang fp contract(off)
-  const size_t row = blockIdx.x;
-  const int iz = (int)(row / N), iy = (int)(row % N);
-  const size_t plane = (size_t)N * ngx;
-  for (int ix = threadIdx.x; ix < N; ix += blockDim.x) {
-    double v[3];
-    vel_at(phi, N, (size_t)ngx, plane, ix, iy, iz, v);
-    out[row * N + ix] = make_float4((float)v[0], (float)v[1], (float)v[2], dens[row * ngx + ix]);
-  }
 }
 
 // A cell's velocity differences (and density) from its record or from phi.
@@ -593,7 +710,7 @@ __global__ __launch_bounds__(256) void k_src_beams(BeamArgs a, const float4 *__r
 
 // Builds the per-cell records on the context's stream: velocity differences
 // and density (16 bytes per cell), with `tidal` also the tidal tensor (24
-// bytes per cell, k_tidal), when they fit in a quarter of the free device
+// bytes per cell), when they fit in a quarter of the free device
 // memory (buffers kept for later calls); false: the callers read phi directly.
 bool clr_cell_records(clr_ctx *c, bool tidal) {
   const size_t cells = (size_t)c->N * c->N * c->N;
@@ -609,12 +726,9 @@ bool clr_cell_records(clr_ctx *c, bool tidal) {
   }
   if (clr_ensure(c, &c->velrec, &c->velrec_n, vb)) return false;
   if (tidal && clr_ensure(c, &c->tidal, &c->tidal_n, tb)) return false;
-  hipLaunchKernelGGL(k_cell_records, dim3((unsigned)((size_t)c->N * c->N)), dim3(256), 0, c->stream, c->npot, c->dens,
-                     c->N, c->ngx, (float4 *)c->velrec);
-  if (tidal)
-    hipLaunchKernelGGL(k_tidal, dim3((unsigned)((size_t)c->N * c->N)), dim3(256), 0, c->stream, c->npot, c->N,
-                       c->ngx, (float)c->dx, (float)c->obs[0], (float)c->obs[1], (float)c->obs[2],
-                       (float)((c->r_max + 2 * c->dx) * (c->r_max + 2 * c->dx)), (float2 *)c->tidal);
+  // the marches stay within r_max, the sources within L/2 + 20 (their cells'
+  // corners and the CIC neighbours within 2 cells of that)
+  launch_records(c, tidal, true, (float)(std::max(c->r_max, 0.5 * c->L + 20.) + 3 * c->dx));
   return hipGetLastError() == hipSuccess;
 }
 
@@ -723,7 +837,7 @@ namespace {
 
 struct SkwArgs {
   const float *phi, *dens;
-  const float4 *vrec;   // per cell (k_cell_records), or null
+  const float4 *vrec;   // per cell (k_records), or null
   int N, ngx, nr, na, gaussian;
   double idx, dr, idr, ox, oy, oz, factor_vel, sigma2;
   double glob_idr, r_last, v1_0, v1_last, d1_last;
@@ -909,45 +1023,69 @@ namespace {
 
 struct CstmArgs {
   const float *dens;
-  int N, ngx, ir_min, ir_max, model;
+  int N, ngx, ir_min, ir_max, model, lg;   // 2^lg lanes per pixel
   double idx, dr, ox, oy, oz;
 };
 
+// (1 + d)^b for d > -1 (the model-0 branch of bias_model_f64) as exp(b log1p):
+// a few 1e-16 relative, and half of pow's instructions; the map is FP32.
+__device__ inline double bias_model_march(double d, double b, int model) {
+  if (model == 0) return d <= -1 ? 0.0 : exp(b * log1p(d));
+  return bias_model_f64(d, b, model);
+}
+
+// 2^lg consecutive lanes per pixel (lanes_lg), each taking every 2^lg-th step
+// (ONE: a lane per pixel); the trilinear density as seven lerps.
+template <bool ONE>
 __global__ __launch_bounds__(256) void k_cstm(CstmArgs a, const double *__restrict__ kz,
                                               const double *__restrict__ bz, const double *__restrict__ nz,
                                               int64_t nside, int64_t npix, float *__restrict__ out) {
-#pragma clang fp contract(off)
-  const int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lg = ONE ? 0 : a.lg, sub = ONE ? 0 : (int)(t & ((1 << lg) - 1)), K = 1 << lg;
+  const int64_t ip = t >> lg;
   if (ip >= npix) return;
   double u[3];
   pix2vec_nest(nside, ip, u);
   const int N = a.N;
   const size_t ngx = (size_t)a.ngx, plane = (size_t)N * ngx;
   double cval = 0;
-  for (int irr = a.ir_min; irr <= a.ir_max; irr++) {
-    const double rm = (irr + 0.5) * a.dr;
-    const double xn[3] = {(rm * u[0] + a.ox) * a.idx, (rm * u[1] + a.oy) * a.idx, (rm * u[2] + a.oz) * a.idx};
-    int i0[3], i1[3];
-    double h0[3], h1[3];
-    for (int ax = 0; ax < 3; ax++) {
-      const int c = (int)xn[ax];
-      h0[ax] = xn[ax] - c;
-      h1[ax] = 1 - h0[ax];
-      i0[ax] = wrap1(c, N);
-      i1[ax] = wrap1(c + 1, N);
-    }
-    double d = 0;
+  constexpr int U = 2;   // steps in flight
+  for (int irr = a.ir_min + sub; irr <= a.ir_max; irr += U * K) {
+    float f[U][8];
+    double h[U][3];
 #pragma unroll
-    for (int c = 0; c < 8; c++) {
-      const int bx = c & 1, by = (c >> 1) & 1, bzc = c >> 2;
-      const double w = (bzc ? h0[2] : h1[2]) * (by ? h0[1] : h1[1]) * (bx ? h0[0] : h1[0]);
-      d += (double)a.dens[(size_t)(bzc ? i1[2] : i0[2]) * plane + (size_t)(by ? i1[1] : i0[1]) * ngx +
-                          (bx ? i1[0] : i0[0])] * w;
+    for (int s = 0; s < U; s++) {
+      const double rm = (min(irr + s * K, a.ir_max) + 0.5) * a.dr;
+      const double o[3] = {a.ox, a.oy, a.oz};
+      int i0[3], i1[3];
+#pragma unroll
+      for (int ax = 0; ax < 3; ax++) {
+        const double xn = (rm * u[ax] + o[ax]) * a.idx;
+        const int c = (int)xn;
+        h[s][ax] = xn - c;
+        i0[ax] = wrap1(c, N);
+        i1[ax] = wrap1(c + 1, N);
+      }
+#pragma unroll
+      for (int c = 0; c < 8; c++)
+        f[s][c] = a.dens[(size_t)(c & 4 ? i1[2] : i0[2]) * plane + (size_t)(c & 2 ? i1[1] : i0[1]) * ngx +
+                         (c & 1 ? i1[0] : i0[0])];
     }
-    // the reference holds d as flouble before bias_model
-    cval += kz[irr] * (bias_model_f64((double)(float)d, bz[irr], a.model) * nz[irr] - 1);
+#pragma unroll
+    for (int s = 0; s < U; s++) {
+      const int j = irr + s * K;
+      if (j > a.ir_max) break;
+      double e[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) e[c] = fma(h[s][0], (double)f[s][2 * c + 1] - (double)f[s][2 * c], (double)f[s][2 * c]);
+      const double e0 = fma(h[s][1], e[1] - e[0], e[0]), e1 = fma(h[s][1], e[3] - e[2], e[2]);
+      const double d = fma(h[s][2], e1 - e0, e0);
+      // the reference holds d as flouble before bias_model
+      cval += kz[j] * (bias_model_march((double)(float)d, bz[j], a.model) * nz[j] - 1);
+    }
   }
-  out[ip] = (float)(cval * a.dr);
+  for (int o = 1; o < K; o <<= 1) cval += __shfl_xor(cval, o);
+  if (sub == 0) out[ip] = (float)(cval * a.dr);
 }
 
 }  // namespace
@@ -1000,14 +1138,20 @@ int clr_launch_cstm(clr_ctx *c, int ipop, int nside, float *out) {
   a.ir_min = ir_min;
   a.ir_max = ir_max;
   a.model = T.model;
+  a.lg = lanes_lg(npix, ir_max - ir_min + 1);
   a.idx = N / c->L;
   a.dr = dr;
   a.ox = c->obs[0];
   a.oy = c->obs[1];
   a.oz = c->obs[2];
   CLR_HIP(c, hipEventRecord(c->ev0, c->stream));
-  hipLaunchKernelGGL(k_cstm, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, c->stream, a, dt, dt + nr,
-                     dt + 2 * nr, (int64_t)nside, npix, dout);
+  const dim3 g((unsigned)(((npix << a.lg) + 255) / 256));
+  if (a.lg == 0)
+    hipLaunchKernelGGL(k_cstm<true>, g, dim3(256), 0, c->stream, a, dt, dt + nr, dt + 2 * nr, (int64_t)nside, npix,
+                       dout);
+  else
+    hipLaunchKernelGGL(k_cstm<false>, g, dim3(256), 0, c->stream, a, dt, dt + nr, dt + 2 * nr, (int64_t)nside, npix,
+                       dout);
   CLR_HIP(c, hipGetLastError());
   CLR_HIP(c, hipEventRecord(c->ev1, c->stream));
   CLR_HIP(c, hipMemcpyAsync(out, dout, (size_t)npix * sizeof(float), hipMemcpyDeviceToHost, c->stream));
