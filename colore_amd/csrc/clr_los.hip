@@ -35,18 +35,23 @@ struct LosArgs {
   double inv_rmax[kMaxPlanes];
 };
 
-__device__ inline int wrapi(long v, int N) {
-  if (v >= N) v -= N;
-  else if (v < 0) v += N;
-  return (int)v;
+// The reference wraps once (beaming.c:129-133), which covers every cell the
+// march and the source reads reach when r_max is below the box size; the
+// full modulo keeps other inputs inside the grid.
+__device__ inline int wrap1(int v, int N) {
+  if (v >= N || v < 0) {
+    v %= N;
+    if (v < 0) v += N;
+  }
+  return v;
 }
 
 // The NGP cells of a march: step i reads cell (long)((rm u + x_obs) idx + 1/2)
-// per axis, rm = (i + 1/2) dr, wrapped once.  The position is kept in 32.32
+// per axis, rm = (i + 1/2) dr, wrapped.  The position is kept in 32.32
 // fixed point, base + i step, whose integer half is the cell; it is off by at
 // most (i + 1) 2^-33 + 2^-40 of a cell, so where the fraction comes within
 // 2^-20 of a cell edge (or the position is negative, where the reference
-// truncates towards zero) the FP64 expression decides: the same cells as it,
+// truncates towards zero, or two boxes away) the FP64 expression decides: the same cells as it,
 // for 2 + 2 integer operations per axis instead of 5 FP64 ones and 4 to wrap.
 // Needs |x| < 2^30 cells and at most 2^12 steps.
 struct Ray {
@@ -70,15 +75,15 @@ __device__ inline void ray_cell(const Ray &r, const int64_t x[3], int i, int N, 
   bool close = false;
 #pragma unroll
   for (int ax = 0; ax < 3; ax++) {
-    c[ax] = (int)(x[ax] >> 32);
-    close = close || (uint32_t)x[ax] + G < 2 * G || c[ax] < 0;
-    c[ax] = c[ax] >= N ? c[ax] - N : c[ax];
+    const uint32_t v = (uint32_t)(x[ax] >> 32);
+    close = close || (uint32_t)x[ax] + G < 2 * G || v >= 2u * N;
+    c[ax] = (int)min(v, v - N);
   }
   if (close) {
     const double rm = (i + 0.5) * dr;
-    c[0] = wrapi((long)((rm * r.u[0] + ox) * idx + 0.5), N);
-    c[1] = wrapi((long)((rm * r.u[1] + oy) * idx + 0.5), N);
-    c[2] = wrapi((long)((rm * r.u[2] + oz) * idx + 0.5), N);
+    c[0] = wrap1((int)((rm * r.u[0] + ox) * idx + 0.5), N);
+    c[1] = wrap1((int)((rm * r.u[1] + oy) * idx + 0.5), N);
+    c[2] = wrap1((int)((rm * r.u[2] + oz) * idx + 0.5), N);
   }
 }
 
@@ -499,15 +504,15 @@ int clr_fetch_kappa(clr_ctx *c, float *out) {
 // Sources' line-of-sight properties: srcs_beams_preproc_single
 // (srcs.c:425-445), srcs_get_beam_properties_single (srcs.c:452-625, the
 // build without _USE_FAST_LENSING) and srcs_beams_postproc_single
-// (srcs.c:634-737) for one population.  One thread per source in catalogue
-// order: sources of one wavefront come from neighbouring cells, so their
-// rays run side by side and share the cache lines of the stencil reads.
+// (srcs.c:634-737) for one population.  2^lg lanes per source, sources in the
+// order of their directions (k_dir_*), so that the rays of a wavefront, and of
+// the wavefronts that run beside it on an XCD, cross the same cells.
 // ---------------------------------------------------------------------------
 namespace {
 
 struct BeamArgs {
   const float *phi;
-  int N, ngx, nr, na;
+  int N, ngx, nr, na, lg;                 // 2^lg lanes per source
   double idx, dr, idr, ox, oy, oz, factor_vel;
   double glob_idr, r_last, z_last, v1_0, v1_last;
   const double *r_arr, *z_arr, *v1_arr;   // background r-tables
@@ -516,17 +521,6 @@ struct BeamArgs {
   const float4 *vrec;                     // per cell (k_records): phi's central differences, delta
   const float2 *t6;                       // per cell (k_records): the tidal tensor's second differences
 };
-
-// The reference wraps once (beaming.c:129-133), which covers every cell the
-// march and the source reads reach when r_max is below the box size; the
-// full modulo keeps other inputs inside the grid.
-__device__ inline int wrap1(int v, int N) {
-  if (v >= N || v < 0) {
-    v %= N;
-    if (v < 0) v += N;
-  }
-  return v;
-}
 
 // get_element (beaming.c:31-117), RETURN_VEL: unscaled central differences,
 // periodic in x, y and z on one GPU (fourier.c:412-413).
@@ -544,7 +538,7 @@ __device__ inline void vel_at(const float *__restrict__ phi, int N, size_t ngx, 
 // get_element, RETURN_VEL | RETURN_TID: velocity and the 19-point tidal
 // tensor (xx, xy, xz, yy, yz, zz; mixed terms with 1/4).
 __device__ inline void vel_tid_at(const float *__restrict__ phi, int N, size_t ngx, size_t plane, int ix, int iy,
-                                  int iz, double v[3], double t[6]) {
+                                  int iz, float v[3], float t[6]) {
 #pragma clang fp contract(off)
   const int xh = ix == N - 1 ? 0 : ix + 1, xl = ix == 0 ? N - 1 : ix - 1;
   const int yh = iy == N - 1 ? 0 : iy + 1, yl = iy == 0 ? N - 1 : iy - 1;
@@ -581,12 +575,116 @@ __device__ inline void vel_cell(const float4 *__restrict__ vrec, const float *__
   }
 }
 
+// Order of the marches: sources by direction (cells of a G x G grid on each
+// face of a cube around the observer, in Morton order), so that the lanes of a
+// wavefront take nearly the same cells.  A counting sort: k_dir_count numbers the sources of a
+// bin, k_dir_scan sums the bins, k_dir_place writes the permutation (its order
+// within a bin is the atomics'; a source's result does not depend on it).
+constexpr int kDirG = 64;
+// The order pays where the records in reach (40 bytes per cell) are more than
+// the 256 MB last-level cache holds, from 32768 sources on: 950k sources at
+// 512^3 3.57 -> 2.00 ms with the records' pass, 384^3 1.84 -> 1.10, 256^3 0.71
+// -> 0.61, but 192^3 0.38 -> 0.41 and 128^3 0.20 -> 0.28; 19k sources at 512^3
+// 1.07 -> 1.08.  16 sources per bin (64: 2.07 ms; bins of 4 shells of distance
+// in 4 times wider cells, 2.08).
+constexpr int kDirMinN = 256;
+constexpr long long kDirMin = 32768, kDirPer = 16;
+constexpr size_t kBeamKeep = (size_t)1 << 30;
+
+__device__ inline uint32_t spread(uint32_t v) {
+  v = (v | (v << 4)) & 0x0f0fu;
+  v = (v | (v << 2)) & 0x3333u;
+  return (v | (v << 1)) & 0x5555u;
+}
+
+__device__ inline uint32_t dir_bin(const float4 p, int G) {
+  const float ax = fabsf(p.x), ay = fabsf(p.y), az = fabsf(p.z);
+  int face;
+  float m, u, v;
+  if (ax >= ay && ax >= az) { face = p.x < 0; m = ax; u = p.y; v = p.z; }
+  else if (ay >= az) { face = 2 + (p.y < 0); m = ay; u = p.x; v = p.z; }
+  else { face = 4 + (p.z < 0); m = az; u = p.x; v = p.y; }
+  const float s = m > 0 ? __builtin_amdgcn_rcpf(m) : 0.f;
+  const int iu = min(max((int)((u * s * 0.5f + 0.5f) * G), 0), G - 1);
+  const int iv = min(max((int)((v * s * 0.5f + 0.5f) * G), 0), G - 1);
+  return (uint32_t)(face * G * G) + (spread(iu) | spread(iv) << 1);
+}
+
+__global__ void k_dir_zero(uint32_t *__restrict__ cnt, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) cnt[i] = 0;
+}
+
+__global__ __launch_bounds__(256) void k_dir_count(const float4 *__restrict__ pos, uint32_t n, int G,
+                                                   uint32_t *__restrict__ cnt, uint2 *__restrict__ kr) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t k = dir_bin(pos[i], G);
+  kr[i] = make_uint2(k, atomicAdd(&cnt[k], 1u));
+}
+
+// Exclusive sum of cnt[nb] in place, nb a multiple of 4: one block, all of a
+// thread's loads in flight together (a run of bins per thread took 40 us).
+__global__ __launch_bounds__(1024) void k_dir_scan(uint4 *__restrict__ cnt, int nb4) {
+  constexpr int C = (6 * kDirG * kDirG + 4095) / 4096;
+  __shared__ uint32_t ws[C][16];
+  const int t = threadIdx.x, lane = t & 63;
+  uint4 v[C];
+  uint32_t inc[C];
+#pragma unroll
+  for (int k = 0; k < C; k++) v[k] = k * 1024 + t < nb4 ? cnt[k * 1024 + t] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int k = 0; k < C; k++) {
+    inc[k] = v[k].x + v[k].y + v[k].z + v[k].w;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t x = __shfl_up(inc[k], o);
+      if (lane >= o) inc[k] += x;
+    }
+    if (lane == 63) ws[k][t >> 6] = inc[k];
+  }
+  __syncthreads();
+  uint32_t base = 0;
+#pragma unroll
+  for (int k = 0; k < C; k++) {
+    uint32_t run = base + inc[k] - (v[k].x + v[k].y + v[k].z + v[k].w);
+    for (int w = 0; w < 16; w++) {
+      const uint32_t x = ws[k][w];
+      base += x;
+      if (w < (t >> 6)) run += x;
+    }
+    const uint4 e = make_uint4(run, run + v[k].x, run + v[k].x + v[k].y, run + v[k].x + v[k].y + v[k].z);
+    if (k * 1024 + t < nb4) cnt[k * 1024 + t] = e;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_dir_place(const uint2 *__restrict__ kr, uint32_t n,
+                                                   const uint32_t *__restrict__ off, uint32_t *__restrict__ perm) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const uint2 e = kr[i];
+  perm[off[e.x] + e.y] = i;
+}
+
+// A thread takes every 2^lg-th step of a source.  The projections of the
+// tidal tensor and of the gradient are constant along a ray, so the march
+// sums the six and two or three components with their radial weights in FP64
+// and projects the sums: 9 FP64 multiply-adds per step, where projecting at
+// each step took 17 + 5 multiplies and as many adds.  Bound by the latency of
+// the records' loads: 950k sources of 512^3 2.87 -> 0.96 ms (two steps in
+// flight: the same), 48k of 256^3 0.34 -> 0.21 with the records' pass.  Blocks of neighbouring
+// directions follow each other on one XCD (block b is logical block
+// (b % 8) (gridDim.x / 8) + b / 8, gridDim.x a multiple of 8).
 template <bool LENS, bool REC>
-__global__ __launch_bounds__(256) void k_src_beams(BeamArgs a, const float4 *__restrict__ pos, long long n,
+__global__ __launch_bounds__(256) void k_src_beams(BeamArgs a, const float4 *__restrict__ pos,
+                                                   const uint32_t *__restrict__ perm, long long n,
                                                    float *__restrict__ dz, float *__restrict__ lens) {
 #pragma clang fp contract(off)
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const unsigned blk = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  const int lg = LENS ? a.lg : 0, K = 1 << lg;
+  const long long j = ((long long)blk * 256 + threadIdx.x) >> lg;
+  const int sub = threadIdx.x & (K - 1);
+  if (j >= n) return;
+  const long long i = perm ? (long long)perm[j] : j;
   const float4 p = pos[i];
   const int N = a.N;
   const size_t ngx = (size_t)a.ngx, plane = (size_t)N * ngx;
@@ -633,7 +731,7 @@ __global__ __launch_bounds__(256) void k_src_beams(BeamArgs a, const float4 *__r
     }
   }
   const double vg = f_of_r(a.r_arr, a.v1_arr, a.glob_idr, a.r_last, rz, a.v1_0, a.v1_last);
-  dz[i] = (float)((double)vr * (vg * a.factor_vel));
+  if (sub == 0) dz[i] = (float)((double)vr * (vg * a.factor_vel));
   if (!LENS) return;
 
   double cth = u[2];
@@ -655,48 +753,53 @@ __global__ __launch_bounds__(256) void k_src_beams(BeamArgs a, const float4 *__r
                          (2 * sth * sph) * pre,        (2 * cth * sph * cph) * pre,
                          (-2 * sth * cph) * pre};
   const double *__restrict__ f0 = a.fac, *__restrict__ f1 = a.fac + a.nr, *__restrict__ f2 = a.fac + 2 * a.nr;
-  double dtx = 0, dty = 0, kp = 0, e1 = 0, e2 = 0;
+  double st[6] = {}, sv[3] = {};
   const int irmax = min((int)(r * a.idr + 0.5), a.nr - 1);
-  for (int i_r = 0; i_r <= irmax; i_r++) {
-    const double rm = (i_r + 0.5) * a.dr;
-    int ix[3];
-    ix[0] = wrap1((int)((rm * u[0] + a.ox) * a.idx + 0.5), N);
-    ix[1] = wrap1((int)((rm * u[1] + a.oy) * a.idx + 0.5), N);
-    ix[2] = wrap1((int)((rm * u[2] + a.oz) * a.idx + 0.5), N);
-    double vp[3], tp[6];
-    if (REC) {
-      const size_t o = ((size_t)ix[2] * N + ix[1]) * N + ix[0];
-      const float4 q = a.vrec[o];
-      const float2 t0 = a.t6[3 * o], t1 = a.t6[3 * o + 1], t2 = a.t6[3 * o + 2];
-      vp[0] = q.x;
-      vp[1] = q.y;
-      vp[2] = q.z;
-      tp[0] = t0.x;
-      tp[1] = t0.y;
-      tp[2] = t1.x;
-      tp[3] = t1.y;
-      tp[4] = t2.x;
-      tp[5] = t2.y;
-    } else {
-      vel_tid_at(phi, N, ngx, plane, ix[0], ix[1], ix[2], vp, tp);
-    }
-    const double fr = f1[i_r] * r - f2[i_r];
-    const double frm = 2 * (f0[i_r] * r - f1[i_r]);
-    double de1 = 0, de2 = 0, dk = 0;
+  Ray ray;
+  int64_t x[3];
 #pragma unroll
-    for (int q = 0; q < 6; q++) {
-      de1 += re1[q] * tp[q];
-      de2 += (q < 5 ? re2[q] : 0.0) * tp[q];
-      dk += rk[q] * tp[q];
+  for (int ax = 0; ax < 3; ax++) ray.u[ax] = u[ax];
+  ray_setup(ray, a.dr, a.idx, a.ox, a.oy, a.oz);
+#pragma unroll
+  for (int ax = 0; ax < 3; ax++) x[ax] = ray.base[ax] + (int64_t)sub * ray.step[ax];
+  for (int i_r = sub; i_r <= irmax; i_r += K) {
+    int c[3];
+    ray_cell(ray, x, i_r, N, a.dr, a.idx, a.ox, a.oy, a.oz, c);
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) x[ax] += ray.step[ax] << lg;
+    float vp[4], tp[6];
+    if (REC) {
+      const size_t o = ((size_t)c[2] * N + c[1]) * N + c[0];
+      const float *q = (const float *)(a.t6 + 3 * o);
+      __builtin_memcpy(vp, &a.vrec[o], 16);
+      __builtin_memcpy(tp, q, 16);
+      __builtin_memcpy(tp + 4, q + 4, 8);
+    } else {
+      vel_tid_at(phi, N, ngx, plane, c[0], c[1], c[2], vp, tp);
     }
-    const double dvx = ux[0] * vp[0] + ux[1] * vp[1] + ux[2] * vp[2];
-    const double dvy = uy[0] * vp[0] + uy[1] * vp[1] + 0.0 * vp[2];
-    e1 += de1 * fr;
-    e2 += de2 * fr;
-    kp += dk * fr;
-    dtx += dvx * frm;
-    dty += dvy * frm;
+    const double fr = fma(f1[i_r], r, -f2[i_r]);
+    const double frm = 2 * fma(f0[i_r], r, -f1[i_r]);
+#pragma unroll
+    for (int q = 0; q < 6; q++) st[q] = fma(fr, (double)tp[q], st[q]);
+#pragma unroll
+    for (int q = 0; q < 3; q++) sv[q] = fma(frm, (double)vp[q], sv[q]);
   }
+  for (int o = 1; o < K; o <<= 1) {
+#pragma unroll
+    for (int q = 0; q < 6; q++) st[q] += __shfl_xor(st[q], o);
+#pragma unroll
+    for (int q = 0; q < 3; q++) sv[q] += __shfl_xor(sv[q], o);
+  }
+  if (sub != 0) return;
+  double kp = 0, e1 = 0, e2 = 0;
+#pragma unroll
+  for (int q = 0; q < 6; q++) {
+    e1 += re1[q] * st[q];
+    if (q < 5) e2 += re2[q] * st[q];
+    kp += rk[q] * st[q];
+  }
+  const double dtx = ux[0] * sv[0] + ux[1] * sv[1] + ux[2] * sv[2];
+  const double dty = uy[0] * sv[0] + uy[1] * sv[1];
   const double RTOD = 57.2957795;
   float *o = lens + 5 * i;
   o[0] = (float)e1;
@@ -746,23 +849,53 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
   const int nr = N / 2;
   const double dr = r_max / nr;
   // fac_r_0/1/2 (srcs.c:470-480), FP64 on the host from the uploaded tables
-  std::vector<double> rr(na), zz(na), dd(na);
-  CLR_HIP(c, hipMemcpy(rr.data(), c->bg, na * sizeof(double), hipMemcpyDeviceToHost));
-  CLR_HIP(c, hipMemcpy(zz.data(), c->bg + na, na * sizeof(double), hipMemcpyDeviceToHost));
-  CLR_HIP(c, hipMemcpy(dd.data(), c->bg + 2 * (size_t)na, na * sizeof(double), hipMemcpyDeviceToHost));
+  const double *rr = c->h_r.data(), *zz = c->h_z.data(), *dd = c->h_d1.data();
   std::vector<double> fac(3 * (size_t)nr);
   for (int i = 0; i < nr; i++) {
     const double rm = (i + 0.5) * dr;
-    const double pg = f_of_r(rr.data(), dd.data(), c->glob_idr, c->r_last, rm, 1.0, dd[na - 1]) *
-                      (1 + f_of_r(rr.data(), zz.data(), c->glob_idr, c->r_last, rm, 0.0, zz[na - 1]));
+    const double pg = f_of_r(rr, dd, c->glob_idr, c->r_last, rm, 1.0, dd[na - 1]) *
+                      (1 + f_of_r(rr, zz, c->glob_idr, c->r_last, rm, 0.0, zz[na - 1]));
     fac[i] = pg * dr;
     fac[nr + i] = rm * pg * dr;
     fac[2 * nr + i] = rm * rm * pg * dr;
   }
-  const size_t tab_bytes = (3 * (size_t)nr + na) * sizeof(double);
-  int rc = clr_ensure(c, &c->misc, &c->misc_n, tab_bytes);
-  if (rc) return rc;
-  double *dfac = (double *)c->misc, *da2r = dfac + 3 * nr;
+  const size_t tab_bytes = (3 * (size_t)nr + na + 1) / 2 * 2 * sizeof(double);
+  const int per = lens ? 6 : 1;
+  // the results and the order of the marches follow the tables in the
+  // context's scratch buffer up to kBeamKeep bytes, else in one of this call
+  bool order = lens && N >= kDirMinN && n >= kDirMin && n < (1ll << 31);
+  int G = 1;
+  while (G < kDirG && 24ll * G * G * kDirPer <= n) G *= 2;
+  const int nb = (6 * G * G + 3) / 4 * 4;
+  struct Own {
+    void *p = nullptr;
+    ~Own() {
+      if (p) (void)hipFree(p);
+    }
+  } own;
+  char *buf = nullptr;
+  for (;;) {
+    const size_t need =
+        tab_bytes + (order ? (size_t)(n + 1) * 12 + (size_t)nb * 4 : 0) + (size_t)n * per * sizeof(float);
+    int rc = CLR_OK;
+    if (need <= kBeamKeep) {
+      rc = clr_ensure(c, &c->misc, &c->misc_n, need);
+      buf = (char *)c->misc;
+    } else if (hipMalloc(&own.p, need) != hipSuccess) {
+      (void)hipGetLastError();
+      own.p = nullptr;
+      rc = clr_fail(c, CLR_ERR_HIP, "source beams: no device memory for %zu bytes", need);
+    } else {
+      buf = (char *)own.p;
+    }
+    if (rc == CLR_OK) break;
+    if (!order) return rc;
+    order = false;
+  }
+  double *dfac = (double *)buf, *da2r = dfac + 3 * nr;
+  uint32_t *cnt = (uint32_t *)(buf + tab_bytes), *perm = cnt + (order ? nb : 0);
+  uint2 *kr = (uint2 *)(perm + (order ? (n + 1) / 2 * 2 : 0));
+  float *tmp = (float *)(kr + (order ? n : 0));
   CLR_HIP(c, hipMemcpyAsync(dfac, fac.data(), 3 * (size_t)nr * sizeof(double), hipMemcpyHostToDevice, c->stream));
   CLR_HIP(c, hipMemcpyAsync(da2r, r_arr_a2r, na * sizeof(double), hipMemcpyHostToDevice, c->stream));
   BeamArgs a{};
@@ -792,27 +925,34 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
   a.v1_arr = c->bg + 3 * (size_t)na;
   a.a2r = da2r;
   a.fac = dfac;
-  const int per = lens ? 6 : 1;
-  float *tmp = nullptr;
-  CLR_HIP(c, hipMalloc((void **)&tmp, (size_t)n * per * sizeof(float)));
   CLR_HIP(c, hipEventRecord(c->ev0, c->stream));
-  const dim3 grid((unsigned)((n + 255) / 256));
+  const float4 *pos = (const float4 *)C.pos;
+  a.lg = lens ? lanes_lg(n, nr) : 0;
+  const unsigned nblk = (unsigned)((((n << a.lg) + 255) / 256 + 7) / 8 * 8);
+  const dim3 grid(nblk);
+  if (order) {
+    const unsigned g1 = (unsigned)((n + 255) / 256);
+    hipLaunchKernelGGL(k_dir_zero, dim3((nb + 255) / 256), dim3(256), 0, c->stream, cnt, nb);
+    hipLaunchKernelGGL(k_dir_count, dim3(g1), dim3(256), 0, c->stream, pos, (uint32_t)n, G, cnt, kr);
+    hipLaunchKernelGGL(k_dir_scan, dim3(1), dim3(1024), 0, c->stream, (uint4 *)cnt, nb / 4);
+    hipLaunchKernelGGL(k_dir_place, dim3(g1), dim3(256), 0, c->stream, kr, (uint32_t)n, cnt, perm);
+  } else {
+    perm = nullptr;
+  }
   // per-cell records (velocity differences; with lensing also the tidal
   // tensor) when they fit in a quarter of the free device memory
   const bool rec = clr_cell_records(c, lens != nullptr);
   a.vrec = (const float4 *)c->velrec;
   a.t6 = (const float2 *)c->tidal;
   if (lens && rec)
-    hipLaunchKernelGGL((k_src_beams<true, true>), grid, dim3(256), 0, c->stream, a, (const float4 *)C.pos, n, tmp,
-                       tmp + n);
+    hipLaunchKernelGGL((k_src_beams<true, true>), grid, dim3(256), 0, c->stream, a, pos, perm, n, tmp, tmp + n);
   else if (lens)
-    hipLaunchKernelGGL((k_src_beams<true, false>), grid, dim3(256), 0, c->stream, a, (const float4 *)C.pos, n, tmp,
-                       tmp + n);
+    hipLaunchKernelGGL((k_src_beams<true, false>), grid, dim3(256), 0, c->stream, a, pos, perm, n, tmp, tmp + n);
   else if (rec)
-    hipLaunchKernelGGL((k_src_beams<false, true>), grid, dim3(256), 0, c->stream, a, (const float4 *)C.pos, n, tmp,
+    hipLaunchKernelGGL((k_src_beams<false, true>), grid, dim3(256), 0, c->stream, a, pos, perm, n, tmp,
                        (float *)nullptr);
   else
-    hipLaunchKernelGGL((k_src_beams<false, false>), grid, dim3(256), 0, c->stream, a, (const float4 *)C.pos, n, tmp,
+    hipLaunchKernelGGL((k_src_beams<false, false>), grid, dim3(256), 0, c->stream, a, pos, perm, n, tmp,
                        (float *)nullptr);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipEventRecord(c->ev1, c->stream);
@@ -820,7 +960,6 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
   if (e == hipSuccess && lens)
     e = hipMemcpyAsync(lens, tmp + n, (size_t)n * 5 * sizeof(float), hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  (void)hipFree(tmp);
   if (e != hipSuccess) return clr_fail(c, CLR_ERR_HIP, "source beams: %s", hipGetErrorString(e));
   float ms = 0;
   hipEventElapsedTime(&ms, c->ev0, c->ev1);
