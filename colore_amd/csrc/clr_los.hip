@@ -861,8 +861,8 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
   }
   const size_t tab_bytes = (3 * (size_t)nr + na + 1) / 2 * 2 * sizeof(double);
   const int per = lens ? 6 : 1;
-  // the results and the order of the marches follow the tables in the
-  // context's scratch buffer up to kBeamKeep bytes, else in one of this call
+  // the tables, the order of the marches and the results: in a buffer that the
+  // context keeps up to kBeamKeep bytes, else in one of this call
   bool order = lens && N >= kDirMinN && n >= kDirMin && n < (1ll << 31);
   int G = 1;
   while (G < kDirG && 24ll * G * G * kDirPer <= n) G *= 2;
@@ -879,8 +879,8 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
         tab_bytes + (order ? (size_t)(n + 1) * 12 + (size_t)nb * 4 : 0) + (size_t)n * per * sizeof(float);
     int rc = CLR_OK;
     if (need <= kBeamKeep) {
-      rc = clr_ensure(c, &c->misc, &c->misc_n, need);
-      buf = (char *)c->misc;
+      rc = clr_ensure(c, &c->beam_ws, &c->beam_ws_n, need);
+      buf = (char *)c->beam_ws;
     } else if (hipMalloc(&own.p, need) != hipSuccess) {
       (void)hipGetLastError();
       own.p = nullptr;
