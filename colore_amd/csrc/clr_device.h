@@ -23,13 +23,23 @@ __host__ __device__ constexpr int grid_pitch(int N) { return (2 * (N / 2 + 1) + 
 // ---------------------------------------------------------------------------
 struct u32x4 { uint32_t x, y, z, w; };
 
+// a ^ b ^ c: one v_bitop3_b32 (the compiler's two v_xor_b32 were a third of a
+// draw's instructions)
+__host__ __device__ inline uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 __host__ __device__ inline u32x4 philox4x32_10(u32x4 c, uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int i = 0; i < 10; i++) {
     if (i) { k0 += 0x9E3779B9u; k1 += 0xBB67AE85u; }
     // one 32x32->64 product per multiplier (a single v_mad_u64_u32 on gfx950)
     const uint64_t p0 = (uint64_t)0xD2511F53u * c.x, p1 = (uint64_t)0xCD9E8D57u * c.z;
-    c = u32x4{(uint32_t)(p1 >> 32) ^ c.y ^ k0, (uint32_t)p1, (uint32_t)(p0 >> 32) ^ c.w ^ k1, (uint32_t)p0};
+    c = u32x4{xor3((uint32_t)(p1 >> 32), c.y, k0), (uint32_t)p1, xor3((uint32_t)(p0 >> 32), c.w, k1), (uint32_t)p0};
   }
   return c;
 }

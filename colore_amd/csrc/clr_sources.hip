@@ -45,7 +45,7 @@ struct PopTab {
   const float4 *tab;         // k_pop_table's bins, bound and coarse bounds
   double bz0, norm0, normf;
   int model, ipop;
-  uint8_t *cnt8;             // one byte per cell
+  uint8_t *cnt8;             // one byte per cell, unset in the blocks whose bytes would all be 0
   uint32_t *btot;            // one total per block
   const long long *boff;     // exclusive prefix of btot
   uint4 *desc;               // the catalogue's position buffer, holding descriptors
@@ -292,15 +292,22 @@ __device__ inline int settle_cell(const SrcArgs &a, const float4 *tab, int model
 
 // k_count works on 1024 cells per wavefront (16 per lane, two of the 512-cell
 // blocks whose totals k_scan and k_fill use), so that its fixed costs per
-// wavefront -- the density loads' latency, the coarse-bound gathers, the queue
-// pass -- are shared by twice the cells.
+// wavefront -- the density loads' latency, the coarse-bound gathers -- are
+// shared by twice the cells.  It is bound by its vector instructions.
 constexpr int kCountLaneCells = 16;
 constexpr int kCountCells = kLanes * kCountLaneCells;
 constexpr int kCountSubs = kCountCells / kBlockCells;
+static_assert(kCountSubs == 2, "half a wavefront of k_count and k_fill is one block");
+constexpr int kFillWaves = 4;   // wavefronts per block of k_fill (N is a multiple of 16, N^3 of 4 x 1024)
 // queue entry: cell within the wavefront's 1024 (bits 0-9) | population
 // (bits 10-13) | the uniform's high 16 bits << 16.  The queue is worked when
-// another population's 1024 entries might not fit, so usually once.
-constexpr int kQueueCap = kCountCells + kCountCells / 4;
+// another 8 cells per lane might not fit, and after the last population.  It is
+// kept that short because the wavefronts that fit a CU's LDS hide the loads'
+// latency: with room for a population's 1024 cells more, three sparse
+// populations at 1024^3 took 2.12 ms instead of 1.84 and a dense one at 512^3
+// 0.87 instead of 0.80 (256 cells: 1.90 and 0.86; one queue for four
+// wavefronts, 1.84 and 0.94).
+constexpr int kQueueCap = kCountCells / 2 + kLanes;
 
 template <bool FUSED>
 __global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(6))) void k_count(SrcArgs a) {
@@ -334,7 +341,32 @@ __global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(6))) voi
       smodel[ip] = a.pop[ip].model;
     }
   }
-
+  int qn = 0;   // uniform
+  // --- B: the queue, all lanes busy ------------------------------------------
+  auto work = [&]() {
+    __syncthreads();   // one wavefront: orders the LDS writes before the reads below
+    for (int i = lane; i < qn; i += kLanes) {
+      const uint32_t e = queue[i];
+      const int cb = (int)(e & (kCountCells - 1));
+      const int q = (int)((e >> 10) & 15u);
+      const uint32_t hi = e >> 16;
+      const size_t cell = base + cb;
+      const uint2 gl = sgeo[cb / kCountLaneCells];
+      const int ix = (int)(gl.x & 0xFFFFu) + cb % kCountLaneCells, iy = (int)(gl.x >> 16), iz = (int)gl.y;
+      const float dl = cell_density(a, a.g[((size_t)iz * N + iy) * a.ngx + ix], ix, iy, iz);
+      const int k = settle_cell(a, stab[q], smodel[q], a.pop[0].ipop + q, q, cell, ix, iy, iz, dl, hi);
+      ((uint8_t *)(sbytes + q * kLanes))[cb] = (uint8_t)(k < 0 ? kBytePending : (k < kBytePending ? k : kByteEscape));
+      if (k > 0) atomicAdd(&stot[q][cb / kBlockCells], (uint32_t)k);
+      if (k >= kBytePending) {
+        // the exact count of a saturated byte goes to the escape list
+        const unsigned x = atomicAdd(a.esc_n, 1u);
+        if (x < a.esc_cap)
+          a.esc[x] = make_ulonglong2(((unsigned long long)q << 56) | (unsigned long long)cell, (unsigned long long)k);
+      }
+    }
+    __syncthreads();
+    qn = 0;
+  };
   // --- the lane's 16 cells: largest delta and the range of their radii ------
   // Every count of the lane is 0 where u < exp(-lambda_max) for an upper
   // bound lambda_max of the reference's lambda over the 16 cells:
@@ -386,7 +418,6 @@ __global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(6))) voi
     }
   }
 
-  int qn = 0;   // uniform
   for (int ip = 0; ip < a.npop; ip++) {
     const PopTab &P = a.pop[ip];
     const int model = P.model;
@@ -417,8 +448,9 @@ __global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(6))) voi
       }
     }
     if (__ballot(hcrit < 65536) != 0ull) {
-#pragma unroll
+#pragma unroll 1
       for (int g = 0; g < kCountLaneCells / 8; g++) {
+        if (qn > kQueueCap - 8 * kLanes) work();
         // the high 16 bits of 8 cells come from one draw at site cell/8
         const u32x4 rr = draw((cell0 >> 3) + g, stream_poisson(P.ipop), 0u, a.seed);
 #pragma unroll
@@ -435,38 +467,16 @@ __global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(6))) voi
         }
       }
     }
-    // --- B: the queue, all lanes busy; run when another population might
-    // not fit, and after the last -------------------------------------------
-    if (qn > kQueueCap - kCountCells || ip == a.npop - 1) {
-      __syncthreads();   // one wavefront: orders the LDS writes above before the reads below
-      for (int i = lane; i < qn; i += kLanes) {
-        const uint32_t e = queue[i];
-        const int cb = (int)(e & (kCountCells - 1));
-        const int q = (int)((e >> 10) & 15u);
-        const uint32_t hi = e >> 16;
-        const size_t cell = base + cb;
-        const uint2 gl = sgeo[cb / kCountLaneCells];
-        const int ix = (int)(gl.x & 0xFFFFu) + cb % kCountLaneCells, iy = (int)(gl.x >> 16), iz = (int)gl.y;
-        const float dl = cell_density(a, a.g[((size_t)iz * N + iy) * a.ngx + ix], ix, iy, iz);
-        const int k = settle_cell(a, stab[q], smodel[q], a.pop[0].ipop + q, q, cell, ix, iy, iz, dl, hi);
-        ((uint8_t *)(sbytes + q * kLanes))[cb] =
-            (uint8_t)(k < 0 ? kBytePending : (k < kBytePending ? k : kByteEscape));
-        if (k > 0) atomicAdd(&stot[q][cb / kBlockCells], (uint32_t)k);
-        if (k >= kBytePending) {
-          // the exact count of a saturated byte goes to the escape list
-          const unsigned x = atomicAdd(a.esc_n, 1u);
-          if (x < a.esc_cap)
-            a.esc[x] = make_ulonglong2(((unsigned long long)q << 56) | (unsigned long long)cell, (unsigned long long)k);
-        }
-      }
-      __syncthreads();
-      qn = 0;
-    }
   }
-  // --- the bytes of the lane's 16 cells and the two block totals -------------
+  work();
+  // --- the bytes of the lane's 16 cells and the two block totals; the bytes
+  // of a block (half a wavefront) only where one is not 0: a third of the
+  // stores and of k_fill's reads where a population has 0.4 sources per block
   for (int ip = 0; ip < a.npop; ip++) {
     const PopTab &P = a.pop[ip];
-    *(uint4 *)(P.cnt8 + cell0) = sbytes[ip * kLanes + lane];
+    const uint4 w = sbytes[ip * kLanes + lane];
+    const unsigned long long any = __ballot((w.x | w.y | w.z | w.w) != 0);
+    if ((uint32_t)(any >> (lane & 32)) != 0) *(uint4 *)(P.cnt8 + cell0) = w;
     if (lane < kCountSubs) P.btot[blk * kCountSubs + lane] = stot[ip][lane];
   }
 }
@@ -583,52 +593,89 @@ __device__ inline int escaped_count(const ulonglong2 *esc, unsigned n, unsigned 
 }
 
 // One wavefront per kCountCells cells (two 512-cell blocks of the scan): a lane
-// reads the 16 count bytes of its cells per population.
-__global__ __launch_bounds__(kLanes) void k_fill(SrcArgs a) {
+// reads the 16 count bytes of its cells per population where its block holds
+// sources, and visits the cells whose byte is not 0 (three sparse populations
+// at 1024^3: 747 -> 434 us; all 16 cells unrolled, 95 VGPRs, 810).
+__global__ __launch_bounds__(kFillWaves *kLanes) void k_fill(SrcArgs a) {
   constexpr int G = 2;   // populations whose loads are in flight together
-  const int lane = threadIdx.x;
-  const size_t w0 = (size_t)blockIdx.x * kCountSubs;   // first 512-cell block
-  const uint64_t cell0 = (uint64_t)blockIdx.x * kCountCells + (uint64_t)kCountLaneCells * lane;
+  const int lane = threadIdx.x & 63;
+  const size_t wave = (size_t)blockIdx.x * kFillWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t w0 = wave * kCountSubs;   // first 512-cell block
+  const uint64_t cell0 = (uint64_t)wave * kCountCells + (uint64_t)kCountLaneCells * lane;
   for (int g0 = 0; g0 < a.npop; g0 += G) {
-    long long b0[G], b1[G];
+    long long b0[G], bm[G], b1[G];
     uint4 w[G];
 #pragma unroll
     for (int q = 0; q < G; q++) {
-      b0[q] = b1[q] = 0;
-      w[q] = make_uint4(0u, 0u, 0u, 0u);
+      b0[q] = bm[q] = b1[q] = 0;
       if (g0 + q < a.npop) {
         const PopTab &P = a.pop[g0 + q];
         b0[q] = P.boff[w0];
+        bm[q] = P.boff[w0 + 1];
         b1[q] = P.boff[w0 + kCountSubs];
-        w[q] = *(const uint4 *)(P.cnt8 + cell0);
       }
     }
 #pragma unroll
     for (int q = 0; q < G; q++) {
-      if (g0 + q >= a.npop || b1[q] == b0[q]) continue;   // uniform: no sources in these cells
-      const uint32_t wd[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
-      int k[kCountLaneCells];
-      long long mine = 0;
-#pragma unroll
-      for (int c = 0; c < kCountLaneCells; c++) {
-        k[c] = (int)((wd[c / 4] >> (8 * (c & 3))) & 0xFFu);
-        if (k[c] == kByteEscape)
-          k[c] = escaped_count(a.esc, a.esc_count, ((unsigned long long)(g0 + q) << 56) | (cell0 + c));
-        mine += k[c];
+      w[q] = make_uint4(0u, 0u, 0u, 0u);
+      if (lane < 32 ? bm[q] != b0[q] : b1[q] != bm[q]) w[q] = *(const uint4 *)(a.pop[g0 + q].cnt8 + cell0);
+    }
+    for (int q = 0; q < G; q++) {
+      if (b1[q] == b0[q]) continue;   // uniform: no sources in these cells
+      uint64_t lo = w[q].x | (uint64_t)w[q].y << 32, hi = w[q].z | (uint64_t)w[q].w << 32;
+      const unsigned long long key = ((unsigned long long)(g0 + q) << 56) | cell0;
+      auto next = [&](int &c) -> int {   // the next cell with sources (its byte cleared) and its count
+        const bool l = lo != 0;
+        const uint64_t v = l ? lo : hi;
+        const int sh = __builtin_ctzll(v) & ~7;
+        c = (sh >> 3) + (l ? 0 : 8);
+        const uint64_t rest = v & ~(0xFFull << sh);
+        if (l) lo = rest;
+        else hi = rest;
+        const int k = (int)(v >> sh) & 0xFF;
+        return k == kByteEscape ? escaped_count(a.esc, a.esc_count, key + c) : k;
+      };
+      // the lane's sources: its byte sum, or by cell where one has escaped
+      long long mine;
+      {
+        uint32_t sum = __builtin_amdgcn_sad_u8(w[q].x, 0u, 0u);
+        sum = __builtin_amdgcn_sad_u8(w[q].y, 0u, sum);
+        sum = __builtin_amdgcn_sad_u8(w[q].z, 0u, sum);
+        sum = __builtin_amdgcn_sad_u8(w[q].w, 0u, sum);
+        mine = sum;
+        if (sum >= kByteEscape) {
+          const uint64_t l0 = lo, h0 = hi;
+          int c;
+          mine = 0;
+          while (lo | hi) mine += next(c);
+          lo = l0;
+          hi = h0;
+        }
       }
-      long long incl = mine;
+      long long pid = b0[q];
+      if (__ballot(mine >= kByteEscape) == 0) {
+        int incl = (int)mine;
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const long long y = __shfl_up(incl, off);
-        if (lane >= off) incl += y;
+        for (int off = 1; off < 64; off <<= 1) {
+          const int y = __shfl_up(incl, off);
+          if (lane >= off) incl += y;
+        }
+        pid += incl - (int)mine;
+      } else {
+        long long incl = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+          const long long y = __shfl_up(incl, off);
+          if (lane >= off) incl += y;
+        }
+        pid += incl - mine;
       }
-      long long pid = b0[q] + incl - mine;
       uint4 *desc = a.pop[g0 + q].desc;
-#pragma unroll
-      for (int c = 0; c < kCountLaneCells; c++) {
+      const long long lim = b1[q] < a.pop[g0 + q].cap ? b1[q] : a.pop[g0 + q].cap;
+      while (lo | hi) {
+        int c;
+        const int k = next(c);
         const uint64_t cell = cell0 + c;
-        const long long lim = b1[q] < a.pop[g0 + q].cap ? b1[q] : a.pop[g0 + q].cap;
-        for (int is = 0; is < k[c]; is++, pid++)
+        for (int is = 0; is < k; is++, pid++)
           if (pid < lim) desc[pid] = make_uint4((uint32_t)cell, (uint32_t)(cell >> 32), (uint32_t)is, 0u);
       }
     }
@@ -760,14 +807,16 @@ __global__ void k_graph_flags(const unsigned *__restrict__ esc_n, const unsigned
 
 // Per-cell counts (the reference's nsources array, srcs.c:125, without the
 // row padding) of cells [cell0, cell0+n) of population slot q: the count
-// byte, or the escape-list entry of a saturated byte.
-__global__ void k_expand_counts(const uint8_t *__restrict__ cnt8, const ulonglong2 *__restrict__ esc,
+// byte, or the escape-list entry of a saturated byte; 0 in blocks without
+// sources, whose bytes are not set.
+__global__ void k_expand_counts(const uint8_t *__restrict__ cnt8, const uint32_t *__restrict__ btot,
+                                const ulonglong2 *__restrict__ esc,
                                 unsigned nesc, unsigned long long q, uint64_t cell0, uint64_t n,
                                 int32_t *__restrict__ out) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const uint64_t cell = cell0 + i;
-  int k = cnt8[cell];
+  int k = btot[cell / kBlockCells] ? cnt8[cell] : 0;
   if (k == kByteEscape) k = escaped_count(esc, nesc, (q << 56) | cell);
   out[i] = k;
 }
@@ -1191,7 +1240,7 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
   }
   CLR_HIP(c, hipEventRecord(c->ev2, c->stream));
   if (total > 0) {
-    hipLaunchKernelGGL(k_fill, dim3((unsigned)(ncells / kCountCells)), dim3(kLanes), 0, c->stream, a);
+    hipLaunchKernelGGL(k_fill, dim3((unsigned)(ncells / (kFillWaves * kCountCells))), dim3(kFillWaves * kLanes), 0, c->stream, a);
     CLR_HIP(c, hipGetLastError());
   }
   rc = clr_phi_ready(c, 0);   // k_write reads phi
@@ -1274,7 +1323,7 @@ int clr_launch_fetch_counts(clr_ctx *c, int ipop, int iz0, int nz, int32_t *out)
   int32_t *tmp = nullptr;
   CLR_HIP(c, hipMalloc((void **)&tmp, n * sizeof(int32_t)));
   hipLaunchKernelGGL(k_expand_counts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, cnt8,
-                     (const ulonglong2 *)((char *)c->esc + 16), c->cnt_nesc, (unsigned long long)q, cell0, n, tmp);
+                     (const uint32_t *)(cnt8 + (size_t)N * N * N), (const ulonglong2 *)((char *)c->esc + 16), c->cnt_nesc, (unsigned long long)q, cell0, n, tmp);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemcpyAsync(out, tmp, n * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -1572,7 +1621,7 @@ int clr_enqueue_sources(clr_ctx *c, hipStream_t st, uint32_t seed, int nside_bas
   hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nsb, (unsigned)np), dim3(kScanB), 0, st, sp, nblocks);
   hipLaunchKernelGGL(k_graph_flags, dim3(1), dim3(64), 0, st, (const unsigned *)a.esc_n,
                      (const unsigned *)a.exq_n, a.exq_cap, np, gt, flag_dev);
-  hipLaunchKernelGGL(k_fill, dim3((unsigned)(ncells / kCountCells)), dim3(kLanes), 0, st, a);
+  hipLaunchKernelGGL(k_fill, dim3((unsigned)(ncells / (kFillWaves * kCountCells))), dim3(kFillWaves * kLanes), 0, st, a);
   for (int i = 0; i < np; i++) {
     CatalogDev &C = c->cat[i];
     WriteArgs w{};
