@@ -623,7 +623,7 @@ __global__ __launch_bounds__(256) void k_shell_final(const double *__restrict__ 
 }
 
 // Per tracer t: norm table on the NA r-grid.  sums = [nz][nq] from
-// k_shell_final; work = scratch of 2*nz doubles.
+// k_shell_final.
 constexpr int kNormMaxShells = 1024;
 struct NormOuts {
   double *p[3 * CLR_NPOP_MAX];
@@ -640,16 +640,17 @@ __global__ __launch_bounds__(256) void k_norm_table(const double *__restrict__ s
 #pragma clang fp contract(off)
   __shared__ double zarr[kNormMaxShells], nrm[kNormMaxShells];
   const int t = blockIdx.y;
-  if (threadIdx.x == 0) {
-    for (int iz = 0; iz < nz; iz++) {
-      const double n = sums[iz * nq + 0];
-      zarr[iz] = sums[iz * nq + 1];
-      nrm[iz] = sums[iz * nq + 2 + t];
-      if (n > 0) {
-        zarr[iz] /= n;
-        nrm[iz] = n / nrm[iz];
-      }
+  for (int iz = threadIdx.x; iz < nz; iz += blockDim.x) {
+    const double n = sums[iz * nq + 0];
+    zarr[iz] = sums[iz * nq + 1];
+    nrm[iz] = sums[iz * nq + 2 + t];
+    if (n > 0) {
+      zarr[iz] /= n;
+      nrm[iz] = n / nrm[iz];
     }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
     zarr[0] = 0;
     zarr[nz - 1] = zmax;
     nrm[0] = nrm[1];
@@ -804,8 +805,7 @@ int clr_launch_density(clr_ctx *c, int dens_type, double sigma2) {
 // ---------------------------------------------------------------------------
 constexpr size_t kNoAllocVals = 320;
 constexpr size_t kNoAllocTabFloat4 = (size_t)CLR_NA * (2 + kMaxTr) / 2;
-constexpr size_t kNoAllocDoubles = (size_t)kShellBlocks * kNoAllocVals + kNoAllocVals + 2 * (size_t)kNormMaxShells +
-                                   2 * (size_t)kMaxTr;
+constexpr size_t kNoAllocDoubles = (size_t)kShellBlocks * kNoAllocVals + kNoAllocVals + 2 * (size_t)kMaxTr;
 constexpr size_t kNoAllocBytes = (kNoAllocDoubles * sizeof(double) + 255) / 256 * 256 + kNoAllocTabFloat4 * 16;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -882,7 +882,7 @@ int clr_launch_norms(clr_ctx *c, int lognormal_fused, double sigma2, int cap, in
   bool all0 = true;
   for (int t = 0; t < ntr; t++) all0 = all0 && a.model[t] == CLR_BIAS_EXPONENTIAL;
   const size_t nvals = (size_t)nz * nq;
-  double *partial, *fin, *work;
+  double *partial, *fin;   // (the tracers' edge values follow the sums)
   float2 *tab;
   if (scratch_base) {
     // no allocation: everything in the device's static scratch
@@ -893,15 +893,13 @@ int clr_launch_norms(clr_ctx *c, int lognormal_fused, double sigma2, int cap, in
       return clr_fail(c, CLR_ERR_ARG, "r-tables of %d entries exceed the static scratch", na);
     partial = (double *)scratch_base;
     fin = partial + (size_t)kShellBlocks * nvals;
-    work = fin + nvals;
     tab = (float2 *)((char *)scratch_base + (kNoAllocDoubles * sizeof(double) + 255) / 256 * 256);
   } else {
-    const size_t need = (size_t)kShellBlocks * nvals + nvals + 2 * nz + 2 * ntr;
+    const size_t need = (size_t)kShellBlocks * nvals + nvals + 2 * ntr;
     int rc = clr_ensure(c, (void **)&c->red, &c->red_n, need * sizeof(double));
     if (rc) return rc;
     partial = c->red;
     fin = c->red + (size_t)kShellBlocks * nvals;
-    work = fin + nvals;
     rc = clr_ensure(c, &c->misc, &c->misc_n, (size_t)na * nq * sizeof(float2));
     if (rc) return rc;
     tab = (float2 *)c->misc;
@@ -923,7 +921,7 @@ int clr_launch_norms(clr_ctx *c, int lognormal_fused, double sigma2, int cap, in
       outs.e[t] = c->tr[tk[t]][tp[t]].edge;
     }
     hipLaunchKernelGGL(k_norm_table, dim3((unsigned)((na + 255) / 256), (unsigned)ntr), dim3(256), 0, c->stream,
-                       fin, nz, nq, zmax, r, zt, c->glob_idr, c->r_last, z_last, na, outs, work + 2 * nz);
+                       fin, nz, nq, zmax, r, zt, c->glob_idr, c->r_last, z_last, na, outs, fin + nvals);
     CLR_HIP(c, hipGetLastError());
   }
   CLR_HIP(c, hipEventRecord(c->ev1, c->stream));
@@ -936,9 +934,7 @@ int clr_launch_norms(clr_ctx *c, int lognormal_fused, double sigma2, int cap, in
     hv.resize(nvals + 2 * ntr);
     h = hv.data();
   }
-  CLR_HIP(c, hipMemcpyAsync(h, fin, nvals * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  CLR_HIP(c, hipMemcpyAsync(h + nvals, work + 2 * nz, 2 * ntr * sizeof(double), hipMemcpyDeviceToHost,
-                            c->stream));
+  CLR_HIP(c, hipMemcpyAsync(h, fin, (nvals + 2 * ntr) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   CLR_HIP(c, hipStreamSynchronize(c->stream));
   for (int t = 0; t < ntr; t++) {
     TracerDev &T = c->tr[tk[t]][tp[t]];

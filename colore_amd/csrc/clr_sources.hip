@@ -42,7 +42,7 @@ constexpr unsigned long long kCountInvalid = ~0ull;
 
 struct PopTab {
   const double *amp, *bz, *norm;
-  const float4 *tab;         // k_pop_table's bins, bound and coarse bounds
+  const float4 *tab;         // k_pop_tables' bins, bound and coarse bounds
   double bz0, norm0, normf;
   int model, ipop;
   uint8_t *cnt8;             // one byte per cell, unset in the blocks whose bytes would all be 0
@@ -107,7 +107,7 @@ __device__ inline float cell_density(const SrcArgs &a, float g, int ix, int iy, 
 constexpr float kBinZero = -1.f, kBinTiny = -2.f, kBinOther = -3.f;
 
 // After the bins and the bound (element na) come the coarse bounds, written
-// by k_pop_coarse: entry j covers the bins [16j, 16j+16), i.e. the nodes
+// by k_pop_tables: entry j covers the bins [16j, 16j+16), i.e. the nodes
 // 16j..16j+16, as (Pmax, bmin, bmax, 0):
 //   Pmax >= n(r) dx^3 norm(r) for the reference's separate FP64 interpolants
 //   of n and norm anywhere in those bins (the largest n times the largest
@@ -119,9 +119,8 @@ constexpr int kCoarse = 16;
 inline int coarse_count(int na) { return (na + kCoarse - 1) / kCoarse; }
 inline size_t pop_table_len(int na) { return (size_t)na + 1 + coarse_count(na); }
 
-__global__ void k_pop_table(const double *__restrict__ amp, const double *__restrict__ bz,
-                            const double *__restrict__ norm, double cv, int na, float4 *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void pop_bin(const double *__restrict__ amp, const double *__restrict__ bz,
+                               const double *__restrict__ norm, double cv, int na, float4 *__restrict__ out, int i) {
   if (i >= na) return;
   const int j = i + 1 < na ? i + 1 : i;
   const double f0 = amp[i], f1 = amp[j], n0 = norm[i], n1 = norm[j], b0 = bz[i], b1 = bz[j];
@@ -148,14 +147,15 @@ __global__ void k_pop_table(const double *__restrict__ amp, const double *__rest
   out[i] = make_float4(kBinOther, 0.f, 0.f, 0.f);
 }
 
-__global__ void k_pop_coarse(const double *__restrict__ amp, const double *__restrict__ bz,
-                             const double *__restrict__ norm, double cv, int na, float4 *__restrict__ out) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ inline void pop_coarse(const double *__restrict__ amp, const double *__restrict__ bz,
+                                  const double *__restrict__ norm, double cv, int na, float4 *__restrict__ out, int j) {
   if (j >= (na + kCoarse - 1) / kCoarse) return;
   const int i0 = j * kCoarse, i1 = min(i0 + kCoarse, na - 1);
   double nmax = 0, mmax = 0, bmin = 1e300, bmax = 0;
   bool ok = true;
-  for (int i = i0; i <= i1; i++) {
+#pragma unroll
+  for (int d = 0; d <= kCoarse; d++) {   // (a node past the last repeats it: all loads in flight together)
+    const int i = min(i0 + d, i1);
     const double n = amp[i], m = norm[i], b = bz[i];
     if (isinf(n)) ok = false;
     else if (n > nmax) nmax = n;
@@ -171,6 +171,37 @@ __global__ void k_pop_coarse(const double *__restrict__ amp, const double *__res
   const double P = nmax * cv * mmax;
   out[na + 1 + j] = ok && P <= 1e30 ? make_float4((float)(P * (1 + 1e-6)), (float)bmin, (float)bmax, 0.f)
                                     : make_float4(INFINITY, -INFINITY, INFINITY, 0.f);
+}
+
+// The tables of every population of a pass (blockIdx.y): bins, then coarse
+// bounds.  k_src_begin has cleared the bounds' elements.  (A launch per
+// population and part, the coarse one looping over its nodes, took 14 us each.)
+struct PopSrc {
+  const double *amp[CLR_NPOP_MAX], *bz[CLR_NPOP_MAX], *norm[CLR_NPOP_MAX];
+  float4 *out[CLR_NPOP_MAX];
+};
+__global__ __launch_bounds__(256) void k_pop_tables(PopSrc s, double cv, int na, int nbin) {
+  const int p = blockIdx.y;
+  if ((int)blockIdx.x < nbin)
+    pop_bin(s.amp[p], s.bz[p], s.norm[p], cv, na, s.out[p], blockIdx.x * 256 + threadIdx.x);
+  else
+    pop_coarse(s.amp[p], s.bz[p], s.norm[p], cv, na, s.out[p], (blockIdx.x - nbin) * 256 + threadIdx.x);
+}
+
+// Clears the lists' counters and the error bounds of npop tables (a kernel
+// rather than memset nodes: graph-safe).
+__global__ void k_src_begin(PopSrc s, int npop, int na, unsigned *__restrict__ esc_n, unsigned *__restrict__ exq_n) {
+  const int t = threadIdx.x;
+  if (t < npop) s.out[t][na] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (t == 0) *esc_n = 0;
+  if (t == 1) *exq_n = 0;
+}
+
+void launch_src_begin(const PopSrc &ps, int npop, int na, double cv, const SrcArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_src_begin, dim3(1), dim3(64), 0, s, ps, npop, na, a.esc_n, a.exq_n);
+  if (npop == 0) return;
+  const int nbin = (na + 255) / 256, nco = (coarse_count(na) + 255) / 256;
+  hipLaunchKernelGGL(k_pop_tables, dim3((unsigned)(nbin + nco), (unsigned)npop), dim3(256), 0, s, ps, cv, na, nbin);
 }
 
 // The reference's FP64 count of cell (ix,iy,iz) (srcs.c:136-187) from the
@@ -481,13 +512,9 @@ __global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(6))) voi
   }
 }
 
-// The FP64 counts of the cells k_count left pending: block totals, bytes and
-// escape entries completed in place (one thread per entry).
-__global__ __launch_bounds__(256) void k_exact(SrcArgs a) {
-  const unsigned j = blockIdx.x * blockDim.x + threadIdx.x;
-  const unsigned n = *a.exq_n;
-  if (j >= n || j >= a.exq_cap) return;
-  const uint4 e = a.exq[j];
+// The FP64 count of a cell k_count left pending: block total, byte and escape
+// entry completed in place.
+__device__ inline void exact_cell(const SrcArgs &a, const uint4 e) {
   const uint64_t cell = (uint64_t)e.x | ((uint64_t)e.y << 32);
   const int ip = (int)e.z;
   const PopTab &P = a.pop[ip];
@@ -517,6 +544,14 @@ __global__ __launch_bounds__(256) void k_exact(SrcArgs a) {
   }
 }
 
+// (a bounded grid: the queue's capacity, which other stages' scratch may have
+// grown, launched 14 us of empty blocks)
+constexpr unsigned kExactBlocks = 1024;
+__global__ __launch_bounds__(256) void k_exact(SrcArgs a) {
+  const unsigned n = min(*a.exq_n, a.exq_cap);
+  for (unsigned j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) exact_cell(a, a.exq[j]);
+}
+
 // exclusive scan of n uint32 -> int64 offsets (out[n] = total), for every
 // population at once (blockIdx.y).  Three kernels: per-block sums, scan of
 // the block sums (one block per population), block-local scan.
@@ -525,7 +560,65 @@ struct ScanPtrs {
   const uint32_t *in[CLR_NPOP_MAX];
   long long *bsum[CLR_NPOP_MAX];
   long long *out[CLR_NPOP_MAX];
+  // when set: the totals of the np populations, then *esc_n and *exq_n, for one copy
+  long long *res;
+  const unsigned *esc_n, *exq_n;
+  int np;
 };
+__device__ inline void scan_result(const ScanPtrs &p, int ip, long long total) {
+  if (!p.res) return;
+  p.res[ip] = total;
+  if (ip == 0) {
+    p.res[p.np] = *p.esc_n;
+    p.res[p.np + 1] = *p.exq_n;
+  }
+}
+
+// Up to kScanOne blocks of cells (192^3) in one kernel: all of a thread's loads
+// in flight, in one block per population.  (The three kernels 13 us.)
+constexpr int kScanOne = 16384;
+__global__ __launch_bounds__(kScanB) void k_scan_one(ScanPtrs p, int n4) {
+  constexpr int C = kScanOne / (4 * kScanB);
+  __shared__ long long ws[C][kScanB / 64];
+  const int ip = blockIdx.y, t = threadIdx.x, lane = t & 63;
+  const uint4 *__restrict__ in = (const uint4 *)p.in[ip];
+  long long *__restrict__ out = p.out[ip];
+  uint4 v[C];
+  long long inc[C];
+#pragma unroll
+  for (int k = 0; k < C; k++) v[k] = k * kScanB + t < n4 ? in[k * kScanB + t] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+  for (int k = 0; k < C; k++) {
+    inc[k] = (long long)v[k].x + v[k].y + v[k].z + v[k].w;
+    for (int o = 1; o < 64; o <<= 1) {
+      const long long x = __shfl_up(inc[k], o);
+      if (lane >= o) inc[k] += x;
+    }
+    if (lane == 63) ws[k][t >> 6] = inc[k];
+  }
+  __syncthreads();
+  long long base = 0;
+#pragma unroll
+  for (int k = 0; k < C; k++) {
+    long long run = base + inc[k] - ((long long)v[k].x + v[k].y + v[k].z + v[k].w);
+    for (int w = 0; w < kScanB / 64; w++) {
+      const long long x = ws[k][w];
+      base += x;
+      if (w < (t >> 6)) run += x;
+    }
+    if (k * kScanB + t < n4) {
+      long long *o = out + 4 * (k * kScanB + t);
+      o[0] = run;
+      o[1] = run += v[k].x;
+      o[2] = run += v[k].y;
+      o[3] = run += v[k].z;
+    }
+  }
+  if (t == 0) {
+    out[4 * n4] = base;
+    scan_result(p, ip, base);
+  }
+}
 __global__ __launch_bounds__(kScanB) void k_scan_blocks(ScanPtrs p, size_t n) {
   __shared__ long long s[kScanB];
   const uint32_t *__restrict__ in = p.in[blockIdx.y];
@@ -560,7 +653,10 @@ __global__ __launch_bounds__(kScanB) void k_scan_top(ScanPtrs p, size_t nb) {
     if (threadIdx.x == kScanB - 1) carry += s[kScanB - 1];
     __syncthreads();
   }
-  if (threadIdx.x == 0) bsum[nb] = carry;
+  if (threadIdx.x == 0) {
+    bsum[nb] = carry;
+    scan_result(p, blockIdx.y, carry);
+  }
 }
 __global__ __launch_bounds__(kScanB) void k_scan_apply(ScanPtrs p, size_t n) {
   __shared__ long long s[kScanB];
@@ -579,6 +675,17 @@ __global__ __launch_bounds__(kScanB) void k_scan_apply(ScanPtrs p, size_t n) {
   }
   if (i < n) out[i] = bsum[blockIdx.x] + s[threadIdx.x] - v;
   if (i == n - 1) out[n] = bsum[gridDim.x];
+}
+
+void launch_scan(const ScanPtrs &sp, int np, size_t n, hipStream_t s) {
+  if (n <= kScanOne && n % 4 == 0) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1, (unsigned)np), dim3(kScanB), 0, s, sp, (int)(n / 4));
+    return;
+  }
+  const size_t nsb = (n + kScanB - 1) / kScanB;
+  hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nsb, (unsigned)np), dim3(kScanB), 0, s, sp, n);
+  hipLaunchKernelGGL(k_scan_top, dim3(1, (unsigned)np), dim3(kScanB), 0, s, sp, nsb);
+  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nsb, (unsigned)np), dim3(kScanB), 0, s, sp, n);
 }
 
 // count of an escaped cell from the sorted escape list
@@ -779,12 +886,6 @@ __global__ __launch_bounds__(256) void k_write(WriteArgs a) {
   }
   a.pos[pid] = make_float4(pp[0], pp[1], pp[2], (float)dz_rsd);
   a.ipix[pid] = a.r2n[vec2pix_ring32(a.nside_base, (double)pp[0], (double)pp[1], (double)pp[2])];
-}
-
-// Zero n 32-bit words (a kernel rather than a memset node: graph-safe).
-__global__ void k_zero_words(uint32_t *__restrict__ p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
 }
 
 // Status of a graph-captured sampling pass: 1 saturated counts (escape list
@@ -1060,16 +1161,14 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
   int rc = clr_ring2nest_table(c, nside_base);
   if (rc) return rc;
   const double dx = c->L / N, cell_vol = dx * dx * dx;
-  // packed FP32 tables, rebuilt from the current norm tables
+  PopSrc ps{};
   for (int i = p0; i < p1; i++) {
     TracerDev &T = c->tr[CLR_TRACER_SRCS][i];
     if (!T.ptab) CLR_HIP(c, hipMalloc((void **)&T.ptab, pop_table_len(na) * sizeof(float4)));
-    CLR_HIP(c, hipMemsetAsync((float4 *)T.ptab + na, 0, sizeof(float4), c->stream));
-    hipLaunchKernelGGL(k_pop_table, dim3((na + 255) / 256), dim3(256), 0, c->stream, T.amp, T.bz, T.norm, cell_vol,
-                       na, (float4 *)T.ptab);
-    hipLaunchKernelGGL(k_pop_coarse, dim3((coarse_count(na) + 255) / 256), dim3(256), 0, c->stream, T.amp, T.bz,
-                       T.norm, cell_vol, na, (float4 *)T.ptab);
-    CLR_HIP(c, hipGetLastError());
+    ps.amp[i - p0] = T.amp;
+    ps.bz[i - p0] = T.bz;
+    ps.norm[i - p0] = T.norm;
+    ps.out[i - p0] = (float4 *)T.ptab;
   }
   const int np = p1 - p0;
   const size_t nblocks = ncells / kBlockCells;
@@ -1077,7 +1176,8 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
   // scratch per population: bytes (ncells), block totals, offsets, scan partials
   // (a multiple of 256 bytes: every population's bytes start aligned)
   const size_t per_pop = (ncells + nblocks * 4 + (nblocks + 1) * 8 + (nsb + 1) * 8 + 64 + 255) / 256 * 256;
-  rc = clr_ensure(c, (void **)&c->rowcnt, &c->rows_n, (size_t)np * per_pop);
+  // (after the last population: the totals and list lengths for the host)
+  rc = clr_ensure(c, (void **)&c->rowcnt, &c->rows_n, (size_t)np * per_pop + (CLR_NPOP_MAX + 2) * sizeof(long long));
   if (rc) return rc;
 
   SrcArgs a{};
@@ -1149,8 +1249,9 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
     a.exq_n = (unsigned int *)c->misc;
     a.exq = (uint4 *)((char *)c->misc + 16);
     a.exq_cap = (unsigned int)((c->misc_n - 16) / 16);
-    CLR_HIP(c, hipMemsetAsync(a.esc_n, 0, sizeof(unsigned int), c->stream));
-    CLR_HIP(c, hipMemsetAsync(a.exq_n, 0, sizeof(unsigned int), c->stream));
+    // packed FP32 tables, rebuilt from the current norm tables
+    launch_src_begin(ps, attempt == 0 ? np : 0, na, cell_vol, a, c->stream);
+    CLR_HIP(c, hipGetLastError());
     CLR_HIP(c, hipEventRecord(c->ev2, c->stream));
     if (fused)
       hipLaunchKernelGGL(k_count<true>, dim3((unsigned)(ncells / kCountCells)), dim3(kLanes),
@@ -1159,7 +1260,7 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
       hipLaunchKernelGGL(k_count<false>, dim3((unsigned)(ncells / kCountCells)), dim3(kLanes),
                          (size_t)np * kLanes * sizeof(uint4), c->stream, a);
     CLR_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_exact, dim3((a.exq_cap + 255) / 256), dim3(256), 0, c->stream, a);
+    hipLaunchKernelGGL(k_exact, dim3(std::min((a.exq_cap + 255) / 256, kExactBlocks)), dim3(256), 0, c->stream, a);
     CLR_HIP(c, hipGetLastError());
     CLR_HIP(c, hipEventRecord(c->ev3, c->stream));
     ScanPtrs sp{};
@@ -1168,17 +1269,18 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
       sp.bsum[i] = bsum[i];
       sp.out[i] = (long long *)a.pop[i].boff;
     }
-    hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nsb, (unsigned)np), dim3(kScanB), 0, c->stream, sp, nblocks);
-    hipLaunchKernelGGL(k_scan_top, dim3(1, (unsigned)np), dim3(kScanB), 0, c->stream, sp, nsb);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nsb, (unsigned)np), dim3(kScanB), 0, c->stream, sp, nblocks);
+    sp.res = (long long *)((char *)c->rowcnt + (size_t)np * per_pop);
+    sp.esc_n = a.esc_n;
+    sp.exq_n = a.exq_n;
+    sp.np = np;
+    launch_scan(sp, np, nblocks, c->stream);
     CLR_HIP(c, hipGetLastError());
-    for (int i = 0; i < np; i++)
-      CLR_HIP(c, hipMemcpyAsync(&tot[i], a.pop[i].boff + nblocks, sizeof(long long), hipMemcpyDeviceToHost,
-                                c->stream));
-    unsigned int nexq = 0;
-    CLR_HIP(c, hipMemcpyAsync(&nesc, a.esc_n, sizeof(unsigned int), hipMemcpyDeviceToHost, c->stream));
-    CLR_HIP(c, hipMemcpyAsync(&nexq, a.exq_n, sizeof(unsigned int), hipMemcpyDeviceToHost, c->stream));
+    long long res[CLR_NPOP_MAX + 2];
+    CLR_HIP(c, hipMemcpyAsync(res, sp.res, (np + 2) * sizeof(long long), hipMemcpyDeviceToHost, c->stream));
     CLR_HIP(c, hipStreamSynchronize(c->stream));
+    for (int i = 0; i < np; i++) tot[i] = res[i];
+    nesc = (unsigned int)res[np];
+    const unsigned int nexq = (unsigned int)res[np + 1];
     if (nesc <= a.esc_cap && nexq <= a.exq_cap) break;
     if (attempt == 1) return clr_fail(c, CLR_ERR_STATE, "source lists overflow (%u, %u entries)", nesc, nexq);
     if (nesc > a.esc_cap) {
@@ -1419,9 +1521,7 @@ int clr_launch_sources_stream(clr_ctx *c, int ipop, int nthr, const int *iz_begi
     sp.in[0] = a.cnt;
     sp.bsum[0] = bsum;
     sp.out[0] = off;
-    hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nsb, 1), dim3(kScanB), 0, c->stream, sp, ncells);
-    hipLaunchKernelGGL(k_scan_top, dim3(1, 1), dim3(kScanB), 0, c->stream, sp, nsb);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nsb, 1), dim3(kScanB), 0, c->stream, sp, ncells);
+    launch_scan(sp, 1, ncells, c->stream);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpyAsync(&total, off + ncells, sizeof(long long), hipMemcpyDeviceToHost, c->stream);
@@ -1543,7 +1643,7 @@ int clr_prepare_sources(clr_ctx *c, int nside_base, const long long *cap) {
 int clr_enqueue_sources(clr_ctx *c, hipStream_t st, uint32_t seed, int nside_base, int *flag_dev) {
   const int np = c->n_tr[CLR_TRACER_SRCS], N = c->N, na = c->na;
   const size_t ncells = (size_t)N * N * N, per_pop = src_per_pop(ncells);
-  const size_t nblocks = ncells / kBlockCells, nsb = (nblocks + kScanB - 1) / kScanB;
+  const size_t nblocks = ncells / kBlockCells;
   if (c->rows_n < (size_t)np * per_pop || !c->esc || c->misc_n < 16 + 16 * 4096 || c->r2n_nside != nside_base)
     return clr_fail(c, CLR_ERR_STATE, "sampling buffers not prepared");
   const double dx = c->L / N, cell_vol = dx * dx * dx;
@@ -1573,6 +1673,7 @@ int clr_enqueue_sources(clr_ctx *c, hipStream_t st, uint32_t seed, int nside_bas
   a.exq_cap = (unsigned int)((c->misc_n - 16) / 16);
   std::vector<long long *> bsum(np);
   GraphTotals gt{};
+  PopSrc ps{};
   for (int i = 0; i < np; i++) {
     TracerDev &T = c->tr[CLR_TRACER_SRCS][i];
     CatalogDev &C = c->cat[i];
@@ -1598,27 +1699,23 @@ int clr_enqueue_sources(clr_ctx *c, hipStream_t st, uint32_t seed, int nside_bas
     P.desc = (uint4 *)C.pos;
     gt.tot[i] = off + nblocks;
     gt.cap[i] = C.cap;
-    // packed tables from the current norm tables
-    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, st, (uint32_t *)((float4 *)T.ptab + na), 4);
-    hipLaunchKernelGGL(k_pop_table, dim3((na + 255) / 256), dim3(256), 0, st, T.amp, T.bz, T.norm, cell_vol, na,
-                       (float4 *)T.ptab);
-    hipLaunchKernelGGL(k_pop_coarse, dim3((coarse_count(na) + 255) / 256), dim3(256), 0, st, T.amp, T.bz, T.norm,
-                       cell_vol, na, (float4 *)T.ptab);
+    ps.amp[i] = T.amp;
+    ps.bz[i] = T.bz;
+    ps.norm[i] = T.norm;
+    ps.out[i] = (float4 *)T.ptab;
   }
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, st, (uint32_t *)a.esc_n, 1);
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, st, (uint32_t *)a.exq_n, 1);
+  // packed tables from the current norm tables
+  launch_src_begin(ps, np, na, cell_vol, a, st);
   hipLaunchKernelGGL(k_count<false>, dim3((unsigned)(ncells / kCountCells)), dim3(kLanes),
                      (size_t)np * kLanes * sizeof(uint4), st, a);
-  hipLaunchKernelGGL(k_exact, dim3((a.exq_cap + 255) / 256), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_exact, dim3(std::min((a.exq_cap + 255) / 256, kExactBlocks)), dim3(256), 0, st, a);
   ScanPtrs sp{};
   for (int i = 0; i < np; i++) {
     sp.in[i] = a.pop[i].btot;
     sp.bsum[i] = bsum[i];
     sp.out[i] = (long long *)a.pop[i].boff;
   }
-  hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nsb, (unsigned)np), dim3(kScanB), 0, st, sp, nblocks);
-  hipLaunchKernelGGL(k_scan_top, dim3(1, (unsigned)np), dim3(kScanB), 0, st, sp, nsb);
-  hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nsb, (unsigned)np), dim3(kScanB), 0, st, sp, nblocks);
+  launch_scan(sp, np, nblocks, st);
   hipLaunchKernelGGL(k_graph_flags, dim3(1), dim3(64), 0, st, (const unsigned *)a.esc_n,
                      (const unsigned *)a.exq_n, a.exq_cap, np, gt, flag_dev);
   hipLaunchKernelGGL(k_fill, dim3((unsigned)(ncells / (kFillWaves * kCountCells))), dim3(kFillWaves * kLanes), 0, st, a);

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("N,scales", [
     (32, (1.0, 1e-2, 1e-4, 3e-6)),
     (64, (1.0, 1e-3, 1e-5, 1e-2)),
-    (192, (0.3, 1e-4, 1e-6)),
+    (192, (0.3, 1e-4, 1e-6)),   # the most blocks of the one-kernel scan
+    (256, (1e-2, 1e-6)),        # three scan kernels
 ])
 def test_dense_then_sparse(workdir, N, scales):
     from colore_amd import lib
