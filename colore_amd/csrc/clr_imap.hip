@@ -37,84 +37,86 @@ struct ImapArgs {
 };
 
 // Sub-point arithmetic.  The reference's chain for a sub-point (cart2sph,
-// imap.c:24-41, then he_ang2pix) costs three FP64 divisions, an FP64 atan2
-// and the pixel's floors.  pixel_fast evaluates the same chain with one
-// division (cos theta = z/r, exact as the reference takes it) and an
-// approximate azimuth -- atan of min/max by the Abramowitz & Stegun 4.4.49
-// polynomial (Hastings; |error| <= 2e-8 rad on [0, 1]) -- and accepts its
-// result only when every floor it takes is certain: the value lies further
-// than the azimuth's error bound (carried through each product) from an
-// integer.  Otherwise, and on the z axis or within the bound of phi = 0
-// (where the reference's wrap to [0, 2pi) could differ), the exact chain
-// runs.  The accepted pixel is therefore the exact chain's pixel.
+// imap.c:24-41, then he_ang2pix) costs an FP64 square root, three divisions, an
+// FP64 atan2 and the pixel's floors.  The fast path evaluates the same chain
+// from one reciprocal square root (hardware, 2^-24 relative, and a Newton step:
+// 1e-14) and an approximate azimuth -- atan of min/max by the Abramowitz &
+// Stegun 4.4.49 polynomial (Hastings; |error| <= 2e-8 rad on [0, 1]) -- and
+// accepts its shell and pixel only when every comparison and floor it takes is
+// certain: the value lies further than its error bound (carried through each
+// product) from the edge or integer.  Otherwise, and near the z axis or within
+// the bound of phi = 0 (where the reference's wrap to [0, 2pi) could differ),
+// the exact chain runs.  The accepted shell and pixel are therefore the exact
+// chain's.  k_imap and k_imap_wave are bound by these vector instructions.
 constexpr double kAtanErr = 2e-8;   // A&S 4.4.49 bound; the polynomial's measured maximum is 1.36e-8
 
 __device__ inline double atan01(double t) {
-#pragma clang fp contract(off)
   const double t2 = t * t;
   double p = 0.0028662257;
-  p = p * t2 - 0.0161657367;
-  p = p * t2 + 0.0429096138;
-  p = p * t2 - 0.0752896400;
-  p = p * t2 + 0.1065626393;
-  p = p * t2 - 0.1420889944;
-  p = p * t2 + 0.1999355085;
-  p = p * t2 - 0.3333314528;
-  p = p * t2 + 1.0;
+  p = fma(p, t2, -0.0161657367);
+  p = fma(p, t2, 0.0429096138);
+  p = fma(p, t2, -0.0752896400);
+  p = fma(p, t2, 0.1065626393);
+  p = fma(p, t2, -0.1420889944);
+  p = fma(p, t2, 0.1999355085);
+  p = fma(p, t2, -0.3333314528);
+  p = fma(p, t2, 1.0);
   return t * p;
 }
 
-// floor(v) when [v - e, v + e] holds no integer and v - e >= 0, else -1
-__device__ inline int certain_floor(double v, double e) {
-  const double lo = floor(v - e);
-  return (lo >= 0 && lo == floor(v + e)) ? (int)lo : -1;
+// 1/sqrt(v) to 1e-14
+__device__ inline double rsqrt_1e14(double v) {
+  const double q = __builtin_amdgcn_rsq(v);
+  const double e = fma(-v * q, q, 1.0);
+  return fma(0.5 * q, e, q);
 }
 
-// RING pixel of the sub-point (x, y, z) with cth = z / r (r > 0) as the
-// reference's chain gives it, or -1 when a floor is too close to call.
-// nside is a power of two.
+// (int)v, v >= 0 but for its error; ok stays set when no integer lies within e
+__device__ inline int certain_floor(double v, double e, bool &ok) {
+  ok = ok && fabs(__builtin_amdgcn_fract(v) - 0.5) < 0.5 - e;
+  return (int)v;
+}
+
+// RING pixel of the sub-point (x, y, z) with cth = z / r (r > 0) to 1e-14, or
+// -1 when a floor is too close to call.  nside is a power of two.
 __device__ inline int pixel_fast(int nside, double x, double y, double cth) {
-#pragma clang fp contract(off)
-  const double ax = fabs(x), ay = fabs(y);
-  const double mx = fmax(ax, ay), mn = fmin(ax, ay);
-  if (!(mx > 0)) return -1;
-  // the ratio through the hardware reciprocal and two Newton steps (a few
-  // ulp; the exact quotient is not needed: the error stays far inside the
-  // margin the floors are certified with)
+  const bool swap = fabs(y) > fabs(x);
+  const double mx = fmax(fabs(x), fabs(y)), mn = fmin(fabs(x), fabs(y));
   double rm = __builtin_amdgcn_rcp(mx);
-  rm = rm * (2.0 - mx * rm);
-  rm = rm * (2.0 - mx * rm);
-  double a = atan01(mn * rm);
-  if (ay > ax) a = 1.5707963267948966 - a;
-  if (x < 0) a = 3.141592653589793 - a;
-  if (y < 0) a = -a;
-  // |a - atan2(y/r, x/r)| <= kAtanErr + 1e-14 (the reference's own roundings
-  // and the constants' included)
-  if (fabs(a) <= 4 * kAtanErr) return -1;
-  const double ph = a < 0 ? a + 6.283185307179586 : a;
-  const double tt = ph * 0.6366197723675814;
-  const double ett = 0.6366197723675814 * (kAtanErr + 1e-14) + 1e-13;   // bound on |tt - tt_ref|
-  const double dn = (double)nside;
-  if (fabs(cth) <= 2.0 / 3.0) {
-    const double t1 = dn * (0.5 + tt), t2 = dn * cth * 0.75;
-    const double e = dn * ett + 1e-10;
-    const int jp = certain_floor(t1 - t2, e), jm = certain_floor(t1 + t2, e);
-    if (jp < 0 || jm < 0) return -1;
+  rm = fma(rm, fma(-mx, rm, 1.0), rm);
+  const double t = mn * rm;
+  // the azimuth in quarter turns, c + s (2/pi) atan(t) by octant
+  const uint32_t xh = (uint32_t)__double2hiint(x), yh = (uint32_t)__double2hiint(y);
+  const double at = atan01(t);
+  const uint32_t sg = ((xh ^ yh) ^ (swap ? 0x80000000u : 0u)) & 0x80000000u;
+  const double sa = __hiloint2double((int)((uint32_t)__double2hiint(at) ^ sg), __double2loint(at));
+  const double c = swap ? (y < 0 ? 3.0 : 1.0) : (x < 0 ? 2.0 : (y < 0 ? 4.0 : 0.0));
+  const double tt = fma(sa, 0.6366197723675814, c);
+  const double ett = 0.6366197723675814 * (kAtanErr + 1e-13) + 1e-13;   // bound on |tt - tt_ref|
+  const double dn = (double)nside, az = fabs(cth);
+  // (phi near 0 or pi, and the edge of the polar caps, where the two forms differ)
+  bool ok = (swap || t > 1e-7) && fabs(az - 2.0 / 3.0) > 1e-12;
+  if (az <= 2.0 / 3.0) {
+    const double t1 = fma(dn, tt, 0.5 * dn), t2 = dn * 0.75 * cth;
+    const double e = fma(dn, ett, 1e-10);
+    const int jp = certain_floor(t1 - t2, e, ok), jm = certain_floor(t1 + t2, e, ok);
+    if (!ok) return -1;
     const int ir = nside + 1 + jp - jm;
     const int kshift = 1 - (ir & 1);
     const int ip = ((jp + jm - nside + kshift + 1) / 2) & (4 * nside - 1);
     return nside * (nside - 1) * 2 + (ir - 1) * 4 * nside + ip;
   }
-  const int k = certain_floor(tt, ett);
-  if (k < 0) return -1;
+  const int k = certain_floor(tt, ett, ok);
   const double tp = tt - k;
-  const double tmp = dn * sqrt(3 * (1 - fabs(cth)));
-  const int jp = certain_floor(tp * tmp, tmp * ett + 1e-10);
-  const int jm = certain_floor((1.0 - tp) * tmp, tmp * (ett + 1e-15) + 1e-10);
-  if (jp < 0 || jm < 0) return -1;
+  const double q = 3 * (1 - az);
+  // sqrt(q) >= 1e-3 carries at most 3e-11 of cth's error
+  ok = ok && q > 1e-6;
+  const double tmp = dn * (q * rsqrt_1e14(q));
+  const double e = fma(tmp, ett + 1e-13, fma(dn, 1e-10, 1e-10));
+  const int jp = certain_floor(tp * tmp, e, ok), jm = certain_floor((1.0 - tp) * tmp, e, ok);
   const int ir = jp + jm + 1;
-  int ip = certain_floor(tt * ir, ir * ett + 1e-10);
-  if (ip < 0) return -1;
+  int ip = certain_floor(tt * ir, fma((double)ir, ett, 1e-10), ok);
+  if (!ok) return -1;
   if (ip >= 4 * ir) ip -= 4 * ir;
   if (cth > 0) return 2 * ir * (ir - 1) + ip;
   return 12 * nside * nside - 2 * ir * (ir + 1) + ip;
@@ -169,13 +171,14 @@ __device__ inline double rvel_cell(const ImapArgs &a, int ix, int iy, int iz, do
 // and the RSD shift v_r V1(r)/H(r) (imap.c:185-200), and the sub-sampling
 // nsub of its shell (imap.c:201-209).  false when the cell is outside the
 // shells' range or has T(r) = 0.
-// The shells its sub-points can reach: their shifted radii lie in [rlo, rhi]
-// (the cube's centre radius +- half its diagonal, plus the cell's shift),
-// and when no shell edge but r0[wi0 + 1] lies inside (wok), a sub-point's
-// shell is wi0 or wi0 + 1 by one comparison (wf0, wf1: their rf).
+// The shells its sub-points can reach: their shifted radii lie within the
+// cube's centre radius +- half its diagonal, plus the cell's shift, and when
+// no shell edge but wb = r0[wi0 + 1] lies inside (wok), a sub-point's shell is
+// wi0 or wi0 + 1 by one comparison, if below the shell's end (wf0, wf1: its rf,
+// at most the last shell's).  m: the margin of these comparisons.
 struct CellPaint {
   double x0, y0, z0, dr_rsd, dxs;
-  double rlo, rhi, wb, wf0, wf1;
+  double m, wb, wf0, wf1;
   float temp;
   int ns, wi0;
   bool wok;
@@ -222,30 +225,20 @@ __device__ inline bool cell_paint(const ImapArgs &a, const double *__restrict__ 
     const double xc = x0 + 0.5 * a.dx, yc = y0 + 0.5 * a.dx, zc = z0 + 0.5 * a.dx;
     const double rc = sqrt(xc * xc + yc * yc + zc * zc), hd = 0.8660254038 * a.dx;
     const double m = 1e-9 * (rc + hd + fabs(cp.dr_rsd)) + 1e-9;
-    cp.rlo = rc - hd + cp.dr_rsd - m;
-    cp.rhi = rc + hd + cp.dr_rsd + m;
+    const double rlo = rc - hd + cp.dr_rsd - m, rhi = rc + hd + cp.dr_rsd + m;
+    cp.m = 1e-2 * m;
     int lo = -1, hi = a.nr - 1;   // largest i with r0[i] <= rlo, or -1
     while (hi > lo) {
       const int mid = (lo + hi + 1) / 2;
-      if (r0s[mid] <= cp.rlo) lo = mid; else hi = mid - 1;
+      if (r0s[mid] <= rlo) lo = mid; else hi = mid - 1;
     }
     cp.wi0 = lo;
     cp.wb = lo + 1 < a.nr ? r0s[lo + 1] : INFINITY;
-    cp.wf0 = lo >= 0 ? rfs[lo] : 0.0;
-    cp.wf1 = lo + 1 < a.nr ? rfs[lo + 1] : 0.0;
-    cp.wok = lo + 2 >= a.nr || cp.rhi < r0s[lo + 2];
+    cp.wf0 = lo >= 0 ? fmin(rfs[lo], a.rf_last) : -INFINITY;
+    cp.wf1 = lo + 1 < a.nr ? fmin(rfs[lo + 1], a.rf_last) : -INFINITY;
+    cp.wok = lo + 2 >= a.nr || rhi < r0s[lo + 2];
   }
   return true;
-}
-
-// shell_of for a sub-point of the cell (the same index)
-__device__ inline int shell_near(const ImapArgs &a, const double *__restrict__ r0s, const double *__restrict__ rfs,
-                                 const CellPaint &cp, double rs) {
-  if (!(cp.wok && rs >= cp.rlo && rs <= cp.rhi)) return shell_of(r0s, rfs, a.nr, rs);
-  const int i = rs >= cp.wb ? cp.wi0 + 1 : cp.wi0;
-  if (i < 0) return -1;
-  if (rs >= a.rf_last) return a.nr;
-  return rs < (i == cp.wi0 ? cp.wf0 : cp.wf1) ? i : -2;
 }
 
 // The shell (or < 0 outside the shells) and RING pixel of sub-point
@@ -257,12 +250,24 @@ __device__ inline int subpoint_shell_pixel(const ImapArgs &a, const double *__re
   const double z = cp.z0 + (izz + 0.5) * cp.dxs;
   const double y = cp.y0 + (iyy + 0.5) * cp.dxs;
   const double x = cp.x0 + (ixx + 0.5) * cp.dxs;
+  {
+    const double r2 = fma(x, x, fma(y, y, z * z)), q = rsqrt_1e14(r2);
+    const double rs = fma(r2, q, cp.dr_rsd);
+    const bool up = rs >= cp.wb;
+    const double end = up ? cp.wf1 : cp.wf0;
+    if (cp.wok && fabs(rs - cp.wb) > cp.m && fabs(rs - end) > cp.m) {
+      if (!(rs < end)) return -1;
+      const int p = pixel_fast((int)a.nside, x, y, z * q);
+      if (p >= 0) {
+        pix = p;
+        return up ? cp.wi0 + 1 : cp.wi0;
+      }
+    }
+  }
   const double r = sqrt(x * x + y * y + z * z);
-  const int irad = shell_near(a, r0s, rfs, cp, r + cp.dr_rsd);
+  const int irad = shell_of(r0s, rfs, a.nr, r + cp.dr_rsd);
   if (irad < 0 || irad >= a.nr) return -1;
-  pix = -1;
-  if (r != 0) pix = pixel_fast((int)a.nside, x, y, z / r);
-  if (pix < 0) pix = pixel_exact(a.nside, x, y, z, r);
+  pix = pixel_exact(a.nside, x, y, z, r);
   return irad;
 }
 
@@ -492,11 +497,13 @@ __global__ __launch_bounds__(64 * kImapWaves) void k_imap_wave(ImapArgs a, const
     CellPaint cp;
     if (!cell_paint(a, r0s, rfs, nsub, ix, iy, iz, cp)) continue;
     if (cp.ns <= kThreadSub) continue;   // k_imap's cell
-    const int ns = cp.ns, nq = ns * ns * ns;
+    // (the cell is the wavefront's: its sub-point grid in scalar arithmetic,
+    // the lane's indices advanced by 64 with carries)
+    const int ns = __builtin_amdgcn_readfirstlane(cp.ns), nq = ns * ns * ns;
+    const int sx = 64 % ns, sy = (64 / ns) % ns, sz = 64 / (ns * ns);
+    int ixx = lane % ns, iyy = (lane / ns) % ns, izz = lane / (ns * ns);
     for (int q0 = 0; q0 < nq; q0 += 64) {
-      const int q = q0 + lane;
-      if (q < nq) {
-        const int ixx = q % ns, iyy = (q / ns) % ns, izz = q / (ns * ns);
+      if (q0 + lane < nq) {
         int64_t pix;
         const int s = subpoint_shell_pixel(a, r0s, rfs, cp, izz, iyy, ixx, pix);
         if (s >= 0) {
@@ -512,6 +519,11 @@ __global__ __launch_bounds__(64 * kImapWaves) void k_imap_wave(ImapArgs a, const
           }
         }
       }
+      ixx += sx;
+      iyy += sy;
+      izz += sz;
+      if (ixx >= ns) { ixx -= ns; iyy++; }
+      if (iyy >= ns) { iyy -= ns; izz++; }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       __builtin_amdgcn_wave_barrier();
       if (__hip_atomic_load(&b.nused, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) > kWaveFill)
