@@ -131,7 +131,7 @@ struct clr_ctx {
   size_t velrec_n = 0;
   void *lpt_ws = nullptr;    // clr_lpt_density's grids (clr_lpt.hip)
   size_t lpt_ws_n = 0;
-  void *beam_ws = nullptr;   // clr_source_beams' tables, order and results (clr_los.hip)
+  void *beam_ws = nullptr;   // source beams' tables, order and results, skewers' staging (clr_los.hip)
   size_t beam_ws_n = 0;
   std::string los_plan;
   void *los_buf = nullptr;

@@ -1111,11 +1111,13 @@ int clr_launch_src_skewers(clr_ctx *c, int ipop, int gaussian, double sigma2, fl
   a.d1_arr = c->bg + 2 * (size_t)na;
   a.v1_arr = c->bg + 3 * (size_t)na;
   a.vrec = clr_cell_records(c, false) ? (const float4 *)c->velrec : nullptr;
-  // sources per launch: at most 2^26 skewer values (512 MiB of staging)
+  // sources per launch: at most 2^26 skewer values (512 MiB of staging, kept in
+  // the source passes' buffer: allocating and freeing it took as long as the kernel)
   const long long chunk = std::max(1LL, (1LL << 26) / a.nr);
   const long long cap = std::min(n, chunk);
-  float *tmp = nullptr;
-  CLR_HIP(c, hipMalloc((void **)&tmp, (size_t)cap * a.nr * 2 * sizeof(float)));
+  const int wrc = clr_ensure(c, &c->beam_ws, &c->beam_ws_n, (size_t)cap * a.nr * 2 * sizeof(float));
+  if (wrc) return wrc;
+  float *tmp = (float *)c->beam_ws;
   hipError_t e = hipEventRecord(c->ev0, c->stream);
   float kms = 0;
   for (long long s0 = 0; s0 < n && e == hipSuccess; s0 += cap) {
@@ -1147,7 +1149,6 @@ int clr_launch_src_skewers(clr_ctx *c, int ipop, int gaussian, double sigma2, fl
   c->stage_ms[ST_SKW] = kms;
   if (e == hipSuccess) e = hipEventRecord(c->ev1, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  (void)hipFree(tmp);
   if (e != hipSuccess) return clr_fail(c, CLR_ERR_HIP, "source skewers: %s", hipGetErrorString(e));
   return CLR_OK;
 }
