@@ -588,7 +588,11 @@ constexpr int kDirG = 64;
 // 1.07 -> 1.08.  16 sources per bin (64: 2.07 ms; bins of 4 shells of distance
 // in 4 times wider cells, 2.08).
 constexpr int kDirMinN = 256;
-constexpr long long kDirMin = 32768, kDirPer = 16;
+// Skewers, whose every step of a source is a gather of its own, pay the order's
+// 20 us back from fewer sources on: with it 189k sources at 512^3 1.41 -> 0.90
+// ms, 29k at 384^3 184 -> 152 us, at 256^3 90 -> 83, at 192^3 57 -> 62; 5k at
+// 384^3 51 -> 66.
+constexpr long long kDirMin = 32768, kDirMinSkw = 24576, kDirPer = 16;
 constexpr size_t kBeamKeep = (size_t)1 << 30;
 
 __device__ inline uint32_t spread(uint32_t v) {
@@ -663,6 +667,23 @@ __global__ __launch_bounds__(256) void k_dir_place(const uint2 *__restrict__ kr,
   if (i >= n) return;
   const uint2 e = kr[i];
   perm[off[e.x] + e.y] = i;
+}
+
+// Bins' grid for n sources, and the order itself: cnt[dir_bins(G)] and kr[n]
+// are scratch, perm[n] the result.
+inline int dir_grid(long long n) {
+  int G = 1;
+  while (G < kDirG && 24ll * G * G * kDirPer <= n) G *= 2;
+  return G;
+}
+inline int dir_bins(int G) { return (6 * G * G + 3) / 4 * 4; }
+void launch_order(const float4 *pos, long long n, int G, uint32_t *cnt, uint2 *kr, uint32_t *perm, hipStream_t s) {
+  const int nb = dir_bins(G);
+  const unsigned g = (unsigned)((n + 255) / 256);
+  hipLaunchKernelGGL(k_dir_zero, dim3((nb + 255) / 256), dim3(256), 0, s, cnt, nb);
+  hipLaunchKernelGGL(k_dir_count, dim3(g), dim3(256), 0, s, pos, (uint32_t)n, G, cnt, kr);
+  hipLaunchKernelGGL(k_dir_scan, dim3(1), dim3(1024), 0, s, (uint4 *)cnt, nb / 4);
+  hipLaunchKernelGGL(k_dir_place, dim3(g), dim3(256), 0, s, kr, (uint32_t)n, cnt, perm);
 }
 
 // A thread takes every 2^lg-th step of a source.  The projections of the
@@ -864,9 +885,7 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
   // the tables, the order of the marches and the results: in a buffer that the
   // context keeps up to kBeamKeep bytes, else in one of this call
   bool order = lens && N >= kDirMinN && n >= kDirMin && n < (1ll << 31);
-  int G = 1;
-  while (G < kDirG && 24ll * G * G * kDirPer <= n) G *= 2;
-  const int nb = (6 * G * G + 3) / 4 * 4;
+  const int G = dir_grid(n), nb = dir_bins(G);
   struct Own {
     void *p = nullptr;
     ~Own() {
@@ -931,11 +950,7 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
   const unsigned nblk = (unsigned)((((n << a.lg) + 255) / 256 + 7) / 8 * 8);
   const dim3 grid(nblk);
   if (order) {
-    const unsigned g1 = (unsigned)((n + 255) / 256);
-    hipLaunchKernelGGL(k_dir_zero, dim3((nb + 255) / 256), dim3(256), 0, c->stream, cnt, nb);
-    hipLaunchKernelGGL(k_dir_count, dim3(g1), dim3(256), 0, c->stream, pos, (uint32_t)n, G, cnt, kr);
-    hipLaunchKernelGGL(k_dir_scan, dim3(1), dim3(1024), 0, c->stream, (uint4 *)cnt, nb / 4);
-    hipLaunchKernelGGL(k_dir_place, dim3(g1), dim3(256), 0, c->stream, kr, (uint32_t)n, cnt, perm);
+    launch_order(pos, n, G, cnt, kr, perm, c->stream);
   } else {
     perm = nullptr;
   }
@@ -985,7 +1000,8 @@ struct SkwArgs {
 };
 
 // A block computes 16 steps of 16 consecutive sources (lane = step + 16 x
-// source): neighbouring sources lie in neighbouring cells, so their lines of
+// source), in order of direction (perm) or of the catalogue: neighbouring
+// sources lie in neighbouring directions or cells, so their lines of
 // sight cross nearly the same cells at the same step and share the CIC
 // corners' cache lines, where one thread per (source, step) in row order
 // fetched ~170 bytes of HBM per value.  The blocks of one group of sources
@@ -994,14 +1010,16 @@ struct SkwArgs {
 // (b % 8) (gridDim.x / 8) + b / 8, gridDim.x a multiple of 8.  nr is a
 // multiple of 16.
 template <bool REC>
-__global__ __launch_bounds__(256) void k_src_skewers(SkwArgs a, const float4 *__restrict__ pos, long long n,
+__global__ __launch_bounds__(256) void k_src_skewers(SkwArgs a, const float4 *__restrict__ pos,
+                                                     const uint32_t *__restrict__ perm, long long n,
                                                      float *__restrict__ dg, float *__restrict__ vs) {
 #pragma clang fp contract(off)
   const long long blk = (long long)(blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
   const int ntile = a.nr / 16;
-  const long long i = (blk / ntile) * 16 + threadIdx.x / 16;
+  const long long j = (blk / ntile) * 16 + threadIdx.x / 16;
   const int i_r = (int)(blk % ntile) * 16 + (int)(threadIdx.x % 16);
-  if (i >= n) return;
+  if (j >= n) return;
+  const long long i = perm ? (long long)perm[j] : j;
   const long long t = i * a.nr + i_r;
   const float4 p = pos[i];
   const int N = a.N;
@@ -1115,9 +1133,15 @@ int clr_launch_src_skewers(clr_ctx *c, int ipop, int gaussian, double sigma2, fl
   // the source passes' buffer: allocating and freeing it took as long as the kernel)
   const long long chunk = std::max(1LL, (1LL << 26) / a.nr);
   const long long cap = std::min(n, chunk);
-  const int wrc = clr_ensure(c, &c->beam_ws, &c->beam_ws_n, (size_t)cap * a.nr * 2 * sizeof(float));
+  const bool order = N >= kDirMinN && cap >= kDirMinSkw;
+  const int G = dir_grid(cap), nb = dir_bins(G);
+  const size_t obytes = order ? ((size_t)nb * 4 + (size_t)cap * 12 + 15) / 16 * 16 : 0;
+  const int wrc = clr_ensure(c, &c->beam_ws, &c->beam_ws_n, obytes + (size_t)cap * a.nr * 2 * sizeof(float));
   if (wrc) return wrc;
-  float *tmp = (float *)c->beam_ws;
+  uint32_t *cnt = (uint32_t *)c->beam_ws;
+  uint2 *kr = (uint2 *)(cnt + nb);
+  uint32_t *perm = order ? (uint32_t *)(kr + cap) : nullptr;
+  float *tmp = (float *)((char *)c->beam_ws + obytes);
   hipError_t e = hipEventRecord(c->ev0, c->stream);
   float kms = 0;
   for (long long s0 = 0; s0 < n && e == hipSuccess; s0 += cap) {
@@ -1128,12 +1152,13 @@ int clr_launch_src_skewers(clr_ctx *c, int ipop, int gaussian, double sigma2, fl
     const unsigned nblk = (unsigned)(((m + 15) / 16 * (a.nr / 16) + 7) / 8 * 8);
     e = hipEventRecord(c->ev2, c->stream);
     if (e == hipSuccess) {
+      if (order) launch_order((const float4 *)C.pos + s0, m, G, cnt, kr, perm, c->stream);
       if (a.vrec)
         hipLaunchKernelGGL(k_src_skewers<true>, dim3(nblk), dim3(256), 0, c->stream, a,
-                           (const float4 *)C.pos + s0, m, tmp, tmp + (size_t)cap * a.nr);
+                           (const float4 *)C.pos + s0, perm, m, tmp, tmp + (size_t)cap * a.nr);
       else
         hipLaunchKernelGGL(k_src_skewers<false>, dim3(nblk), dim3(256), 0, c->stream, a,
-                           (const float4 *)C.pos + s0, m, tmp, tmp + (size_t)cap * a.nr);
+                           (const float4 *)C.pos + s0, perm, m, tmp, tmp + (size_t)cap * a.nr);
     }
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(c->ev3, c->stream);
