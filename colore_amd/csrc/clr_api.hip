@@ -53,6 +53,22 @@ int clr_phi_ready(clr_ctx *c, int host) {
   return CLR_OK;
 }
 
+void clr_captured_state(const clr_ctx *c, std::string &out) {
+  auto put = [&out](auto v) { out.append((const char *)&v, sizeof v); };
+  for (const void *p : {(const void *)c->bg, (const void *)c->d1f, (const void *)c->pk, (const void *)c->amp,
+                        (const void *)c->red, (const void *)c->red_out, (const void *)c->rowcnt, (const void *)c->esc,
+                        (const void *)c->misc, (const void *)c->r2n, (const void *)c->los_buf})
+    put(p);
+  for (size_t n : {c->red_n, c->rows_n, c->esc_bytes, c->misc_n, c->los_buf_n}) put(n);
+  for (const CatalogDev &C : c->cat) {
+    put(C.pos);
+    put(C.ipix);
+    put(C.cap);
+  }
+  put(c->r2n_nside);
+  out += c->los_plan;
+}
+
 int clr_ring2nest_table(clr_ctx *c, int nside) {
   if (c->r2n && c->r2n_nside == nside) return CLR_OK;
   const int64_t npix = 12LL * nside * nside;

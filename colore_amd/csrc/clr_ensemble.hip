@@ -6,7 +6,8 @@
 // (srcs.c:120-283) and a kappa map (kappa.c:78-175), as kernel launches only
 // (no allocation, no memset node, no host wait inside the graph).  The graph
 // is captured once per seed set, instantiated, and replayed by every later
-// clr_ensemble_run with the same seeds; realisations are spread round-robin
+// clr_ensemble_run with the same seeds while the contexts' buffers stay where
+// they are; realisations are spread round-robin
 // over `nstreams` captured streams, so independent realisations overlap on
 // the device.  Each realisation's results equal a single-context run of the
 // same stages bit for bit (same kernels, same reductions).
@@ -21,6 +22,8 @@ struct clr_ensemble {
   std::vector<clr_ctx *> ctx;
   int nside_base = 2, nside_kappa = 0;
   std::vector<double> r_kappa;
+  std::vector<long long> src_cap;
+  std::string held;   // the contexts' buffers that the graph holds (clr_captured_state)
   hipStream_t origin = nullptr;
   std::vector<hipStream_t> streams;
   std::vector<hipEvent_t> ev_join;
@@ -61,6 +64,27 @@ void drop_graph(clr_ensemble *e) {
   e->exec = nullptr;
   e->graph = nullptr;
   e->seeds.clear();
+}
+
+// Realisation i's buffers (also its context's again, after single calls on it
+// have replaced some).
+int prepare(clr_ensemble *e, int i) {
+  clr_ctx *c = e->ctx[i];
+  int rc = clr_phi_ready(c, 1);
+  if (!rc) rc = clr_prepare_fields(c);
+  if (!rc) rc = clr_prepare_norms(c);
+  if (!rc) {
+    std::vector<long long> cap(c->n_tr[CLR_TRACER_SRCS], e->src_cap[i]);
+    rc = clr_prepare_sources(c, e->nside_base, cap.data());
+  }
+  if (!rc && e->nside_kappa > 0) rc = clr_prepare_kappa(c, e->nside_kappa, 1, &e->r_kappa[i]);
+  return rc ? ens_fail(e, rc, "realisation " + std::to_string(i) + ": " + c->err) : CLR_OK;
+}
+
+std::string captured_state(const clr_ensemble *e) {
+  std::string s;
+  for (const clr_ctx *c : e->ctx) clr_captured_state(c, s);
+  return s;
 }
 
 int capture(clr_ensemble *e) {
@@ -119,17 +143,11 @@ int clr_ensemble_create(clr_ensemble **out, int n, clr_ctx *const *ctxs, int nsi
     if (!c || c->device != e->device) return ens_fail(e, CLR_ERR_ARG, "every context must be on the same device");
     if (!c->tables_set || c->n_tr[CLR_TRACER_SRCS] < 1)
       return ens_fail(e, CLR_ERR_STATE, "realisation " + std::to_string(i) + " has no tables or populations");
-    int rc = clr_phi_ready(c, 1);
-    if (!rc) rc = clr_prepare_fields(c);
-    if (!rc) rc = clr_prepare_norms(c);
-    if (!rc) {
-      std::vector<long long> cap(c->n_tr[CLR_TRACER_SRCS], src_cap[i]);
-      rc = clr_prepare_sources(c, nside_base, cap.data());
-    }
-    if (!rc && nside_kappa > 0) rc = clr_prepare_kappa(c, nside_kappa, 1, &r_kappa[i]);
-    if (rc) return ens_fail(e, rc, "realisation " + std::to_string(i) + ": " + c->err);
     e->ctx.push_back(c);
     e->r_kappa.push_back(nside_kappa > 0 ? r_kappa[i] : 0.0);
+    e->src_cap.push_back(src_cap[i]);
+    const int rc = prepare(e, i);
+    if (rc) return rc;
   }
   ENS_HIP(e, hipStreamCreateWithFlags(&e->origin, hipStreamNonBlocking));
   e->streams.resize(nstreams);
@@ -145,6 +163,7 @@ int clr_ensemble_create(clr_ensemble **out, int n, clr_ctx *const *ctxs, int nsi
   ENS_HIP(e, hipMalloc((void **)&e->flags_dev, n * sizeof(int)));
   e->flags.assign(n, 0);
   e->sigma2.assign(n, 0.0);
+  e->held = captured_state(e);
   return CLR_OK;
 }
 
@@ -171,6 +190,18 @@ int clr_ensemble_run(clr_ensemble *e, const uint32_t *seeds, const double *r_smo
                      int *n_invalid, float *ms) {
   if (!e || !seeds || !r_smooth) return CLR_ERR_ARG;
   ENS_HIP(e, hipSetDevice(e->device));
+  // The graph holds the contexts' buffers by address.  Single calls on a
+  // context (a flagged realisation is re-run with them) may have moved some
+  // since: then the buffers are set up and the graph is captured again.
+  const bool moved = captured_state(e) != e->held;
+  if (moved) {
+    drop_graph(e);
+    for (int i = 0; i < e->n; i++) {
+      const int rc = prepare(e, i);
+      if (rc) return rc;
+    }
+    e->held = captured_state(e);
+  }
   const bool same = e->exec && e->smooth_potential == (smooth_potential ? 1 : 0) &&
                     std::equal(seeds, seeds + e->n, e->seeds.begin()) &&
                     std::equal(r_smooth, r_smooth + e->n, e->r_smooth.begin());

@@ -201,6 +201,10 @@ int clr_launch_norm_tables_given(clr_ctx *c, int ntr, const int *kinds, const in
 // allocation, no memset, no host wait; sigma^2 and the norm edges stay on the
 // device).  Same kernels and results as the launchers above.
 int clr_prepare_fields(clr_ctx *c);
+// Appends what a captured graph holds of a context: the addresses and
+// capacities of its buffers (any single call may grow or replace one), the base
+// pixels' nside and the kappa plan.
+void clr_captured_state(const clr_ctx *c, std::string &out);
 int clr_autotune_fields(clr_ctx *c, int reps, int cap, float *ms, int *ncand, int *best);
 int clr_fft_candidate_count(int N);
 int clr_fft3d(clr_ctx *c, float *g, int forward);

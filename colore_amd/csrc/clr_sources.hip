@@ -1140,6 +1140,19 @@ __global__ void k_src_props(const float4 *__restrict__ pos, long long n, const d
 
 }  // namespace
 
+// Count scratch of a population: bytes (ncells), block totals, offsets, scan
+// partials (a multiple of 256 bytes: every population's bytes start aligned).
+static size_t src_per_pop(size_t ncells) {
+  const size_t nblocks = ncells / kBlockCells, nsb = (nblocks + kScanB - 1) / kScanB;
+  return (ncells + nblocks * 4 + (nblocks + 1) * 8 + (nsb + 1) * 8 + 64 + 255) / 256 * 256;
+}
+// Of a pass over np populations: after the last, the totals and list lengths
+// for the host.  clr_prepare_sources reserves as much, so that a single call
+// on an ensemble's context finds the buffer that the captured graph holds.
+static size_t src_scratch(int np, size_t ncells) {
+  return (size_t)np * src_per_pop(ncells) + (CLR_NPOP_MAX + 2) * sizeof(long long);
+}
+
 int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long long *nsrc, int fused) {
   const int nall = c->n_tr[CLR_TRACER_SRCS];
   if (ipop < -1 || ipop >= nall) return clr_fail(c, CLR_ERR_ARG, "no source population %d", ipop);
@@ -1172,12 +1185,8 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
   }
   const int np = p1 - p0;
   const size_t nblocks = ncells / kBlockCells;
-  const size_t nsb = (nblocks + kScanB - 1) / kScanB;
-  // scratch per population: bytes (ncells), block totals, offsets, scan partials
-  // (a multiple of 256 bytes: every population's bytes start aligned)
-  const size_t per_pop = (ncells + nblocks * 4 + (nblocks + 1) * 8 + (nsb + 1) * 8 + 64 + 255) / 256 * 256;
-  // (after the last population: the totals and list lengths for the host)
-  rc = clr_ensure(c, (void **)&c->rowcnt, &c->rows_n, (size_t)np * per_pop + (CLR_NPOP_MAX + 2) * sizeof(long long));
+  const size_t per_pop = src_per_pop(ncells);
+  rc = clr_ensure(c, (void **)&c->rowcnt, &c->rows_n, src_scratch(np, ncells));
   if (rc) return rc;
 
   SrcArgs a{};
@@ -1600,11 +1609,6 @@ int clr_launch_sources_stream(clr_ctx *c, int ipop, int nthr, const int *iz_begi
 // result invalid (the caller then re-runs the realisation with
 // clr_sample_sources).  Same kernels, streams and order as clr_launch_sources.
 // ---------------------------------------------------------------------------
-static size_t src_per_pop(size_t ncells) {
-  const size_t nblocks = ncells / kBlockCells, nsb = (nblocks + kScanB - 1) / kScanB;
-  return (ncells + nblocks * 4 + (nblocks + 1) * 8 + (nsb + 1) * 8 + 64 + 255) / 256 * 256;
-}
-
 int clr_prepare_sources(clr_ctx *c, int nside_base, const long long *cap) {
   const int np = c->n_tr[CLR_TRACER_SRCS], N = c->N, na = c->na;
   const size_t ncells = (size_t)N * N * N;
@@ -1633,7 +1637,7 @@ int clr_prepare_sources(clr_ctx *c, int nside_base, const long long *cap) {
       C.cap = cap[i];
     }
   }
-  rc = clr_ensure(c, (void **)&c->rowcnt, &c->rows_n, (size_t)np * src_per_pop(ncells));
+  rc = clr_ensure(c, (void **)&c->rowcnt, &c->rows_n, src_scratch(np, ncells));
   if (rc) return rc;
   rc = clr_ensure(c, &c->esc, &c->esc_bytes, c->esc_bytes > 0 ? c->esc_bytes : (size_t)16 + 16 * 65536);
   if (rc) return rc;
@@ -1644,7 +1648,7 @@ int clr_enqueue_sources(clr_ctx *c, hipStream_t st, uint32_t seed, int nside_bas
   const int np = c->n_tr[CLR_TRACER_SRCS], N = c->N, na = c->na;
   const size_t ncells = (size_t)N * N * N, per_pop = src_per_pop(ncells);
   const size_t nblocks = ncells / kBlockCells;
-  if (c->rows_n < (size_t)np * per_pop || !c->esc || c->misc_n < 16 + 16 * 4096 || c->r2n_nside != nside_base)
+  if (c->rows_n < src_scratch(np, ncells) || !c->esc || c->misc_n < 16 + 16 * 4096 || c->r2n_nside != nside_base)
     return clr_fail(c, CLR_ERR_STATE, "sampling buffers not prepared");
   const double dx = c->L / N, cell_vol = dx * dx * dx;
   SrcArgs a{};

@@ -375,8 +375,9 @@ int clr_sample_sources_surrogate(clr_ctx *ctx, clr_mlp *net, int ipop, uint32_t 
  * r_kappa[i] (nside_kappa; 0: no map), spread over nstreams captured streams.
  * Buffers are set up by clr_ensemble_create (catalogue capacity src_cap[i]
  * per population).  clr_ensemble_run captures and instantiates the graph on
- * the first call and whenever the seeds or smoothing change, then replays
- * it; afterwards every context is in the state the single calls leave
+ * the first call and whenever the seeds or smoothing change or a single call
+ * on one of the contexts has moved a buffer that it holds, then replays it;
+ * afterwards every context is in the state the single calls leave
  * (clr_fetch_sources, clr_fetch_grid, clr_get_norm_table work) and its
  * results equal those calls' bit for bit.  A realisation whose counts hit a
  * case the graph does not handle (counts of 254 or more in a cell, an
