@@ -190,6 +190,12 @@ int clr_ensemble_run(clr_ensemble *e, const uint32_t *seeds, const double *r_smo
                      int *n_invalid, float *ms) {
   if (!e || !seeds || !r_smooth) return CLR_ERR_ARG;
   ENS_HIP(e, hipSetDevice(e->device));
+  // (a clr_gaussian_fields call returns before the potential's last passes have
+  // run; the graph's streams do not wait for the context's)
+  for (clr_ctx *c : e->ctx) {
+    const int rc = clr_phi_ready(c, 1);
+    if (rc) return ens_fail(e, rc, c->err);
+  }
   // The graph holds the contexts' buffers by address.  Single calls on a
   // context (a flagged realisation is re-run with them) may have moved some
   // since: then the buffers are set up and the graph is captured again.

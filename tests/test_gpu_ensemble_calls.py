@@ -87,3 +87,21 @@ def test_flagged_realisation_rerun(workdir):
     ens.close()
     for c in ctxs:
         c.close()
+
+
+def test_fields_call_before_a_replay(workdir):
+    """clr_gaussian_fields returns while the potential's last passes run on the
+    context's second stream; a replay that follows at once must wait for them."""
+    from test_gpu_ensemble import _check, _single
+    rs, runs, ctxs, ens, seeds, rsm = _ensemble(workdir, 4_000_000)
+    wants = [_single(run, r, NSIDE) for run, r in zip(runs, rs)]
+    for rep in range(3):
+        bad, _ = ens.run(seeds, rsm)
+        assert bad == 0
+        for i in range(len(rs)):
+            _check(ens, ctxs, i, wants[i])
+        for c, run in zip(ctxs, runs):
+            c.gaussian_fields(100 + rep, run.scalar("r_smooth"), True)
+    ens.close()
+    for c in ctxs:
+        c.close()
