@@ -262,17 +262,8 @@ k_shells(ShellArgs a, double *__restrict__ partial) {
                              : __int_as_float(__builtin_amdgcn_readlane(__float_as_int(yl), r));
       return __builtin_amdgcn_sqrtf(__builtin_fmaf(x32, x32, __builtin_fmaf(y32, y32, z2)));
     };
-    // Table position in row r.  The fraction of a bin is r idr - i0 rounded
-    // once (fma), in every second group of four y rows from the rounded
-    // product: sums of FP32 terms shift by a few 1e-9 with the choice, and
-    // this one keeps them equal to those of earlier builds.
-    auto pos_at = [&](int r) {
-      const float rf = radius_at(r);
-      TabPos p = tab_pos_f32(rf, a.idr_f, a.na);
-      const bool odd = (((ty * TY * ROWS + r) >> 2) & 1) != 0;
-      p.tq = __builtin_fmaf(odd ? rf * a.idr_f : rf, odd ? 1.f : a.idr_f, -(float)p.i0);
-      return p;
-    };
+    // table position in row r (TY rows of a cube's row share ty)
+    auto pos_at = [&](int r) { return cell_tab_pos_f32(radius_at(r), a.idr_f, a.na, ty * TY * ROWS + r); };
     if (!inside) {
       // no shell in reach: the transform alone
 #pragma unroll 1

@@ -147,6 +147,17 @@ __device__ inline TabPos tab_pos_f32(float rf, float idr_f, int na) {
   p.tq = xq - (float)p.i0;
   return p;
 }
+// The same for a cell in row iy of the grid.  The fraction of a bin is r idr -
+// i0 rounded once (fma), in every second group of four y rows from the rounded
+// product: both are within the same error of the exact fraction, but the FP64
+// sums over shells of few cells would move by a few 1e-9 with one of them in
+// every row.  Both passes take their cells' positions from here.
+__device__ inline TabPos cell_tab_pos_f32(float rf, float idr_f, int na, int iy) {
+  TabPos p = tab_pos_f32(rf, idr_f, na);
+  const bool odd = (iy & 4) != 0;
+  p.tq = __builtin_fmaf(odd ? rf * idr_f : rf, odd ? 1.f : idr_f, -(float)p.i0);
+  return p;
+}
 // D from the bin's (value, slope) pair.
 __device__ inline float growth_at(const TabPos &p, float d0, float slope, float d1_last_f) {
   const float v = __builtin_fmaf(slope, p.tq, d0);

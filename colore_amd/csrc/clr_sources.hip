@@ -83,8 +83,8 @@ struct SrcArgs {
 // the shell pass would have stored.
 __device__ inline float cell_density(const SrcArgs &a, float g, int ix, int iy, int iz) {
   if (!a.fused) return g;
-  const TabPos p = tab_pos_f32(radius_f32(coord_f32(ix, a.dxf, a.oxf), coord_f32(iy, a.dxf, a.oyf),
-                                          coord_f32(iz, a.dxf, a.ozf)), a.idr_f, a.na);
+  const TabPos p = cell_tab_pos_f32(radius_f32(coord_f32(ix, a.dxf, a.oxf), coord_f32(iy, a.dxf, a.oyf),
+                                               coord_f32(iz, a.dxf, a.ozf)), a.idr_f, a.na, iy);
   return lognormal_f32(g, growth_f32(a.d1f, p, a.d1_last_f), a.s2f);
 }
 
