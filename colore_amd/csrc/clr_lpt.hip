@@ -262,9 +262,12 @@ __global__ __launch_bounds__(256) void k_lpt_deposit(const float *__restrict__ p
 // deposit's 5.6 ms at 512^3 (CIC; 17 ms for TSC).  The whole 1LPT density at
 // 512^3 took 10.55 ms (TSC 23.4) and takes 5.67 (6.39); this kernel is now
 // bound by the positions' FP64 chain and their loads.  Below 256^3 the region
-// stays float (256 threads): norms of shells of a few hundred cells keep the
-// rounding of FP32 sums in this order to 1e-9, and FP64 sums (more exact, 0.28
-// -> 0.02 ms at 128^3, TSC) move them by 2e-9.
+// stays float (256 threads): the norms of shells of a few hundred cells stay
+// within 1e-9 of those that FP32 sums gave, from which FP64 sums (more exact,
+// and 0.28 -> 0.02 ms at 128^3, TSC) move them by 2e-9.
+// Without room for `regs` (null) the region's cells are added to the grid with
+// atomics instead (512^3 6.5 ms instead of 6.1, TSC 8.1 instead of 7.5; a particle's
+// weights added straight to the grid took 24.5 and 73.5).
 // Needs N >= 64 and N a multiple of 16, so that a region never wraps onto
 // itself.
 constexpr int kDT = 16, kDHalo = 2, kDR = kDT + 2 * kDHalo;
@@ -356,6 +359,15 @@ __global__ __launch_bounds__(64 * sizeof(R)) void k_lpt_deposit_tiled(PosArgs a,
     }
   }
   __syncthreads();
+  if (!regs) {
+    for (int i = threadIdx.x; i < kDRegion; i += kDThreads) {
+      const float v = (float)reg[i];
+      if (v == 0.f) continue;
+      const int cx = wrapn(ox + i % kDR, N), cy = wrapn(oy + i / kDR % kDR, N), cz = wrapn(oz + i / (kDR * kDR), N);
+      atomicAdd(g + cx + ngx * cy + pl * cz, v);
+    }
+    return;
+  }
   float4 *const out = (float4 *)(regs + (size_t)b * kDRegion);
   for (int i = threadIdx.x; i < kDRegion / 4; i += kDThreads) {
     const R *r = reg + 4 * i;
@@ -469,7 +481,7 @@ int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
   // one workspace for the grids and the tiles' regions, kept for the next call
   // (lpt_release).  The regions need 1.95 grids: 2LPT has them free by then,
   // 1LPT asks for two more grids and without them stores the positions and
-  // deposits with atomics.
+  // adds its regions to the grid with atomics.
   const size_t need = gbytes * nbuf + (tiled && order == 1 ? reg_bytes : 0);
   bool own_regs = tiled;
   if (c->lpt_ws_n < need) {
@@ -593,16 +605,16 @@ int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
   if (ok()) e = hipMemsetAsync(c->dens, 0, gbytes, c->stream);
   if (ok()) {
     const float iag = (float)(N / c->L);
-    if (own_regs) {
-      regs = order == 1 ? ps[0] + 3 * (gbytes / sizeof(float)) : ps[0];
+    if (tiled) {
+      if (own_regs) regs = order == 1 ? ps[0] + 3 * (gbytes / sizeof(float)) : ps[0];
       const dim3 gt((unsigned)((N / kDT) * (N / kDT) * (N / kDT)));
       if (N >= kDWideN) launch_deposit<double>(gt, c->stream, a, c->dens, regs, iag, interp == 1, stored);
       else launch_deposit<float>(gt, c->stream, a, c->dens, regs, iag, interp == 1, stored);
-      hipLaunchKernelGGL(k_lpt_gather, gt, blk, 0, c->stream, regs, c->dens, N, ngx);
+      if (regs) hipLaunchKernelGGL(k_lpt_gather, gt, blk, 0, c->stream, regs, c->dens, N, ngx);
     } else {
       hipLaunchKernelGGL(k_lpt_deposit, gc, blk, 0, c->stream, pos[0], pos[1], pos[2], c->dens, N, ngx, iag, interp);
-      hipLaunchKernelGGL(k_lpt_norm, gc, blk, 0, c->stream, c->dens, N, ngx);
     }
+    if (!regs) hipLaunchKernelGGL(k_lpt_norm, gc, blk, 0, c->stream, c->dens, N, ngx);
     e = hipGetLastError();
   }
   if (ok()) e = hipEventRecord(c->ev1, c->stream);
