@@ -18,6 +18,31 @@ int clr_fail(clr_ctx *c, int code, const char *fmt, ...) {
   return code;
 }
 
+size_t clr_idle_bytes(const clr_ctx *c) {
+  return (c->ws_busy & CLR_WS_LPT ? 0 : c->lpt_ws_n) + (c->ws_busy & CLR_WS_BEAM ? 0 : c->beam_ws_n);
+}
+
+hipError_t clr_malloc(clr_ctx *c, void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && clr_idle_bytes(c) > 0) {
+    (void)hipGetLastError();
+    auto give = [c](int ws, void *&b, size_t &n) {
+      if (c->ws_busy & ws || !b) return;
+      (void)hipFree(b);
+      b = nullptr;
+      n = 0;
+    };
+    give(CLR_WS_LPT, c->lpt_ws, c->lpt_ws_n);
+    give(CLR_WS_BEAM, c->beam_ws, c->beam_ws_n);
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+  }
+  return e;
+}
+
 int clr_ensure(clr_ctx *c, void **p, size_t *have, size_t bytes) {
   if (*have >= bytes && *p) return CLR_OK;
   if (*p) {
@@ -26,9 +51,7 @@ int clr_ensure(clr_ctx *c, void **p, size_t *have, size_t bytes) {
   }
   *p = nullptr;
   *have = 0;
-  if (hipMalloc(p, bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    *p = nullptr;
+  if (clr_malloc(c, p, bytes) != hipSuccess) {
     return clr_fail(c, CLR_ERR_OOM, "device allocation of %zu bytes failed", bytes);
   }
   *have = bytes;
@@ -75,7 +98,7 @@ int clr_ring2nest_table(clr_ctx *c, int nside) {
   std::vector<int32_t> t(npix);
   for (int64_t p = 0; p < npix; p++) t[p] = (int32_t)clr::ring2nest(nside, p);
   if (c->r2n) { CLR_HIP(c, hipStreamSynchronize(c->stream)); hipFree(c->r2n); c->r2n = nullptr; }
-  CLR_HIP(c, hipMalloc((void **)&c->r2n, npix * sizeof(int32_t)));
+  CLR_HIP(c, clr_malloc(c, (void **)&c->r2n, npix * sizeof(int32_t)));
   CLR_HIP(c, hipMemcpy(c->r2n, t.data(), npix * sizeof(int32_t), hipMemcpyHostToDevice));
   c->r2n_nside = nside;
   return CLR_OK;

@@ -133,6 +133,7 @@ struct clr_ctx {
   size_t lpt_ws_n = 0;
   void *beam_ws = nullptr;   // source beams' tables, order and results, skewers' staging (clr_los.hip)
   size_t beam_ws_n = 0;
+  int ws_busy = 0;           // CLR_WS_* of the call that is using one (clr_ws_use)
   std::string los_plan;
   void *los_buf = nullptr;
   size_t los_buf_n = 0;
@@ -156,6 +157,19 @@ int clr_fail(clr_ctx *c, int code, const char *fmt, ...);
   } while (0)
 
 int clr_ensure(clr_ctx *c, void **p, size_t *have, size_t bytes);
+// lpt_ws and beam_ws are kept only to save allocations.  They count as free
+// memory where a call decides what fits (clr_idle_bytes), and an allocation
+// that fails gives them back and is tried once more (clr_malloc), but for
+// those that the present call is using.
+enum { CLR_WS_LPT = 1, CLR_WS_BEAM = 2 };
+struct clr_ws_use {
+  clr_ctx *c;
+  int ws;
+  clr_ws_use(clr_ctx *c_, int ws_) : c(c_), ws(ws_) { c->ws_busy |= ws; }
+  ~clr_ws_use() { c->ws_busy &= ~ws; }
+};
+size_t clr_idle_bytes(const clr_ctx *c);
+hipError_t clr_malloc(clr_ctx *c, void **p, size_t bytes);
 int clr_ring2nest_table(clr_ctx *c, int nside);
 
 // stage launchers (one per file)

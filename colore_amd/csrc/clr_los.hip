@@ -430,7 +430,7 @@ int clr_launch_los(clr_ctx *c, int which, int nside, int nplanes, const double *
   if (which == 0 && steps >= 0.4 * reach) {
     size_t fr = 0, tot = 0;
     if (c->tidal_n >= t6_bytes) use_t6 = true;
-    else if (hipMemGetInfo(&fr, &tot) == hipSuccess && t6_bytes <= fr / 4) use_t6 = true;
+    else if (hipMemGetInfo(&fr, &tot) == hipSuccess && t6_bytes <= (fr + clr_idle_bytes(c)) / 4) use_t6 = true;
     else (void)hipGetLastError();
     if (use_t6) {
       rc = clr_ensure(c, &c->tidal, &c->tidal_n, t6_bytes);
@@ -467,7 +467,7 @@ int clr_prepare_kappa(clr_ctx *c, int nside, int nplanes, const double *r_src) {
     if (c->los_buf) CLR_HIP(c, hipFree(c->los_buf));
     c->los_buf = nullptr;
     c->los_buf_n = 0;
-    CLR_HIP(c, hipMalloc(&c->los_buf, need));
+    CLR_HIP(c, clr_malloc(c, &c->los_buf, need));
     c->los_buf_n = need;
   }
   CLR_HIP(c, hipMemcpy(c->los_buf, f12.data(), f12.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -846,7 +846,7 @@ bool clr_cell_records(clr_ctx *c, bool tidal) {
       (void)hipGetLastError();
       return false;
     }
-    if (need > fr / 4) return false;
+    if (need > (fr + clr_idle_bytes(c)) / 4) return false;
   }
   if (clr_ensure(c, &c->velrec, &c->velrec_n, vb)) return false;
   if (tidal && clr_ensure(c, &c->tidal, &c->tidal_n, tb)) return false;
@@ -900,9 +900,7 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
     if (need <= kBeamKeep) {
       rc = clr_ensure(c, &c->beam_ws, &c->beam_ws_n, need);
       buf = (char *)c->beam_ws;
-    } else if (hipMalloc(&own.p, need) != hipSuccess) {
-      (void)hipGetLastError();
-      own.p = nullptr;
+    } else if (clr_malloc(c, &own.p, need) != hipSuccess) {
       rc = clr_fail(c, CLR_ERR_HIP, "source beams: no device memory for %zu bytes", need);
     } else {
       buf = (char *)own.p;
@@ -911,6 +909,7 @@ int clr_launch_src_beams(clr_ctx *c, int ipop, const double *r_arr_a2r, float *d
     if (!order) return rc;
     order = false;
   }
+  const clr_ws_use use(c, own.p ? 0 : CLR_WS_BEAM);
   double *dfac = (double *)buf, *da2r = dfac + 3 * nr;
   uint32_t *cnt = (uint32_t *)(buf + tab_bytes), *perm = cnt + (order ? nb : 0);
   uint2 *kr = (uint2 *)(perm + (order ? (n + 1) / 2 * 2 : 0));
@@ -1138,6 +1137,7 @@ int clr_launch_src_skewers(clr_ctx *c, int ipop, int gaussian, double sigma2, fl
   const size_t obytes = order ? ((size_t)nb * 4 + (size_t)cap * 12 + 15) / 16 * 16 : 0;
   const int wrc = clr_ensure(c, &c->beam_ws, &c->beam_ws_n, obytes + (size_t)cap * a.nr * 2 * sizeof(float));
   if (wrc) return wrc;
+  const clr_ws_use use(c, CLR_WS_BEAM);
   uint32_t *cnt = (uint32_t *)c->beam_ws;
   uint2 *kr = (uint2 *)(cnt + nb);
   uint32_t *perm = order ? (uint32_t *)(kr + cap) : nullptr;

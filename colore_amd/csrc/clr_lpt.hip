@@ -484,16 +484,14 @@ int clr_launch_lpt(clr_ctx *c, int order, int interp, float *pos_out) {
   // adds its regions to the grid with atomics.
   const size_t need = gbytes * nbuf + (tiled && order == 1 ? reg_bytes : 0);
   bool own_regs = tiled;
+  const clr_ws_use use(c, CLR_WS_LPT);
   if (c->lpt_ws_n < need) {
     lpt_release(c, true);
-    if (hipMalloc(&c->lpt_ws, need) == hipSuccess) {
+    if (clr_malloc(c, &c->lpt_ws, need) == hipSuccess) {
       c->lpt_ws_n = need;
     } else {
-      (void)hipGetLastError();
       own_regs = tiled && order == 2;
-      if (hipMalloc(&c->lpt_ws, gbytes * nbuf) != hipSuccess) {
-        (void)hipGetLastError();
-        c->lpt_ws = nullptr;
+      if (clr_malloc(c, &c->lpt_ws, gbytes * nbuf) != hipSuccess) {
         return clr_fail(c, CLR_ERR_HIP, "out of device memory for the LPT grids");
       }
       c->lpt_ws_n = gbytes * nbuf;

@@ -1177,7 +1177,7 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
   PopSrc ps{};
   for (int i = p0; i < p1; i++) {
     TracerDev &T = c->tr[CLR_TRACER_SRCS][i];
-    if (!T.ptab) CLR_HIP(c, hipMalloc((void **)&T.ptab, pop_table_len(na) * sizeof(float4)));
+    if (!T.ptab) CLR_HIP(c, clr_malloc(c, (void **)&T.ptab, pop_table_len(na) * sizeof(float4)));
     ps.amp[i - p0] = T.amp;
     ps.bz[i - p0] = T.bz;
     ps.norm[i - p0] = T.norm;
@@ -1337,8 +1337,8 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
       C.ipix = nullptr;
       C.cap = 0;
       const long long cap = n + n / 16 + 1024;
-      if (hipMalloc((void **)&C.pos, (size_t)cap * 4 * sizeof(float)) != hipSuccess ||
-          hipMalloc((void **)&C.ipix, (size_t)cap * sizeof(int32_t)) != hipSuccess) {
+      if (clr_malloc(c, (void **)&C.pos, (size_t)cap * 4 * sizeof(float)) != hipSuccess ||
+          clr_malloc(c, (void **)&C.ipix, (size_t)cap * sizeof(int32_t)) != hipSuccess) {
         (void)hipGetLastError();
         return clr_fail(c, CLR_ERR_OOM, "cannot allocate catalogue of %lld sources", n);
       }
@@ -1404,7 +1404,7 @@ int clr_launch_source_props(clr_ctx *c, int ipop, float *out, long long n) {
   if (n == 0) return CLR_OK;
   const int na = c->na;
   float4 *tmp = nullptr;
-  CLR_HIP(c, hipMalloc((void **)&tmp, (size_t)n * sizeof(float4)));
+  CLR_HIP(c, clr_malloc(c, (void **)&tmp, (size_t)n * sizeof(float4)));
   hipLaunchKernelGGL(k_src_props, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream,
                      (const float4 *)C.pos, n, c->bg, c->bg + na, c->glob_idr, c->r_last, c->h_bg_last[1], tmp);
   hipError_t e = hipGetLastError();
@@ -1432,7 +1432,7 @@ int clr_launch_fetch_counts(clr_ctx *c, int ipop, int iz0, int nz, int32_t *out)
   const uint8_t *cnt8 = (const uint8_t *)c->rowcnt + (size_t)q * c->cnt_per_pop;
   const uint64_t n = (uint64_t)N * N * nz, cell0 = (uint64_t)N * N * iz0;
   int32_t *tmp = nullptr;
-  CLR_HIP(c, hipMalloc((void **)&tmp, n * sizeof(int32_t)));
+  CLR_HIP(c, clr_malloc(c, (void **)&tmp, n * sizeof(int32_t)));
   hipLaunchKernelGGL(k_expand_counts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, cnt8,
                      (const uint32_t *)(cnt8 + (size_t)N * N * N), (const ulonglong2 *)((char *)c->esc + 16), c->cnt_nesc, (unsigned long long)q, cell0, n, tmp);
   hipError_t e = hipGetLastError();
@@ -1474,12 +1474,12 @@ int clr_launch_sources_stream(clr_ctx *c, int ipop, int nthr, const int *iz_begi
   uint32_t *dst = nullptr;
   int *dizb = nullptr, *dflag = nullptr;
   const double dx = c->L / N;
-  hipError_t e = hipMalloc((void **)&lam, ncells * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void **)&off, (ncells + 1) * sizeof(long long));
-  if (e == hipSuccess) e = hipMalloc((void **)&bsum, (nsb + 1) * sizeof(long long));
-  if (e == hipSuccess) e = hipMalloc((void **)&dst, (size_t)nthr * stream_len * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMalloc((void **)&dizb, (size_t)(nthr + 1) * sizeof(int));
-  if (e == hipSuccess) e = hipMalloc((void **)&dflag, sizeof(int));
+  hipError_t e = clr_malloc(c, (void **)&lam, ncells * sizeof(double));
+  if (e == hipSuccess) e = clr_malloc(c, (void **)&off, (ncells + 1) * sizeof(long long));
+  if (e == hipSuccess) e = clr_malloc(c, (void **)&bsum, (nsb + 1) * sizeof(long long));
+  if (e == hipSuccess) e = clr_malloc(c, (void **)&dst, (size_t)nthr * stream_len * sizeof(uint32_t));
+  if (e == hipSuccess) e = clr_malloc(c, (void **)&dizb, (size_t)(nthr + 1) * sizeof(int));
+  if (e == hipSuccess) e = clr_malloc(c, (void **)&dflag, sizeof(int));
   auto release = [&]() {
     (void)hipStreamSynchronize(c->stream);
     for (void *q : {(void *)lam, (void *)off, (void *)bsum, (void *)dst, (void *)dizb, (void *)dflag})
@@ -1552,8 +1552,8 @@ int clr_launch_sources_stream(clr_ctx *c, int ipop, int nthr, const int *iz_begi
     C.ipix = nullptr;
     C.cap = 0;
     const long long cap = total + total / 16 + 1024;
-    if (hipMalloc((void **)&C.pos, (size_t)cap * 4 * sizeof(float)) != hipSuccess ||
-        hipMalloc((void **)&C.ipix, (size_t)cap * sizeof(int32_t)) != hipSuccess) {
+    if (clr_malloc(c, (void **)&C.pos, (size_t)cap * 4 * sizeof(float)) != hipSuccess ||
+        clr_malloc(c, (void **)&C.ipix, (size_t)cap * sizeof(int32_t)) != hipSuccess) {
       (void)hipGetLastError();
       release();
       return clr_fail(c, CLR_ERR_OOM, "cannot allocate catalogue of %lld sources", total);
@@ -1620,8 +1620,8 @@ int clr_prepare_sources(clr_ctx *c, int nside_base, const long long *cap) {
   for (int i = 0; i < np; i++) {
     TracerDev &T = c->tr[CLR_TRACER_SRCS][i];
     if (!T.set) return clr_fail(c, CLR_ERR_STATE, "population %d has no tables", i);
-    if (!T.ptab) CLR_HIP(c, hipMalloc((void **)&T.ptab, pop_table_len(na) * sizeof(float4)));
-    if (!T.edge) CLR_HIP(c, hipMalloc((void **)&T.edge, 2 * sizeof(double)));
+    if (!T.ptab) CLR_HIP(c, clr_malloc(c, (void **)&T.ptab, pop_table_len(na) * sizeof(float4)));
+    if (!T.edge) CLR_HIP(c, clr_malloc(c, (void **)&T.edge, 2 * sizeof(double)));
     CatalogDev &C = c->cat[i];
     if (C.cap < cap[i]) {
       if (C.pos) (void)hipFree(C.pos);
@@ -1629,8 +1629,8 @@ int clr_prepare_sources(clr_ctx *c, int nside_base, const long long *cap) {
       C.pos = nullptr;
       C.ipix = nullptr;
       C.cap = 0;
-      if (hipMalloc((void **)&C.pos, (size_t)cap[i] * 4 * sizeof(float)) != hipSuccess ||
-          hipMalloc((void **)&C.ipix, (size_t)cap[i] * sizeof(int32_t)) != hipSuccess) {
+      if (clr_malloc(c, (void **)&C.pos, (size_t)cap[i] * 4 * sizeof(float)) != hipSuccess ||
+          clr_malloc(c, (void **)&C.ipix, (size_t)cap[i] * sizeof(int32_t)) != hipSuccess) {
         (void)hipGetLastError();
         return clr_fail(c, CLR_ERR_OOM, "cannot allocate a catalogue of %lld sources", cap[i]);
       }
