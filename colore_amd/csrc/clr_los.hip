@@ -16,6 +16,7 @@
 // records' fetch); ISW 2.11 ms (3.51), bound by its vector instructions.
 #include "clr_internal.h"
 #include <algorithm>
+#include <limits.h>
 #include <math.h>
 #include <string.h>
 
@@ -359,7 +360,7 @@ static int los_setup(clr_ctx *c, int which, int nside, int nplanes, const double
   const double dr = r_max / nr, idr = 1. / dr;
   std::vector<double> rs(r_src, r_src + nplanes);
   std::vector<float> rsf(nplanes);
-  for (int i = 0; i < nplanes; i++) rsf[i] = (float)rs[i];   // ind_sort sorts flouble values
+  for (int i = 0; i < nplanes; i++) rsf[i] = rs[i] == rs[i] ? (float)rs[i] : -INFINITY;   // ind_sort sorts flouble values
   std::vector<int> order(nplanes);
   for (int i = 0; i < nplanes; i++) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return rsf[x] < rsf[y]; });
@@ -375,9 +376,11 @@ static int los_setup(clr_ctx *c, int which, int nside, int nplanes, const double
   a.nr = nr;
   a.nplanes = nplanes;
   for (int i = 0; i < nplanes; i++) {
-    const int ih = (int)(rs[order[i]] * idr + 0.5);
+    // (a distance that is negative, NaN or no int of steps takes none: -1)
+    const double st = rs[order[i]] * idr + 0.5;
+    const int ih = st > -2147483648. && st < 2147483648. ? (int)st : INT_MIN;
     a.inv_rmax[i] = 1. / (ih * dr);
-    a.irmax[i] = std::min(ih, nr - 1);
+    a.irmax[i] = std::max(-1, std::min(ih, nr - 1));
   }
   // (plane i adds the steps after plane i-1's last)
   a.lg = lanes_lg(12LL * nside * nside, a.irmax[nplanes - 1] + 1);
