@@ -693,7 +693,10 @@ struct ShellPlan {
   size_t lds;
 };
 constexpr int kShellTile[4][4] = {{4, 4, 4, 0}, {8, 4, 8, 0}, {16, 8, 4, 1}, {16, 16, 4, 1}};   // cells in x, y, z; staged
+// Shells x tracers are limited to what four wavefronts' accumulators and one
+// logged shell per lane (a sum per quantity and an index) fit the LDS with.
 int shell_plan(clr_ctx *c, int nz, int NT, ShellPlan &p) {
+  if (kWaves * ((size_t)(nz + 64) * (2 + NT) * sizeof(double) + 64 * sizeof(int)) > 160 * 1024) return CLR_ERR_ARG;
   if (c->shell_dr <= 0) {
     // narrowest shell below r(L/2), and whether z(r) never decreases
     const std::vector<double> &zz = c->h_z, &rr = c->h_r;
