@@ -1184,6 +1184,7 @@ int clr_prepare_norms(clr_ctx *c) {
   const int ntr = norms_tracers(c, tk, tp);
   if (ntr < 1 || ntr > kMaxTr) return clr_fail(c, CLR_ERR_ARG, "%d tracers (1 .. %d)", ntr, kMaxTr);
   const int nz = (int)(c->zmax_half_box / 0.05) + 2;
+  if (nz > kNormMaxShells) return clr_fail(c, CLR_ERR_ARG, "%d redshift shells (at most %d)", nz, kNormMaxShells);
   const size_t nvals = (size_t)nz * (2 + ntr);
   int rc = clr_ensure(c, (void **)&c->red, &c->red_n,
                       ((size_t)kShellBlocks * nvals + nvals + 2 * nz + 2 * ntr) * sizeof(double));

@@ -40,3 +40,12 @@ def test_shells_times_tracers(workdir, nz, ntr, ok):
         with pytest.raises(RuntimeError, match="shells"):
             ctx.shell_norms(lognormal_fused=True, sigma2=s2, ntracers=ntr, cap=1200)
     ctx.close()
+
+
+def test_ensemble_shells(workdir):
+    """An ensemble's contexts have the same limit (the captured pass has no check of its own)."""
+    from colore_amd import lib
+    ctx = _context(workdir, 1025, 1)
+    with pytest.raises(RuntimeError, match="shells"):
+        lib.Ensemble([ctx], src_cap=1000)
+    ctx.close()
