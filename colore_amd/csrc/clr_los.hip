@@ -1196,9 +1196,14 @@ struct CstmArgs {
 };
 
 // (1 + d)^b for d > -1 (the model-0 branch of bias_model_f64) as exp(b log1p):
-// a few 1e-16 relative, and half of pow's instructions; the map is FP32.
+// a few 1e-16 relative, and half of pow's instructions; the map is FP32.  Where
+// that is NaN (0 x infinity: b = 0 and d infinite, ...) pow decides.
 __device__ inline double bias_model_march(double d, double b, int model) {
-  if (model == 0) return d <= -1 ? 0.0 : exp(b * log1p(d));
+  if (model == 0) {
+    if (d <= -1) return 0.0;
+    const double v = exp(b * log1p(d));
+    if (v == v) return v;
+  }
   return bias_model_f64(d, b, model);
 }
 
@@ -1247,7 +1252,15 @@ __global__ __launch_bounds__(256) void k_cstm(CstmArgs a, const double *__restri
 #pragma unroll
       for (int c = 0; c < 4; c++) e[c] = fma(h[s][0], (double)f[s][2 * c + 1] - (double)f[s][2 * c], (double)f[s][2 * c]);
       const double e0 = fma(h[s][1], e[1] - e[0], e[0]), e1 = fma(h[s][1], e[3] - e[2], e[2]);
-      const double d = fma(h[s][2], e1 - e0, e0);
+      double d = fma(h[s][2], e1 - e0, e0);
+      if (d != d) {
+        // a corner that is not finite: by the corners' weights, as the reference
+        d = 0;
+#pragma unroll
+        for (int c = 0; c < 8; c++)
+          d += (double)f[s][c] * ((c & 4 ? h[s][2] : 1 - h[s][2]) * (c & 2 ? h[s][1] : 1 - h[s][1]) *
+                                  (c & 1 ? h[s][0] : 1 - h[s][0]));
+      }
       // the reference holds d as flouble before bias_model
       cval += kz[j] * (bias_model_march((double)(float)d, bz[j], a.model) * nz[j] - 1);
     }
