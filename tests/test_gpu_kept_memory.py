@@ -9,28 +9,11 @@ import numpy as np
 import pytest
 
 from conftest import make_run
+from device_memory import free_bytes, only
 
 pytestmark = pytest.mark.gpu
 
 N = 512
-
-
-def _fill(leave):
-    """Tensors that leave about `leave` bytes of the device free."""
-    import torch
-    torch.cuda.empty_cache()
-    fill = []
-    for _ in range(4):   # (the first large block can leave more free than asked for)
-        extra = torch.cuda.mem_get_info()[0] - leave
-        if extra > 1 << 26:
-            fill.append(torch.empty(extra, dtype=torch.uint8, device="cuda"))
-    return fill
-
-
-def _free(fill):
-    import torch
-    fill.clear()
-    torch.cuda.empty_cache()
 
 
 def _lpt_context(workdir, **kw):
@@ -49,23 +32,20 @@ def _lpt_context(workdir, **kw):
 
 
 def test_records_beside_kept_grids(workdir):
-    import torch
     run, ctx, kept, _ = _lpt_context(workdir)
     r = np.array([run.scalar("r_max")])
     records = 24 * N ** 3
-    fill = _fill(4 * records - kept // 2)
-    free = torch.cuda.mem_get_info()[0]
-    assert free < 4 * records < free + kept, (free, kept, records)
-    before = ctx.lib.clr_device_bytes(ctx.h)
-    got = ctx.kappa(512, r)
-    assert ctx.lib.clr_device_bytes(ctx.h) >= before + records
-    _free(fill)
+    with only(4 * records - kept // 2):
+        free = free_bytes()
+        assert free < 4 * records < free + kept, (free, kept, records)
+        before = ctx.lib.clr_device_bytes(ctx.h)
+        got = ctx.kappa(512, r)
+        assert ctx.lib.clr_device_bytes(ctx.h) >= before + records
     assert np.array_equal(got, ctx.kappa(512, r))
     ctx.close()
 
 
 def test_catalogue_takes_kept_memory(workdir):
-    import torch
     run, ctx, kept, (amp, bz, model) = _lpt_context(workdir)
     ctx.shell_norms(lognormal_fused=False, ntracers=1)
     tab = ctx.norm_table(0, 0)
@@ -77,12 +57,11 @@ def test_catalogue_takes_kept_memory(workdir):
 
     n = sample(1e-2)
     scale = 1e-2 * 3e7 / n   # about 3e7 sources, 600 MB
-    fill = _fill(200 << 20)
-    assert torch.cuda.mem_get_info()[0] < 500 << 20
-    n = sample(scale)
-    assert n * 20 > 500 << 20 and n * 20 < kept
-    pos, ipix = ctx.fetch_sources(0, n)
-    _free(fill)
+    with only(200 << 20):
+        assert free_bytes() < 500 << 20
+        n = sample(scale)
+        assert n * 20 > 500 << 20 and n * 20 < kept
+        pos, ipix = ctx.fetch_sources(0, n)
     assert sample(scale) == n
     pos2, ipix2 = ctx.fetch_sources(0, n)
     assert np.array_equal(pos, pos2) and np.array_equal(ipix, ipix2)

@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("N,interp", [(512, 1), (512, 2)])
 def test_lpt_without_room_for_regions(workdir, N, interp):
-    import torch
     from colore_amd import lib
+    from device_memory import free_bytes, only
     _, run = make_run("C2", N, workdir, z_max=0.6, with_maps=False)
     ctx = lib.Context(N, run.scalar("l_box"))
     ctx.upload_tables(run.tables())
@@ -35,17 +35,10 @@ def test_lpt_without_room_for_regions(workdir, N, interp):
     grid = N * N * ((N + 2 + 31) // 32 * 32) * 4
     regions = (N // 16) ** 3 * 20 ** 3 * 4
     room = 3 * grid + regions // 2
-    torch.cuda.empty_cache()
-    fill = []
-    for _ in range(4):   # (the first large block can leave more free than asked for)
-        extra = torch.cuda.mem_get_info()[0] - room
-        if extra > 1 << 26:
-            fill.append(torch.empty(extra, dtype=torch.uint8, device="cuda"))
-    free = torch.cuda.mem_get_info()[0]
-    assert 3 * grid < free < 3 * grid + regions, (free, grid, regions)
-    got = density()
-    del fill
-    torch.cuda.empty_cache()
+    with only(room):
+        free = free_bytes()
+        assert 3 * grid < free < 3 * grid + regions, (free, grid, regions)
+        got = density()
     ctx.close()
     assert np.abs((got - want) / (2 + want)).max() < 2e-6
     assert abs(got.mean()) < 1e-5
