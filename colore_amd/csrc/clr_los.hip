@@ -585,16 +585,20 @@ __device__ inline void vel_cell(const float4 *__restrict__ vrec, const float *__
 // within a bin is the atomics'; a source's result does not depend on it).
 constexpr int kDirG = 64;
 // The order pays where the records in reach (40 bytes per cell) are more than
-// the 256 MB last-level cache holds, from 32768 sources on: 950k sources at
-// 512^3 3.57 -> 2.00 ms with the records' pass, 384^3 1.84 -> 1.10, 256^3 0.71
-// -> 0.61, but 192^3 0.38 -> 0.41 and 128^3 0.20 -> 0.28; 19k sources at 512^3
-// 1.07 -> 1.08.  16 sources per bin (64: 2.07 ms; bins of 4 shells of distance
-// in 4 times wider cells, 2.08).
+// the 256 MB last-level cache holds: 950k sources at 512^3 3.57 -> 2.00 ms with
+// the records' pass, 384^3 1.84 -> 1.10, 256^3 0.71 -> 0.61, but 192^3 0.38 ->
+// 0.41 and 128^3 0.20 -> 0.28.  The line in sources: 24k in catalogue order and
+// in order of direction 171 and 187 us at 256^3, 452 and 462 at 384^3, 1075 and
+// 1083 at 512^3; 28k 179/184, 464/460, 1097/1089; 33k 188/186, 478/468,
+// 1123/1102; 64k 216/212, 540/495, 1221/1155.  16 sources per bin (64: 2.07 ms;
+// bins of 4 shells of distance in 4 times wider cells, 2.08).
 constexpr int kDirMinN = 256;
 // Skewers, whose every step of a source is a gather of its own, pay the order's
-// 20 us back from fewer sources on: with it 189k sources at 512^3 1.41 -> 0.90
-// ms, 29k at 384^3 184 -> 152 us, at 256^3 90 -> 83, at 192^3 57 -> 62; 5k at
-// 384^3 51 -> 66.
+// 20 us back from fewer sources on: from 24576, where dir_grid's bins become
+// finer (64 -> 16 sources in each).  At 256^3 20k sources took 65 us in
+// catalogue order and 72 in order of direction, 24k 77/83, 28k 88/83, 64k
+// 184/155; at 384^3 12k 92/94, 20k 137/132, 24k 157/149, 28k 179/149; at 512^3
+// 4k 60/73, 12k 140/135, 24k 243/214, 28k 274/219; at 192^3 28k 56/61.
 constexpr long long kDirMin = 32768, kDirMinSkw = 24576, kDirPer = 16;
 constexpr size_t kBeamKeep = (size_t)1 << 30;
 
