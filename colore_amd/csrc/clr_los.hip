@@ -32,6 +32,8 @@ struct LosArgs {
   int N, ngx;
   double idx, dr, ox, oy, oz;
   int nr, nplanes, lg;    // 2^lg lanes per pixel
+  int run;                // k_los_planes
+  int mono;               // irmax does not decrease
   int irmax[kMaxPlanes];
   double inv_rmax[kMaxPlanes];
 };
@@ -106,6 +108,21 @@ __device__ inline void tidal_at(const float *__restrict__ phi, int N, size_t ngx
   t[5] = phi[X0 + Y0 + ZH] + phi[X0 + Y0 + ZL] - 2 * c0;
   t[2] = 0.25f * (phi[xh + Y0 + ZH] + phi[xl + Y0 + ZL] - phi[xh + Y0 + ZL] - phi[xl + Y0 + ZH]);
   t[4] = 0.25f * (phi[X0 + YH + ZH] + phi[X0 + YL + ZL] - phi[X0 + YH + ZL] - phi[X0 + YL + ZH]);
+}
+
+template <int CTRL>
+__device__ inline double dpp_get(double v) {
+  const int l2 = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, true);
+  const int h2 = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, true);
+  return __hiloint2double(h2, l2);
+}
+// Sum over each group of 2^lg consecutive lanes (lg <= 4), in every one of them.
+__device__ inline double lanes_add(double v, int lg) {
+  if (lg > 0) v += dpp_get<0xB1>(v);    // quad_perm [1,0,3,2]
+  if (lg > 1) v += dpp_get<0x4E>(v);    // quad_perm [2,3,0,1]
+  if (lg > 2) v += dpp_get<0x141>(v);   // row_half_mirror
+  if (lg > 3) v += dpp_get<0x140>(v);   // row_mirror
+  return v;
 }
 
 // kappa (KAPPA) or ISW march: 2^lg consecutive lanes per pixel, each taking
@@ -193,6 +210,120 @@ __global__ __launch_bounds__(256) void k_los(LosArgs a, const double *__restrict
     double v = KAPPA ? k1 - a.inv_rmax[pl] * k2 : k1;
     for (int o = 1; o < K; o <<= 1) v += __shfl_xor(v, o);
     if (sub == 0) out[(size_t)pl * npix + ip] = (float)v;
+  }
+}
+
+// The same march for many planes: the steps in flight run on across the planes'
+// ends, and a plane's sum goes out when its last step has been added.  k_los
+// starts anew at each plane, reading up to 4 rounds of steps past its end: with
+// 100 planes ISW at 128^3, nside 64 took 175 us there and takes 26 here, kappa at
+// 512^3, nside 64 505 and 423.  For few planes the plain loop is the faster one
+// (kappa 371 and 409 us with one plane).
+template <bool KAPPA, bool REC, bool ONE>
+__global__ __launch_bounds__(256) void k_los_planes(LosArgs a, const double *__restrict__ fac1,
+                                                    const double *__restrict__ fac2, int64_t nside, int64_t npix,
+                                                    float *__restrict__ out) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lg = ONE ? 0 : a.lg, sub = ONE ? 0 : (int)(t & ((1 << lg) - 1)), K = 1 << lg;
+  const int64_t ip = t >> lg;
+  if (ip >= npix) return;
+  Ray ray;
+  pix2vec_nest(nside, ip, ray.u);
+  ray_setup(ray, a.dr, a.idx, a.ox, a.oy, a.oz);
+  const int N = a.N;
+  const size_t ngx = (size_t)a.ngx, plane = (size_t)N * ngx;
+  const float *__restrict__ phi = a.phi;
+  double rot[6];
+  if (KAPPA) {
+#pragma clang fp contract(off)
+    double cth = ray.u[2];
+    if (cth >= 1) cth = 1;
+    if (cth <= -1) cth = -1;
+    const double sth = sqrt((1 - cth) * (1 + cth));
+    double cph = 1, sph = 0;
+    if (sth != 0) { cph = ray.u[0] / sth; sph = ray.u[1] / sth; }
+    const double pre = a.idx * a.idx;
+    rot[0] = (cth * cth * cph * cph + sph * sph) * pre;
+    rot[1] = (2 * cph * sph * (cth * cth - 1)) * pre;
+    rot[2] = (-2 * cth * sth * cph) * pre;
+    rot[3] = (cth * cth * sph * sph + cph * cph) * pre;
+    rot[4] = (-2 * cth * sth * sph) * pre;
+    rot[5] = (sth * sth) * pre;
+  }
+  double k1 = 0, k2 = 0;
+  constexpr int U = KAPPA && !REC ? 1 : 4;   // rounds of K steps in flight
+  // the values of the U rounds from step i on (steps past the last are read, not added)
+  auto read = [&](int i, int64_t x[3], const int64_t kstep[3], float tt[U][6]) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      int c[3];
+      ray_cell(ray, x, i + u * K, N, a.dr, a.idx, a.ox, a.oy, a.oz, c);
+#pragma unroll
+      for (int ax = 0; ax < 3; ax++) x[ax] += kstep[ax];
+      if (!KAPPA) {
+        tt[u][0] = phi[(size_t)c[2] * plane + (size_t)c[1] * ngx + c[0]];
+      } else if (REC) {
+        const float *r = (const float *)(a.t6 + (((size_t)c[2] * N + c[1]) * N + c[0]) * 3);
+        __builtin_memcpy(tt[u], r, 16);
+        __builtin_memcpy(tt[u] + 4, r + 4, 8);
+      } else {
+        tidal_at(phi, N, ngx, plane, c, tt[u]);
+      }
+    }
+  };
+  auto add = [&](const float t[6], int j, double &s1, double &s2) {
+    if (!KAPPA) {
+      s1 = fma((double)t[0], fac1[j], s1);
+    } else {
+      double dot = rot[0] * (double)t[0];
+#pragma unroll
+      for (int q = 1; q < 6; q++) dot = fma(rot[q], (double)t[q], dot);
+      s1 = fma(dot, fac1[j], s1);
+      s2 = fma(dot, fac2[j], s2);
+    }
+  };
+  auto emit = [&](int pl, double s1, double s2) {
+    double v = KAPPA ? s1 - a.inv_rmax[pl] * s2 : s1;
+    if (!ONE) v = lanes_add(v, lg);
+    if (sub == 0) out[(size_t)pl * npix + ip] = (float)v;
+  };
+  int pl = 0, first = 0, pend = a.irmax[0];   // the next plane, its first step and its last
+  auto next = [&]() { if (++pl < a.nplanes) pend = a.irmax[pl]; };
+  while (pl < a.nplanes) {
+    if (pend < first) {   // no step of its own
+      emit(pl, k1, k2);
+      first = pend + 1;
+      next();
+      continue;
+    }
+    const int end = a.mono ? a.nplanes : pl + 1;   // these planes are one run of steps
+    const int last = a.irmax[end - 1];
+    int b = first >> lg << lg;   // the round's first step
+    int64_t x[3], kstep[3];
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) {
+      x[ax] = ray.base[ax] + (int64_t)(b + sub) * ray.step[ax];
+      kstep[ax] = ray.step[ax] << lg;
+    }
+    for (; b <= last; b += U * K) {
+      float tt[U][6];
+      read(b + sub, x, kstep, tt);
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int bu = b + u * K, j = bu + sub;
+        if (bu > last) break;
+        double n1 = k1, n2 = k2;   // the sums with step j
+        if (ONE || (j >= first && j <= last)) add(tt[u], j, n1, n2);
+        // planes that end before the next round: with the steps up to their last
+        for (; pl < end && pend < bu + K; next()) {
+          const bool in = j <= pend;
+          emit(pl, in ? n1 : k1, in ? n2 : k2);
+        }
+        k1 = n1;
+        k2 = n2;
+      }
+    }
+    first = last + 1;
   }
 }
 
@@ -320,11 +451,14 @@ void launch_records(clr_ctx *c, bool tidal, bool vel, float rlim) {
 
 // Lanes per pixel of a march over nstep steps: as many as bring npix pixels to
 // a quarter of a million threads (4 wavefronts on every SIMD), with 8 steps or
-// more each, at most 16.  nside 32 on 512^3: ISW 194 -> 46 us, a custom map 287 -> 49; nside
-// 64 on 192^3: ISW 57 -> 24, custom map 85 -> 42.
-int lanes_lg(int64_t npix, int nstep) {
+// more each, at most 16.  nside 32 on 512^3: ISW 194 -> 46 us, a custom map 287
+// -> 49; nside 64 on 192^3: ISW 57 -> 24, custom map 85 -> 42.  Every plane adds
+// its sum up over the lanes: where a march has its steps in flight, not more
+// lanes than leave each a step for every second plane (100 planes at 64^3,
+// nside 64: ISW 28 us with one lane, 40 with four).
+int lanes_lg(int64_t npix, int nstep, int nplanes = 1) {
   int lg = 0;
-  while (lg < 4 && (npix << lg) < (1 << 18) && (nstep >> lg) >= 16) lg++;
+  while (lg < 4 && (npix << lg) < (1 << 18) && (nstep >> lg) >= std::max(16, nplanes)) lg++;
   return lg;
 }
 
@@ -333,13 +467,16 @@ void launch_los(const LosArgs &a, const double *df, int nside, float *dout, hipS
   const int64_t npix = 12LL * nside * nside;
   const dim3 g((unsigned)(((npix << a.lg) + 255) / 256)), b(256);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, g, b, 0, s, a, df, df + a.nr, (int64_t)nside, npix, dout); };
-  if (KAPPA && a.t6) {
-    if (a.lg == 0) go(k_los<KAPPA, true, true>);
-    else go(k_los<KAPPA, true, false>);
-  } else {
-    if (a.lg == 0) go(k_los<KAPPA, false, true>);
-    else go(k_los<KAPPA, false, false>);
+  auto pick = [&](auto one, auto many) { go(a.lg == 0 ? one : many); };
+  if constexpr (KAPPA) {
+    if (a.t6) {
+      if (a.run) pick(k_los_planes<true, true, true>, k_los_planes<true, true, false>);
+      else pick(k_los<true, true, true>, k_los<true, true, false>);
+      return;
+    }
   }
+  if (a.run) pick(k_los_planes<KAPPA, false, true>, k_los_planes<KAPPA, false, false>);
+  else pick(k_los<KAPPA, false, true>, k_los<KAPPA, false, false>);
 }
 
 }  // namespace
@@ -382,7 +519,10 @@ static int los_setup(clr_ctx *c, int which, int nside, int nplanes, const double
     a.inv_rmax[i] = 1. / (ih * dr);
     a.irmax[i] = std::max(-1, std::min(ih, nr - 1));
   }
-  // (plane i adds the steps after plane i-1's last)
+  // (plane i adds the steps after plane i-1's last; two distances that only
+  // their float forms put in order may end at decreasing steps)
+  a.mono = 1;
+  for (int i = 1; i < nplanes; i++) a.mono = a.mono && a.irmax[i] >= a.irmax[i - 1];
   a.lg = lanes_lg(12LL * nside * nside, a.irmax[nplanes - 1] + 1);
   const double *rr = c->h_r.data(), *zz = c->h_z.data(), *dd = c->h_d1.data(), *pd = c->h_pd.data();
   f12.assign(2 * (size_t)nr, 0.0);
@@ -439,6 +579,18 @@ int clr_launch_los(clr_ctx *c, int which, int nside, int nplanes, const double *
       rc = clr_ensure(c, &c->tidal, &c->tidal_n, t6_bytes);
       if (rc) return rc;
     }
+  }
+  // k_los_planes where planes end within the steps that k_los has in flight: 4
+  // rounds of steps from records or phi alone (3 planes take the same time both
+  // ways; 10 planes, nside 64: ISW 25 -> 12 us at 64^3, 116 -> 93 at 512^3),
+  // one of the direct march's (30 planes: 65 -> 28 us at 64^3, nside 16 53 -> 26,
+  // but 373 -> 412 at 512^3, nside 64, and 505 -> 423 with 100)
+  const int nstep = a.irmax[nplanes - 1] + 1;
+  if (which != 0 || use_t6) {
+    a.lg = lanes_lg(npix, nstep, nplanes);
+    a.run = nplanes > 3;
+  } else {
+    a.run = 8 * nplanes > nstep;
   }
   CLR_HIP(c, hipEventRecord(c->ev0, c->stream));
   if (use_t6) {
