@@ -329,7 +329,7 @@ constexpr int kCountLaneCells = 16;
 constexpr int kCountCells = kLanes * kCountLaneCells;
 constexpr int kCountSubs = kCountCells / kBlockCells;
 static_assert(kCountSubs == 2, "half a wavefront of k_count and k_fill is one block");
-constexpr int kFillWaves = 4;   // wavefronts per block of k_fill (N is a multiple of 16, N^3 of 4 x 1024)
+constexpr int kFillWaves = 4;   // wavefronts per block of k_fill, at most (N is a multiple of 16, N^3 of 4 x 1024)
 // queue entry: cell within the wavefront's 1024 (bits 0-9) | population
 // (bits 10-13) | the uniform's high 16 bits << 16.  The queue is worked when
 // another 8 cells per lane might not fit, and after the last population.  It is
@@ -706,7 +706,7 @@ __device__ inline int escaped_count(const ulonglong2 *esc, unsigned n, unsigned 
 __global__ __launch_bounds__(kFillWaves *kLanes) void k_fill(SrcArgs a) {
   constexpr int G = 2;   // populations whose loads are in flight together
   const int lane = threadIdx.x & 63;
-  const size_t wave = (size_t)blockIdx.x * kFillWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const size_t wave = (size_t)blockIdx.x * (blockDim.x / kLanes) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t w0 = wave * kCountSubs;   // first 512-cell block
   const uint64_t cell0 = (uint64_t)wave * kCountCells + (uint64_t)kCountLaneCells * lane;
   for (int g0 = 0; g0 < a.npop; g0 += G) {
@@ -787,6 +787,16 @@ __global__ __launch_bounds__(kFillWaves *kLanes) void k_fill(SrcArgs a) {
       }
     }
   }
+}
+
+// One wavefront per block where blocks of four would be fewer than 2048: a
+// catalogue of many sources per cell on a small grid is bound by the writes of
+// the few CUs that work (150 per cell, fill and positions: 32^3 314 -> 234 us,
+// 64^3 622 -> 561; 400 per cell at 32^3 860 -> 642; sparse ones take the same).
+void launch_fill(const SrcArgs &a, size_t ncells, hipStream_t s) {
+  const size_t waves = ncells / kCountCells;
+  const unsigned w = waves >= 2048 * kFillWaves ? kFillWaves : 1;
+  hipLaunchKernelGGL(k_fill, dim3((unsigned)(waves / w)), dim3(w * kLanes), 0, s, a);
 }
 
 struct WriteArgs {
@@ -1351,7 +1361,7 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
   }
   CLR_HIP(c, hipEventRecord(c->ev2, c->stream));
   if (total > 0) {
-    hipLaunchKernelGGL(k_fill, dim3((unsigned)(ncells / (kFillWaves * kCountCells))), dim3(kFillWaves * kLanes), 0, c->stream, a);
+    launch_fill(a, ncells, c->stream);
     CLR_HIP(c, hipGetLastError());
   }
   rc = clr_phi_ready(c, 0);   // k_write reads phi
@@ -1722,7 +1732,7 @@ int clr_enqueue_sources(clr_ctx *c, hipStream_t st, uint32_t seed, int nside_bas
   launch_scan(sp, np, nblocks, st);
   hipLaunchKernelGGL(k_graph_flags, dim3(1), dim3(64), 0, st, (const unsigned *)a.esc_n,
                      (const unsigned *)a.exq_n, a.exq_cap, np, gt, flag_dev);
-  hipLaunchKernelGGL(k_fill, dim3((unsigned)(ncells / (kFillWaves * kCountCells))), dim3(kFillWaves * kLanes), 0, st, a);
+  launch_fill(a, ncells, st);
   for (int i = 0; i < np; i++) {
     CatalogDev &C = c->cat[i];
     WriteArgs w{};
