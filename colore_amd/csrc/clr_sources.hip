@@ -1253,7 +1253,8 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
   CLR_HIP(c, hipEventRecord(c->ev0, c->stream));
   std::vector<long long> tot(np);
   unsigned int nesc = 0;
-  for (int attempt = 0; attempt < 2; attempt++) {
+  // (the escape list's length is known once the FP64 queue is long enough)
+  for (int attempt = 0; attempt < 3; attempt++) {
     // escape list: a counter, then entries (grown and recounted if it overflows)
     const size_t want = c->esc_bytes > 0 ? c->esc_bytes : (size_t)16 + 16 * 65536;
     rc = clr_ensure(c, &c->esc, &c->esc_bytes, want);
@@ -1301,7 +1302,7 @@ int clr_launch_sources(clr_ctx *c, int ipop, uint32_t seed, int nside_base, long
     nesc = (unsigned int)res[np];
     const unsigned int nexq = (unsigned int)res[np + 1];
     if (nesc <= a.esc_cap && nexq <= a.exq_cap) break;
-    if (attempt == 1) return clr_fail(c, CLR_ERR_STATE, "source lists overflow (%u, %u entries)", nesc, nexq);
+    if (attempt == 2) return clr_fail(c, CLR_ERR_STATE, "source lists overflow (%u, %u entries)", nesc, nexq);
     if (nesc > a.esc_cap) {
       rc = clr_ensure(c, &c->esc, &c->esc_bytes, (size_t)16 + 16 * ((size_t)nesc + nesc / 4 + 1024));
       if (rc) return rc;
